@@ -12,6 +12,7 @@
 // Contraction is off in this file: each sum is the same sequence of FP32
 // roundings (bias first, inputs in order) as the CPU oracle, so the forward
 // pass is bit-identical to it.
+#include <algorithm>
 #include <cmath>
 
 #include "omx_common.hpp"
@@ -36,120 +37,201 @@ __device__ __forceinline__ void load_params(float *p, const float *__restrict__ 
     __syncthreads();
 }
 
+// 16 samples per workgroup: a wave takes four, a lane one hidden unit, so the
+// 64 x 64 layer is 64 steps of one weight read and four independent sums
+// (each in the oracle's order: bias, then inputs ascending) instead of a
+// thread walking all 64 units of a sample by itself.  Bound by launch,
+// parameter load and those sums' latency: 2658 samples 47 -> 7 us, a single
+// sample (one step of the LU's policy) 52 -> 7 us.
+constexpr int kFS = 16;        // samples per workgroup
+constexpr int kFW = kFS / 4;   // per wave
+
 __global__ void __launch_bounds__(256)
 k_mlp_forward(int64_t batch, const float *__restrict__ params, const float *__restrict__ X, float *__restrict__ H1,
               float *__restrict__ H2, float *__restrict__ Z) {
     __shared__ float p[kNP];
+    __shared__ __align__(16) float xs[4][kIn][kFW];  // [wave][input][sample]
+    __shared__ __align__(16) float hs[4][kH][kFW];   // hidden layer of the wave's samples
+    const int wave = threadIdx.x >> 6, j = threadIdx.x & 63;
+    const int64_t s0 = (int64_t)blockIdx.x * kFS + wave * kFW;
+    {
+        const int64_t s = s0 + (j >> 4);
+        xs[wave][j & 15][j >> 4] = s < batch ? X[s * kIn + (j & 15)] : 0.0f;
+    }
     load_params(p, params);
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= batch) return;
-    float x[kIn], h1[kH];
+    float a[kFW];
 #pragma unroll
-    for (int i = 0; i < kIn; ++i) x[i] = X[s * kIn + i];
-    for (int j = 0; j < kH; ++j) {
-        float a = p[kB1 + j];
+    for (int u = 0; u < kFW; ++u) a[u] = p[kB1 + j];
 #pragma unroll
-        for (int i = 0; i < kIn; ++i) a += x[i] * p[kW1 + i * kH + j];
-        h1[j] = a > 0.0f ? a : 0.0f;
-        H1[s * kH + j] = h1[j];
-    }
-    float z[kOut];
+    for (int i = 0; i < kIn; ++i) {
+        const float w = p[kW1 + i * kH + j];
 #pragma unroll
-    for (int j = 0; j < kOut; ++j) z[j] = p[kB3 + j];
-    // h2 one unit at a time; its contribution to z is added after all of h2
-    // is known, in the oracle's order (z_j = b3_j + sum_i h2_i W3[i][j])
-    float h2[kH];
-    for (int j = 0; j < kH; ++j) {
-        float a = p[kB2 + j];
-        for (int i = 0; i < kH; ++i) a += h1[i] * p[kW2 + i * kH + j];
-        h2[j] = a > 0.0f ? a : 0.0f;
-        H2[s * kH + j] = h2[j];
+        for (int u = 0; u < kFW; ++u) a[u] += xs[wave][i][u] * w;
     }
 #pragma unroll
-    for (int j = 0; j < kOut; ++j) {
-        float a = z[j];
-        for (int i = 0; i < kH; ++i) a += h2[i] * p[kW3 + i * kOut + j];
-        Z[s * kOut + j] = a;
+    for (int u = 0; u < kFW; ++u) {
+        const float h = a[u] > 0.0f ? a[u] : 0.0f;
+        hs[wave][j][u] = h;
+        if (s0 + u < batch) H1[(s0 + u) * kH + j] = h;
+        a[u] = p[kB2 + j];
+    }
+    __syncthreads();
+#pragma unroll 16
+    for (int i = 0; i < kH; ++i) {
+        const float w = p[kW2 + i * kH + j];
+#pragma unroll
+        for (int u = 0; u < kFW; ++u) a[u] += hs[wave][i][u] * w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kFW; ++u) {
+        const float h = a[u] > 0.0f ? a[u] : 0.0f;
+        hs[wave][j][u] = h;
+        if (s0 + u < batch) H2[(s0 + u) * kH + j] = h;
+    }
+    __syncthreads();
+    // z_o = b3_o + sum_i h2_i W3[i][o], a lane per (sample, output)
+    if (j < kFW * kOut) {
+        const int u = j / kOut, o = j % kOut;
+        float z = p[kB3 + o];
+#pragma unroll 16
+        for (int i = 0; i < kH; ++i) z += hs[wave][i][u] * p[kW3 + i * kOut + o];
+        if (s0 + u < batch) Z[(s0 + u) * kOut + o] = z;
     }
 }
 
-// Per-sample deltas of the mean loss: dz (3), d2 = dL/d(pre-activation 2)
-// (64), d1 (64), and the sample's loss (FP64).
-__global__ void __launch_bounds__(256)
-k_mlp_delta(int64_t batch, const float *__restrict__ params, const float *__restrict__ H1,
-            const float *__restrict__ H2, const float *__restrict__ Z, const int32_t *__restrict__ y,
-            const float *__restrict__ t, const float *__restrict__ m, float *__restrict__ D,
-            double *__restrict__ lossv) {
-    __shared__ float p[kNP];
-    load_params(p, params);
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= batch) return;
+// Backward of a chunk of samples in one workgroup of 1024 threads, 16
+// samples at a time through LDS: per sample the deltas dz (3), d2 = dL/d
+// (pre-activation 2), d1 (64 each) of the mean loss, then their products with
+// the layer inputs added, sample by sample, to the gradient entries that the
+// threads hold in registers (thread t: the 4 entries of W2 row t / 16 from
+// column 4 (t % 16), one entry of W1, and one of W3 or the biases).  A batch
+// of one chunk is finished here; otherwise the chunk's sums go to part and
+// k_mlp_grad_reduce adds them in chunk order.  The chunks are as many as the
+// workspace holds (one per 41 samples, kMaxChunks at most).  With a thread
+// per parameter walking the whole batch, a thread per sample for the deltas
+// and one thread for the loss, 2658 samples took 874 us (grad 679, loss 137,
+// deltas 58); bound now by LDS reads and the latency of the 64-step d1 sums.
+constexpr int kBS = 16;          // samples per pass
+constexpr int kBT = 1024;        // threads
+constexpr int kMaxChunks = 256;
+
+// bytes of a chunk's partial sums: the gradient and the loss (FP64)
+constexpr size_t kChunkBytes = ((size_t)kNP * sizeof(float) + sizeof(double) + 15) / 8 * 8;
+static_assert(kChunkBytes <= 41 * (kD * sizeof(float) + sizeof(double)), "one chunk per 41 samples");
+
+__global__ void __launch_bounds__(kBT)
+k_mlp_backward(int64_t batch, int64_t chunk, const float *__restrict__ params, const float *__restrict__ X,
+               const float *__restrict__ H1, const float *__restrict__ H2, const float *__restrict__ Z,
+               const int32_t *__restrict__ y, const float *__restrict__ t, const float *__restrict__ m,
+               float *__restrict__ grad, float *__restrict__ loss, float *__restrict__ part,
+               double *__restrict__ lpart) {
+    __shared__ float xs[kBS][kIn], h1[kBS][kH], h2[kBS][kH], dz[kBS][kOut], d1[kBS][kH];
+    __shared__ __align__(16) float d2[kBS][kH];
+    __shared__ double ls[kBS];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int sl = tid >> 6;  // this thread's sample of a pass, in the per-sample phases
+    const int64_t b0 = (int64_t)blockIdx.x * chunk;
+    const int64_t b1 = b0 + chunk < batch ? b0 + chunk : batch;
     const float inv = 1.0f / (float)batch;
-    const float z0 = Z[s * kOut], z1 = Z[s * kOut + 1], z2 = Z[s * kOut + 2];
-    const float mx = z0 > z1 ? z0 : z1;
-    const float e0 = expf(z0 - mx), e1 = expf(z1 - mx);
-    const float lse = mx + logf(e0 + e1);
-    const float p0 = e0 / (e0 + e1), p1 = e1 / (e0 + e1);
-    const int ys = y[s];
-    const float diff = z2 - t[s];
-    lossv[s] = (double)(lse - (ys ? z1 : z0)) + 0.5 * (double)(m[s] * diff * diff);
-    float dz[kOut];
-    dz[0] = (p0 - (ys ? 0.0f : 1.0f)) * inv;
-    dz[1] = (p1 - (ys ? 1.0f : 0.0f)) * inv;
-    dz[2] = m[s] * diff * inv;
-    float *d = D + s * kD;
+    // row `lane` of W2 and of W3
+    float w2[kH], w3[kOut];
 #pragma unroll
-    for (int j = 0; j < kOut; ++j) d[j] = dz[j];
-    float d2[kH];
-    for (int i = 0; i < kH; ++i) {
-        float a = 0.0f;
+    for (int j = 0; j < kH; ++j) w2[j] = params[kW2 + lane * kH + j];
 #pragma unroll
-        for (int j = 0; j < kOut; ++j) a += p[kW3 + i * kOut + j] * dz[j];
-        d2[i] = H2[s * kH + i] > 0.0f ? a : 0.0f;
-        d[kOut + i] = d2[i];
+    for (int j = 0; j < kOut; ++j) w3[j] = params[kW3 + lane * kOut + j];
+    const int gi = tid >> 4, gj = (tid & 15) * 4;  // W2 entries (gi, gj .. gj + 3)
+    float g2[4] = {}, g1 = 0.0f, g3 = 0.0f;
+    double lsum = 0.0;
+    for (int64_t s0 = b0; s0 < b1; s0 += kBS) {
+        const int cnt = (int)(b1 - s0 < kBS ? b1 - s0 : kBS);
+        const int64_t s = s0 + sl;
+        const bool in = sl < cnt;
+        if (in) {
+            h1[sl][lane] = H1[s * kH + lane];
+            h2[sl][lane] = H2[s * kH + lane];
+            if (lane < kIn) xs[sl][lane] = X[s * kIn + lane];
+            // the sample's three deltas, the same in every lane
+            const float z0 = Z[s * kOut], z1 = Z[s * kOut + 1], z2 = Z[s * kOut + 2];
+            const float mx = z0 > z1 ? z0 : z1;
+            const float e0 = expf(z0 - mx), e1 = expf(z1 - mx);
+            const float p0 = e0 / (e0 + e1), p1 = e1 / (e0 + e1);
+            const int ys = y[s];
+            const float ms = m[s], diff = z2 - t[s];
+            const float q0 = (p0 - (ys ? 0.0f : 1.0f)) * inv;
+            const float q1 = (p1 - (ys ? 1.0f : 0.0f)) * inv;
+            const float q2 = ms * diff * inv;
+            if (lane == 0) {
+                dz[sl][0] = q0;
+                dz[sl][1] = q1;
+                dz[sl][2] = q2;
+                const float lse = mx + logf(e0 + e1);
+                ls[sl] = (double)(lse - (ys ? z1 : z0)) + 0.5 * (double)(ms * diff * diff);
+            }
+            float a = 0.0f;
+            a += w3[0] * q0;
+            a += w3[1] * q1;
+            a += w3[2] * q2;
+            d2[sl][lane] = h2[sl][lane] > 0.0f ? a : 0.0f;
+        }
+        __syncthreads();
+        if (in) {
+            float a = 0.0f;
+#pragma unroll
+            for (int j = 0; j < kH; ++j) a += w2[j] * d2[sl][j];
+            d1[sl][lane] = h1[sl][lane] > 0.0f ? a : 0.0f;
+        }
+        __syncthreads();
+        for (int q = 0; q < cnt; ++q) {
+            const float h = h1[q][gi];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) g2[e] += h * d2[q][gj + e];
+            g1 += xs[q][sl] * d1[q][lane];
+        }
+        if (tid < kH * kOut) {
+            for (int q = 0; q < cnt; ++q) g3 += h2[q][tid / kOut] * dz[q][tid % kOut];
+        } else if (tid < kH * kOut + kH) {
+            for (int q = 0; q < cnt; ++q) g3 += d2[q][tid - kH * kOut];
+        } else if (tid < kH * kOut + 2 * kH) {
+            for (int q = 0; q < cnt; ++q) g3 += d1[q][tid - kH * kOut - kH];
+        } else if (tid < kH * kOut + 2 * kH + kOut) {
+            for (int q = 0; q < cnt; ++q) g3 += dz[q][tid - kH * kOut - 2 * kH];
+        } else if (tid == kBT - 1) {
+            for (int q = 0; q < cnt; ++q) lsum += ls[q];
+        }
+        __syncthreads();
     }
-    for (int i = 0; i < kH; ++i) {
-        float a = 0.0f;
-        for (int j = 0; j < kH; ++j) a += p[kW2 + i * kH + j] * d2[j];
-        d[kOut + kH + i] = H1[s * kH + i] > 0.0f ? a : 0.0f;
+    float *out = part ? part + (int64_t)blockIdx.x * kNP : grad;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[kW2 + gi * kH + gj + e] = g2[e];
+    out[kW1 + sl * kH + lane] = g1;
+    if (tid < kH * kOut) out[kW3 + tid] = g3;
+    else if (tid < kH * kOut + kH) out[kB2 + tid - kH * kOut] = g3;
+    else if (tid < kH * kOut + 2 * kH) out[kB1 + tid - kH * kOut - kH] = g3;
+    else if (tid < kH * kOut + 2 * kH + kOut) out[kB3 + tid - kH * kOut - 2 * kH] = g3;
+    else if (tid == kBT - 1) {
+        if (part) lpart[blockIdx.x] = lsum;
+        else *loss = (float)(lsum / (double)batch);
     }
 }
 
-// One thread per parameter: the sum over samples (in order) of its
-// per-sample gradient.
-__global__ void __launch_bounds__(256)
-k_mlp_grad(int64_t batch, const float *__restrict__ X, const float *__restrict__ H1, const float *__restrict__ H2,
-           const float *__restrict__ D, float *__restrict__ grad) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= kNP) return;
-    float g = 0.0f;
-    if (q < kB1) {
-        const int i = q / kH, j = q % kH;
-        for (int64_t s = 0; s < batch; ++s) g += X[s * kIn + i] * D[s * kD + kOut + kH + j];
-    } else if (q < kW2) {
-        const int j = q - kB1;
-        for (int64_t s = 0; s < batch; ++s) g += D[s * kD + kOut + kH + j];
-    } else if (q < kB2) {
-        const int i = (q - kW2) / kH, j = (q - kW2) % kH;
-        for (int64_t s = 0; s < batch; ++s) g += H1[s * kH + i] * D[s * kD + kOut + j];
-    } else if (q < kW3) {
-        const int j = q - kB2;
-        for (int64_t s = 0; s < batch; ++s) g += D[s * kD + kOut + j];
-    } else if (q < kB3) {
-        const int i = (q - kW3) / kOut, j = (q - kW3) % kOut;
-        for (int64_t s = 0; s < batch; ++s) g += H2[s * kH + i] * D[s * kD + j];
-    } else {
-        const int j = q - kB3;
-        for (int64_t s = 0; s < batch; ++s) g += D[s * kD + j];
+// grad = the chunks' sums in chunk order, a thread per parameter; the loss
+// likewise in the last workgroup's last thread.
+__global__ void __launch_bounds__(64)
+k_mlp_grad_reduce(int64_t batch, int nchunk, const float *__restrict__ part, const double *__restrict__ lpart,
+                  float *__restrict__ grad, float *__restrict__ loss) {
+    const int q = blockIdx.x * 64 + threadIdx.x;
+    if (q < kNP) {
+        float g = 0.0f;
+#pragma unroll 16
+        for (int c = 0; c < nchunk; ++c) g += part[(int64_t)c * kNP + q];
+        grad[q] = g;
+    } else if (q == (int)gridDim.x * 64 - 1) {
+        double a = 0.0;
+#pragma unroll 16
+        for (int c = 0; c < nchunk; ++c) a += lpart[c];
+        *loss = (float)(a / (double)batch);
     }
-    grad[q] = g;
-}
-
-__global__ void k_loss_reduce(int64_t batch, const double *__restrict__ lossv, float *__restrict__ loss) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double a = 0.0;
-    for (int64_t s = 0; s < batch; ++s) a += lossv[s];
-    *loss = (float)(a / (double)batch);
 }
 
 __global__ void k_mlp_adam(int64_t np, float *__restrict__ params, const float *__restrict__ grad,
@@ -292,7 +374,7 @@ extern "C" {
 int omx_mlp_forward_f32(int64_t batch, const float *params, const float *X, float *H1, float *H2, float *Z,
                         void *stream) {
     if (batch <= 0 || !params || !X || !H1 || !H2 || !Z) return OMX_ERR_ARG;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)omx_cdiv(batch, 256)), dim3(256), 0, omx_stream(stream),
+    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)omx_cdiv(batch, kFS)), dim3(256), 0, omx_stream(stream),
                        batch, params, X, H1, H2, Z);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
@@ -309,15 +391,24 @@ int omx_mlp_backward_f32(int64_t batch, const float *params, const float *X, con
     if (batch <= 0 || !params || !X || !H1 || !H2 || !Z || !y || !t || !m || !grad || !loss) return OMX_ERR_ARG;
     if (!work || work_bytes < omx_mlp_backward_workspace_bytes(batch)) return OMX_ERR_WORKSPACE;
     hipStream_t st = omx_stream(stream);
-    double *lossv = static_cast<double *>(work);
-    float *D = reinterpret_cast<float *>(lossv + batch);
-    hipLaunchKernelGGL(k_mlp_delta, dim3((unsigned)omx_cdiv(batch, 256)), dim3(256), 0, st, batch, params, H1, H2,
-                       Z, y, t, m, D, lossv);
+    // chunks: as many as their partial sums fit the workspace, multiples of
+    // 41 samples or so each; one chunk writes the results itself
+    const int64_t most = std::min<int64_t>(kMaxChunks, (int64_t)(omx_mlp_backward_workspace_bytes(batch) / kChunkBytes));
+    int64_t nchunk = std::max<int64_t>(1, most);
+    const int64_t chunk = omx_cdiv(batch, nchunk);
+    nchunk = omx_cdiv(batch, chunk);
+    double *lpart = static_cast<double *>(work);
+    float *part = nchunk > 1 ? reinterpret_cast<float *>(lpart + nchunk) : nullptr;
+    hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)nchunk), dim3(kBT), 0, st, batch, chunk, params, X, H1, H2, Z, y,
+                       t, m, grad, loss, part, lpart);
     OMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)omx_cdiv(kNP, 256)), dim3(256), 0, st, batch, X, H1, H2, D, grad);
-    OMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_loss_reduce, dim3(1), dim3(64), 0, st, batch, lossv, loss);
-    OMX_LAUNCH_CHECK();
+    if (nchunk > 1) {
+        // kNP is not a multiple of 64: the last thread is free for the loss
+        static_assert(kNP % 64 != 0, "a spare thread in the last workgroup");
+        hipLaunchKernelGGL(k_mlp_grad_reduce, dim3((unsigned)omx_cdiv(kNP, 64)), dim3(64), 0, st, batch, (int)nchunk,
+                           part, lpart, grad, loss);
+        OMX_LAUNCH_CHECK();
+    }
     return OMX_OK;
 }
 

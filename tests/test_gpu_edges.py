@@ -1,0 +1,52 @@
+"""GPU kernels at the edges of their tiles, chunks and dispatch rules, against
+64-bit references."""
+import numpy as np
+import pytest
+
+from tests.gpu_util import dev, empty, host, ptr, torch_cuda
+
+pytestmark = pytest.mark.gpu
+
+
+def _L():
+    from openmxp_amd import _lib
+    return _lib.lib()
+
+
+# one sample, the 16-sample passes, the 41-sample chunks (one, two, the most
+# kept: 256) and a ragged last pass of each
+@pytest.mark.parametrize("B", [1, 4, 5, 16, 17, 81, 82, 83, 123, 700, 10496, 10497])
+def test_mlp_step_chunks(B):
+    torch = torch_cuda()
+    from openmxp_amd import scheduler
+    L = _L()
+    rng = np.random.default_rng(B)
+    P = dev(scheduler.init_params(B))
+    X = dev(rng.standard_normal((B, 16)).astype(np.float32))
+    y = dev((rng.random(B) < 0.5).astype(np.int32))
+    t, m = dev(rng.random(B).astype(np.float32)), dev((rng.random(B) < 0.5).astype(np.float32))
+    H1, H2, Z = (empty(B * k, torch.float32).fill_(float("nan")) for k in (64, 64, 3))
+    G, loss = empty(P.numel(), torch.float32).fill_(float("nan")), empty(1, torch.float32)
+    wb = L.omx_mlp_backward_workspace_bytes(B)
+    W = empty(wb, torch.uint8).fill_(255)
+    guard = empty(B * 64 + 64, torch.float32).fill_(7.0)
+    assert L.omx_mlp_forward_f32(B, ptr(P), ptr(X), ptr(guard), ptr(H2), ptr(Z), None) == 0
+    assert bool((guard[B * 64:] == 7.0).all())
+    assert L.omx_mlp_forward_f32(B, ptr(P), ptr(X), ptr(H1), ptr(H2), ptr(Z), None) == 0
+    assert L.omx_mlp_backward_f32(B, ptr(P), ptr(X), ptr(H1), ptr(H2), ptr(Z), ptr(y), ptr(t), ptr(m), ptr(G),
+                                  ptr(loss), ptr(W), wb, None) == 0
+    Pd = P.double().cpu().requires_grad_()
+    W1, b1, W2, b2, W3, b3 = torch.split(Pd, [1024, 64, 4096, 64, 192, 3])
+    h1 = torch.relu(X.double().cpu() @ W1.view(16, 64) + b1)
+    h2 = torch.relu(h1 @ W2.view(64, 64) + b2)
+    z = h2 @ W3.view(64, 3) + b3
+    want = torch.nn.functional.cross_entropy(z[:, :2], y.long().cpu()) + \
+        (0.5 * m.cpu() * (z[:, 2] - t.cpu()) ** 2).mean()
+    want.backward()
+    # FP32 sums of at most max(82, B / 256) + 256 terms after three layers of
+    # 64-term sums: (64 * 4 + terms) units of 2^-24 of the largest gradient,
+    # with a factor 4 for terms larger than their sum
+    tol = 4 * (64 * 4 + max(82, B / 256) + 256) * 2.0 ** -24
+    g = Pd.grad.numpy()
+    assert np.max(np.abs(host(G) - g)) <= tol * np.abs(g).max()
+    assert abs(float(host(loss)[0]) - float(want)) <= tol * max(1.0, abs(float(want)))
