@@ -112,6 +112,20 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kMK = 64;         // k per LDS stage
 constexpr int kBLd = kMK + 4;   // row stride of Bs: conflict-free 16-byte reads
 
+// The MFMA kernel takes products with at least this many C entries per
+// launch (2^18 = 512 x 512; smaller ones are latency-bound and the 64 x 64
+// VALU tiles spread them over more CUs) when its alignment conditions hold.
+#ifndef OMX_SGEMM_MFMA_T64
+#define OMX_SGEMM_MFMA_T64 1024
+#endif
+#ifndef OMX_SGEMM_MFMA_MIN
+#define OMX_SGEMM_MFMA_MIN (int64_t{1} << 18)
+#endif
+
+__host__ __device__ __forceinline__ bool mfma_size(int64_t m, int64_t n, int64_t batch) {
+    return m * n * batch >= OMX_SGEMM_MFMA_MIN;
+}
+
 template <int kT, bool kOneStage>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict__ A, int64_t lda,
@@ -256,55 +270,14 @@ k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restri
     }
 }
 
-// ---------------------------------------------------------------------------
-// 64 x 64 diagonal piece of the LU: unblocked right-looking LU in one wave.
-// Lane i holds row i in registers.  Step k: every lane reads row k from
-// lane k (v_readlane into scalar registers, no LDS round trip); the lanes
-// below scale their column-k entry by 1/u_kk (the multiplier) and subtract
-// multiplier x row k from the rest of their row.
-// ---------------------------------------------------------------------------
 __device__ __forceinline__ float lane_bcast(float v, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-
-// Lane i of the calling wave: row i of the 64 x 64 block in r, factored in
-// place (multipliers below the diagonal, U on and above it).  info (may be
-// null): the smallest row0 + k + 1 with a zero pivot u_kk.
-__device__ __forceinline__ void lu64_wave(float (&r)[kNB], int i, int64_t row0, int *info) {
-#pragma unroll
-    for (int k = 0; k < kNB; ++k) {
-        const float ukk = lane_bcast(r[k], k);
-        if (i == 0 && ukk == 0.0f && info) atomicMin(info, (int)(row0 + k + 1));
-        const float inv = 1.0f / ukk;
-        const bool below = i > k;
-        // rows at or above k take multiplier 0: fma(-0, u, r) leaves r as
-        // it is (up to the sign of a zero), with no select per entry
-        const float l = below ? r[k] * inv : 0.0f;
-        if (below) r[k] = l;
-#pragma unroll
-        for (int j = k + 1; j < kNB; ++j) r[j] = __builtin_fmaf(-l, lane_bcast(r[j], k), r[j]);
-    }
 }
 
 // The 64 x 64 triangle T (column-major, leading dimension ldt) into LDS:
 // t[r][c] = T(r, c).
 __device__ __forceinline__ void load_tri64(const float *__restrict__ T, int64_t ldt, float (*t)[kNB + 1]) {
     for (int e = threadIdx.x; e < kNB * kNB; e += blockDim.x) t[e & 63][e >> 6] = T[(e & 63) + (int64_t)(e >> 6) * ldt];
-    __syncthreads();
-}
-
-// Solves of one row (RUNN) or one column (LLNU) of 64 entries by a quad of
-// lanes: lane q of the quad owns entries q, q + 4, ..., q + 60 (16 registers,
-// index s <-> entry q + 4 s).  Step j: the owner (lane j % 4) finalises
-// entry j, the quad reads it with a DPP broadcast, and every lane updates
-// its later entries.  Each entry still receives its terms in the order
-// j = 0, 1, ... with one fused multiply-add each, as in column-by-column
-// substitution, so the results are those of the one-thread sweep; the
-// dependent chain per step is one multiply (or FMA) and one broadcast.
-
-// rd[j] = 1 / t[j][j] (the diagonal's reciprocals, shared by the workgroup)
-__device__ __forceinline__ void diag_recip64(const float (*t)[kNB + 1], float *rd) {
-    if (threadIdx.x < kNB) rd[threadIdx.x] = 1.0f / t[threadIdx.x][threadIdx.x];
     __syncthreads();
 }
 
@@ -315,153 +288,512 @@ __device__ __forceinline__ float quad_bcast(float v) {
                                                               0xF, 0xF, false));
 }
 
-template <int j>
-__device__ __forceinline__ void runn_step(float (&x)[16], int q, const float (*u)[kNB + 1], const float *rd) {
+// rd[j] = 1 / t[j][j] (the diagonal's reciprocals, shared by the workgroup)
+__device__ __forceinline__ void diag_recip64(const float (*t)[kNB + 1], float *rd) {
+    if (threadIdx.x < kNB) rd[threadIdx.x] = 1.0f / t[threadIdx.x][threadIdx.x];
+    __syncthreads();
+}
+
+// Solves of 64 entries a line with a 64 x 64 triangle t in LDS: rows
+// x <- x U^-1 (kUp; RUNN, x_j = (b_j - sum_{l<j} x_l u_lj) rd_j) or columns
+// y <- L^-1 y (LLNU, unit L).  The calling wave owns 16 lines of xs (its
+// rows; nothing else reads or writes them), xs[line][entry].  Entries go in
+// four blocks of 16: inside a block a quad of lanes has a line, lane q the
+// entries q, q + 4, q + 8, q + 12 (step j: the owner, lane j % 4, finalises
+// entry j, the quad reads it with a DPP broadcast, later entries take one
+// fused multiply-add each); then the block's product with the triangle is
+// taken off the later blocks on the matrix cores (v_mfma_f32_16x16x4_f32:
+// lane = line, registers = entries).  The FP32 MFMAs add their products one
+// by one, each rounded as a fused multiply-add, so every entry still gets its
+// terms in the order l = 0, 1, ... with one rounding each, as in
+// column-by-column substitution.  The code is a loop over the blocks on
+// purpose: 64 unrolled steps are 16 KB of instructions that every launch
+// fetches anew, which took longer than the steps.
+constexpr int kXS = kNB + 4;  // row stride of xs: conflict-free operand reads, 16-byte aligned rows
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Step j of a block.  kUp: x holds b_j - sum until the end, where its owner
+// scales it as every lane does here.
+template <int j, bool kUp>
+__device__ __forceinline__ void tri16_step(float (&x)[4], int q, const float (&e)[16][4], const float (&r)[16]) {
     constexpr int o = j & 3, s = j >> 2;
-    const float cand = x[s] * rd[j];
-    const float xj = quad_bcast<o>(cand);
-    if (q == o) x[s] = xj;
-    if (q > o) x[s] = __builtin_fmaf(-xj, u[j][q + 4 * s], x[s]);
+    const float xj = quad_bcast<o>(kUp ? x[s] * r[j] : x[s]);
+    if (o < 3) {
+        const float later = __builtin_fmaf(-xj, e[j][s], x[s]);
+        x[s] = q > o ? later : x[s];
+    }
 #pragma unroll
-    for (int t = s + 1; t < 16; ++t) x[t] = __builtin_fmaf(-xj, u[j][q + 4 * t], x[t]);
+    for (int t = s + 1; t < 4; ++t) x[t] = __builtin_fmaf(-xj, e[j][t], x[t]);
 }
 
-template <int j>
-__device__ __forceinline__ void llnu_step(float (&y)[16], int q, const float (*l)[kNB + 1]) {
-    constexpr int o = j & 3, s = j >> 2;
-    const float t = quad_bcast<o>(y[s]);
-    if (q > o) y[s] = __builtin_fmaf(-t, l[q + 4 * s][j], y[s]);
-#pragma unroll
-    for (int w = s + 1; w < 16; ++w) y[w] = __builtin_fmaf(-t, l[q + 4 * w][j], y[w]);
+template <bool kUp, int... J>
+__device__ __forceinline__ void tri16_steps(float (&x)[4], int q, const float (&e)[16][4], const float (&r)[16],
+                                            std::integer_sequence<int, J...>) {
+    (tri16_step<J, kUp>(x, q, e, r), ...);
 }
 
-template <int... J>
-__device__ __forceinline__ void runn_all(float (&x)[16], int q, const float (*u)[kNB + 1], const float *rd,
-                                         std::integer_sequence<int, J...>) {
-    (runn_step<J>(x, q, u, rd), ...);
+template <bool kUp>
+__device__ __forceinline__ void tri_solve64(float (*xs)[kXS], const float (*t)[kNB + 1], const float *rd) {
+    const int lane = threadIdx.x & 63, q = lane & 3;
+    const int i16 = lane & 15, g = lane >> 4;
+#pragma unroll 1
+    for (int c0 = 0; c0 < kNB; c0 += 16) {
+        float x[4], e[16][4], r[16], a[3][4];
+        float *line = xs[lane >> 2] + c0 + q;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = line[4 * u];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            if (kUp) r[j] = rd[c0 + j];
+#pragma unroll
+            for (int u = j >> 2; u < 4; ++u)
+                e[j][u] = kUp ? t[c0 + j][c0 + q + 4 * u] : t[c0 + q + 4 * u][c0 + j];
+        }
+        // the triangle's operands of the later blocks' products (past the
+        // last block: read from within the triangle, not used)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const int cb = (c0 + 16 * (b + 1)) & (kNB - 1);
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                const int k = c0 + 4 * kk + g;
+                a[b][kk] = kUp ? t[k][cb + i16] : t[cb + i16][k];
+            }
+        }
+        tri16_steps<kUp>(x, q, e, r, std::make_integer_sequence<int, 16>{});
+        if (kUp) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] *= rd[c0 + q + 4 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) line[4 * u] = x[u];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // the solved block's operand: line i16, entry c0 + 4 kk + g
+        float xk[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) xk[kk] = -xs[i16][c0 + 4 * kk + g];
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const int cb = c0 + 16 * (b + 1);
+            if (cb < kNB) {
+                f32x4 *dst = reinterpret_cast<f32x4 *>(&xs[i16][cb + 4 * g]);
+                f32x4 acc = *dst;
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[b][kk], xk[kk], acc, 0, 0, 0);
+                *dst = acc;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
 }
 
-template <int... J>
-__device__ __forceinline__ void llnu_all(float (&y)[16], int q, const float (*l)[kNB + 1],
-                                         std::integer_sequence<int, J...>) {
-    (llnu_step<J>(y, q, l), ...);
-}
-
-// Row i: X(i, :) <- X(i, :) * U^-1 for a 64 x 64 upper non-unit U (RUNN);
-// x_j = (b_j - sum_{l<j} x_l u_lj) * rd_j with rd_j = 1 / u_jj (correctly
-// rounded, formed once per workgroup).  Called by the four lanes of a quad
-// with the same i (q = lane % 4).
-__device__ __forceinline__ void row_runn64(int64_t i, int q, const float (*u)[kNB + 1], const float *rd,
-                                           float *__restrict__ X, int64_t ldx) {
-    float x[16];
-#pragma unroll
-    for (int t = 0; t < 16; ++t) x[t] = X[i + (q + 4 * t) * ldx];
-    runn_all(x, q, u, rd, std::make_integer_sequence<int, kNB>{});
-#pragma unroll
-    for (int t = 0; t < 16; ++t) X[i + (q + 4 * t) * ldx] = x[t];
-}
-
-// Column j: Y(:, j) <- L^-1 Y(:, j) for a 64 x 64 unit lower L (LLNU);
-// y_i -= y_c l_ic for c < i, c ascending.  Called by a quad as above.
-__device__ __forceinline__ void col_llnu64(int64_t j, int q, const float (*l)[kNB + 1], float *__restrict__ Y,
-                                           int64_t ldy) {
-    float y[16];
-    float *col = Y + j * ldy;
-#pragma unroll
-    for (int t = 0; t < 16; ++t) y[t] = col[q + 4 * t];
-    llnu_all(y, q, l, std::make_integer_sequence<int, kNB>{});
-#pragma unroll
-    for (int t = 0; t < 16; ++t) col[q + 4 * t] = y[t];
-}
-
-// 64 rows (or columns) per workgroup of 256 threads, a quad per row.  The
-// quad's lanes stay together: a row past the end exits as a whole quad.
+// 64 rows per workgroup of 256 threads, 16 per wave: X(i, :) <- X(i, :) U^-1.
+// Rows past m are read as row m - 1 and not stored.
 __global__ void __launch_bounds__(256)
 k_trsm_rows_runn64(int64_t m, const float *__restrict__ U, int64_t ldu, float *__restrict__ X,
                    int64_t ldx) {
     __shared__ float u[kNB][kNB + 1];
+    __shared__ __align__(16) float xs[kNB][kXS];
     __shared__ float rd[kNB];
+    // element (row, column): lanes along the rows, 16 columns a wave
+    const int r = threadIdx.x & 63, c0 = 16 * (threadIdx.x >> 6);
+    const int64_t i = (int64_t)blockIdx.x * 64 + r;
+    float *row = X + (i < m ? i : m - 1) + (int64_t)c0 * ldx;
+    float v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = row[c * ldx];
     load_tri64(U, ldu, u);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) xs[r][c0 + c] = v[c];
     diag_recip64(u, rd);
-    const int64_t i = (int64_t)blockIdx.x * 64 + (threadIdx.x >> 2);
-    if (i < m) row_runn64(i, threadIdx.x & 3, u, rd, X, ldx);
+    tri_solve64<true>(xs + c0, u, rd);
+    __syncthreads();
+    if (i < m) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) row[c * ldx] = xs[r][c0 + c];
+    }
 }
 
+// 64 columns per workgroup, 16 per wave: Y(:, j) <- L^-1 Y(:, j).  Columns
+// past n are read as column n - 1 and not stored.
 __global__ void __launch_bounds__(256)
 k_trsm_cols_llnu64(int64_t n, const float *__restrict__ L, int64_t ldl, float *__restrict__ Y,
                    int64_t ldy) {
     __shared__ float l[kNB][kNB + 1];
+    __shared__ __align__(16) float ys[kNB][kXS];
+    const int r = threadIdx.x & 63, c0 = 16 * (threadIdx.x >> 6);
+    const int64_t j = (int64_t)blockIdx.x * 64 + c0;
+    float v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = Y[r + min(j + c, n - 1) * ldy];
     load_tri64(L, ldl, l);
-    const int64_t j = (int64_t)blockIdx.x * 64 + (threadIdx.x >> 2);
-    if (j < n) col_llnu64(j, threadIdx.x & 3, l, Y, ldy);
+    // (the wave's own columns: no barrier before it solves them)
+#pragma unroll
+    for (int c = 0; c < 16; ++c) ys[c0 + c][r] = v[c];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    tri_solve64<false>(ys + c0, l, nullptr);
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+        if (j + c < n) Y[r + (j + c) * ldy] = ys[c0 + c][r];
 }
 
-// One 64-column step of the blocked LU in one launch.  Every workgroup
-// factors the 64 x 64 diagonal block D at Ajj itself (wave 0, lu64_wave;
-// all get the same factors) into LDS; workgroup 0 reports zero pivots.
-// Then workgroups [0, nrw) solve the rows below D (RUNN with D's U), the
-// next nrw the columns right of D (LLNU with D's unit L), 64 per workgroup,
-// a quad per row or column; rest = rows below = columns right of D.  Each
-// quad's entries are loaded before the factorisation, so the loads overlap
-// it.
-// No workgroup writes D back in its own step: the workgroups of a launch
-// need not run at the same time (a concurrent kernel may hold the CUs), so
-// one that starts after D was overwritten would factor the factors.  The
-// factored D of the previous step (still the original in memory, and read
-// by no other workgroup of this launch) is written by one more workgroup,
-// the last one (index max(1, 2 nrw)), when prev is set; the last step's
-// workgroup 0, with nothing below or right of D, writes its own D.
-__global__ void __launch_bounds__(256)
-k_getrf_step64(int64_t rest, int nrw, float *__restrict__ Ajj, int64_t lda, int64_t row0, int *__restrict__ info,
-               int prev) {
-    __shared__ float d[kNB][kNB + 1];
-    __shared__ float rd[kNB];
-    const int tid = threadIdx.x, q = tid & 3;
-    if (prev && (int)blockIdx.x == (nrw > 0 ? 2 * nrw : 1)) {
-        // the previous step's diagonal block, 64 rows and columns up
-        if (tid < kNB) {
-            float *Dp = Ajj - kNB - kNB * lda;
-            float r[kNB];
+// ---------------------------------------------------------------------------
+// One 64-column step j of the blocked LU in one launch, the rank-64 update
+// of the step before (p = j - 64) included.  At its start the column block
+// L_p = A(j.., p) and the row block U_p = A(p, j..) are final and everything
+// at and beyond (j, j) still lacks their product.  Workgroups of 512 threads:
+//   [0, np)        128 rows of the column block j each: the 64 x 64 diagonal
+//                  block D = A_jj - L_p U_p is formed and factored by every
+//                  one of them for itself (into LDS; all get the same
+//                  factors), the rows receive their update and are solved
+//                  with D's U;
+//   [np, 2 np)     128 columns of the row block j likewise, with D's unit L;
+//   1 more (j > 0) D_p, factored once more as in the step before, is written
+//                  (in its own step other workgroups, which need not all run
+//                  at the same time, still read the original);
+//   the rest       the 128 x 64 tiles beyond row and column block j: the
+//                  update alone.
+// The last step's workgroup 0, with nothing below or right of D, writes its
+// own D.  What bounds a step is the chain of one such workgroup (launch,
+// loads, 64 pivots, 64 solve steps), not its operations: with the update in a
+// launch of its own and D factored by one wave a step took 34 us at n = 2560
+// and 36 us at n = 256 (idle GPU), now 20.5 and 15.5 us, with the same
+// factors bit for bit; beside the LU's trailing product, where every
+// launch waits for CUs, half the launches wait.
+//
+// D is factored by eight waves, wave w holding columns 8 w .. 8 w + 7 with
+// lane i = row i: wave s factors its 8 columns (row k read from lane k with
+// v_readlane; multipliers x reciprocal pivot, as sgetrf_nopiv_naive) and
+// hands each over through LDS; the waves beyond apply it meanwhile.  A wave's
+// part of the tile's update (32 x 32, 32 MFMAs) follows its own columns.
+//
+// Operands: L_p straight from global memory (a lane's row, 32 consecutive
+// rows per half-wave: the MFMA's second operand), U_p, contiguous along k,
+// through LDS (the first).  n is a multiple of 64; rows and columns past n of
+// a last, half-empty 128-tile are clamped and not stored.
+// ---------------------------------------------------------------------------
+constexpr int kGT = 512;           // threads
+constexpr int kUS = kXS;           // row stride of the staged U_p: conflict-free 16-byte reads
+
+struct __align__(16) GetrfShared {
+    float su[kNB][kUS];       // U_p, columns of block j (or of the trailing tile): su[c][k]
+    float sx[2 * kNB][kUS];   // U_p, the 128 columns of a row-block workgroup; then the tile to solve
+    float d[kNB][kNB + 1];    // D
+    float rd[kNB];            // reciprocal pivots
+    int prog;                 // columns of D factored so far
+};
+
+// Columns [0, 32 kN) of U (64 rows, leading dimension ld), 16 bytes per thread
+// of 32 columns each, into registers; columns at or past cmax are read as
+// column cmax - 1.  put_u: to su[c][k].
+template <bool kVec, int kN>
+__device__ __forceinline__ void get_u(const float *__restrict__ U, int64_t ld, int64_t cmax, f32x4 (&v)[kN]) {
+    const int k = 4 * (threadIdx.x & 15), c = threadIdx.x >> 4;
 #pragma unroll
-            for (int j = 0; j < kNB; ++j) r[j] = Dp[tid + (int64_t)j * lda];
-            lu64_wave(r, tid, row0 - kNB, nullptr);
+    for (int i = 0; i < kN; ++i) {
+        const float *g = U + min((int64_t)(c + 32 * i), cmax - 1) * ld + k;
+        v[i] = kVec ? *reinterpret_cast<const f32x4 *>(g) : f32x4{g[0], g[1], g[2], g[3]};
+    }
+}
+
+// The update's 64 products of an entry are summed in the order of the products
+// that the library would launch for it: k_sgemm_mfma (0, 32, 1, 33, ...: a
+// lane of half h takes k = 32 h + s in its s-th MFMA) or, for small or
+// unaligned blocks, k_sgemm_nn (0, 1, 2, ..: k = 2 s + h; seq).  su holds
+// k in that order: lane half h reads positions 32 h .. 32 h + 31.
+template <int kN>
+__device__ __forceinline__ void put_u(const f32x4 (&v)[kN], float (*su)[kUS], bool seq) {
+    const int k = 4 * (threadIdx.x & 15), c = threadIdx.x >> 4;
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-            for (int j = 0; j < kNB; ++j) Dp[tid + (int64_t)j * lda] = r[j];
+    for (int i = 0; i < kN; ++i) {
+        float *d = su[c + 32 * i];
+        if (seq) {
+            *reinterpret_cast<f32x2 *>(d + k / 2) = f32x2{v[i].x, v[i].z};
+            *reinterpret_cast<f32x2 *>(d + 32 + k / 2) = f32x2{v[i].y, v[i].w};
+        } else {
+            *reinterpret_cast<f32x4 *>(d + k) = v[i];
+        }
+    }
+}
+
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+// a lane's row of L_p (pointer to it at column 0): 32 of the 64 columns, by
+// half-wave and order (put_u)
+__device__ __forceinline__ void load_l(const float *__restrict__ row, int64_t ld, int h, bool seq, f32x32 &l) {
+    const float *g = row + (seq ? h : 32 * h) * ld;
+    const int64_t step = seq ? 2 * ld : ld;
+#pragma unroll
+    for (int s = 0; s < 32; ++s) l[s] = g[s * step];
+}
+
+// four of the 32 products of a wave's 32 x 32 block: acc[v] is row lane % 32,
+// column 8 (v / 4) + 4 (lane / 32) + v % 4; su is the lane's column of U_p
+// from k = 32 (lane / 32) on
+__device__ __forceinline__ void mfma4(const f32x32 &l, const float *su, int g, f32x16 &acc) {
+    const f32x4 y = *reinterpret_cast<const f32x4 *>(su + 4 * g);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[u], l[4 * g + u], acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ void mfma32(const f32x32 &l, const float *su, f32x16 &acc) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g) mfma4(l, su, g, acc);
+}
+
+// LDS hand-over between the waves; outstanding global loads stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// LDS accesses that other waves of the workgroup watch: relaxed atomics, which
+// stay in program order (volatile ones wait for their completion each time)
+template <class T>
+__device__ __forceinline__ T lds_get(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+template <class T>
+__device__ __forceinline__ void lds_put(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// 1 / u: the hardware reciprocal (1 ulp) and one Newton step, 3 dependent
+// instructions in the pivots' chain where the division has 11.  For pivots
+// that pivot_ok admits; the others take the division (kDiv).
+template <bool kDiv>
+__device__ __forceinline__ float pivot_recip(float u) {
+    if (kDiv) return 1.0f / u;
+    const float y = __builtin_amdgcn_rcpf(u);
+    return __builtin_fmaf(__builtin_fmaf(-u, y, 1.0f), y, y);
+}
+
+// neither u nor 1 / u subnormal, zero, infinite or NaN
+__device__ __forceinline__ bool pivot_ok(float u) {
+    const int ex = (__builtin_bit_cast(int, u) >> 23) & 255;
+    return ex >= 4 && ex <= 250;
+}
+
+// Factorisation of sh.d (see above) by the calling wave's share.  Columns
+// are handed over one by one: the wave that factors writes column g of the
+// factors to sh.d, then sh.prog = g + 1 (LDS operations of a wave complete in
+// order); a wave that waits for it reads both at once, the next column's while
+// it applies the current one.  What it costs is instructions: a wave issues
+// one in about six cycles, dependent or not.  A loop over the stages:
+// unrolled, they are 30 KB of instructions to fetch in every launch.
+template <bool kDiv>
+__device__ __forceinline__ void lu_stages(float (&r)[8], int lane, int wave, GetrfShared &sh) {
+    float *col = &sh.d[lane][0];
+#pragma unroll 1
+    for (int s = 0; s < wave; ++s) {
+        int f = lds_get(&sh.prog);
+        float mg = lds_get(&col[8 * s]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int g = 8 * s + k;
+            while (f <= g) {
+                if (s + 1 < wave) __builtin_amdgcn_s_sleep(2);
+                f = lds_get(&sh.prog);
+                mg = lds_get(&col[g]);
+            }
+            const float m = lane > g ? mg : 0.0f;
+            if (k < 7) {
+                f = lds_get(&sh.prog);
+                mg = lds_get(&col[g + 1]);
+            }
+            float u[8];  // the pivot row, read together: a read just before its use waits
+#pragma unroll
+            for (int c = 0; c < 8; ++c) u[c] = lane_bcast(r[c], g);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) r[c] = __builtin_fmaf(-m, u[c], r[c]);
+        }
+    }
+    const int g0 = 8 * wave, ln = lane - g0;
+    int pv = g0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float inv = pivot_recip<kDiv>(lane_bcast(r[k], g0 + k));
+        // rows at or above the pivot take multiplier 0: fma(-0, u, r) leaves
+        // r as it is (up to the sign of a zero)
+        const float m = (ln > k ? r[k] : 0.0f) * inv;
+        r[k] = ln > k ? m : r[k];
+        lds_put(&col[g0 + k], r[k]);
+        asm volatile("v_add_u32 %0, 1, %0" : "+v"(pv));
+        lds_put(&sh.prog, pv);  // (every lane the same value: no branch)
+        float u[8];
+#pragma unroll
+        for (int c = k + 1; c < 8; ++c) u[c] = lane_bcast(r[c], g0 + k);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = k + 1; c < 8; ++c) r[c] = __builtin_fmaf(-m, u[c], r[c]);
+    }
+}
+
+// A: the order-n block; j: first column of the step; np: 128-row workgroups
+// of the column block (= those of the row block); nti: of them a column of
+// trailing tiles has; first: info is set, not lowered
+template <bool kUpd, bool kVec>
+__global__ void __launch_bounds__(kGT) __attribute__((amdgpu_waves_per_eu(4)))
+k_getrf_step64(int64_t n, int64_t j, int np, float *__restrict__ A, int64_t lda, int *__restrict__ info) {
+    __shared__ GetrfShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bid = blockIdx.x;
+    const int nch = np > 0 ? 2 * np : 1;  // workgroups that solve (the last step: that factors)
+    const bool trail = kUpd && bid > nch;
+    const bool writer = kUpd && bid == nch;
+    const bool cols = !trail && !writer && bid >= np && np > 0;
+    const bool solve = !trail && !writer && np > 0;
+    // the step whose D this workgroup factors, and whose update it applies
+    const int64_t jj = writer ? j - kNB : j;
+    const bool upd = kUpd && jj > 0;
+    const bool seq = !kVec || !mfma_size(n - jj, n - jj, 1);
+    const float *Lp = A + (jj - kNB) * lda;         // column block p: row i at Lp + i
+    const float *Up = A + (jj - kNB);               // row block p: column c at Up + c lda
+    // the tile: rows from i0, columns from c0; the wave's 32 x 32 block of it
+    int64_t i0 = j + kNB, c0 = j;
+    int wr = 32 * (wave & 3), wc = 32 * (wave >> 2);
+    if (trail) {
+        const int t = bid - nch - 1;
+        i0 = j + kNB + (int64_t)(t % np) * 128;
+        c0 = j + kNB + (int64_t)(t / np) * kNB;
+    } else if (cols) {
+        i0 = j;
+        c0 = j + kNB + (int64_t)(bid - np) * 128;
+        wr = 32 * (wave & 1);
+        wc = 32 * (wave >> 1);
+    } else if (solve) {
+        i0 = j + kNB + (int64_t)bid * 128;
+    }
+    f32x16 acc;
+    f32x32 l;
+    float cv[16];
+    const int64_t row = min(i0 + wr + l32, n - 1);  // the lane's row of the tile
+    if (trail) {
+        f32x4 u2[2];
+        get_u<kVec>(Up + c0 * lda, lda, kNB, u2);
+        load_l(Lp + row, lda, h, seq, l);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            acc[v] = 0.0f;
+            cv[v] = A[row + (c0 + wc + 8 * (v >> 2) + 4 * h + (v & 3)) * lda];
+        }
+        put_u(u2, sh.su, seq);
+        lds_barrier();
+        mfma32(l, &sh.su[wc + l32][32 * h], acc);
+        if (i0 + wr + l32 < n) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                A[row + (c0 + wc + 8 * (v >> 2) + 4 * h + (v & 3)) * lda] = cv[v] - acc[v];
         }
         return;
     }
-    const bool rows = (int)blockIdx.x < nrw;
-    const int64_t e = (int64_t)(rows ? (int)blockIdx.x : (int)blockIdx.x - nrw) * 64 + (tid >> 2);
-    const bool act = e < rest;
-    // row e below D: entries (e, q + 4 t); column e right of D: (q + 4 t, e)
-    float *base = rows ? Ajj + kNB + e : Ajj + (kNB + e) * lda;
-    const int64_t step = rows ? lda : 1;
-    float x[16];
-    if (act) {
-#pragma unroll
-        for (int t = 0; t < 16; ++t) x[t] = base[(q + 4 * t) * step];
+    // (a trailing tile may share the CU; the chain goes first)
+    __builtin_amdgcn_s_setprio(3);
+    // D - L_p U_p into LDS, a 32 x 32 quadrant by each of waves 0-3; all
+    // loads first, the products' operands before the rest
+    const int dr = 32 * (wave & 1), dc = 32 * ((wave >> 1) & 1);
+    f32x4 u2[2], u4[4];
+    if (upd) {
+        get_u<kVec>(Up + jj * lda, lda, kNB, u2);
+        if (wave < 4) load_l(Lp + jj + dr + l32, lda, h, seq, l);
+        if (cols) get_u<kVec>(Up + c0 * lda, lda, n - c0, u4);
     }
-    if (tid < kNB) {
-        float r[kNB];
+    if (wave < 4) {
+        const float *dp = A + jj + dr + l32;
 #pragma unroll
-        for (int j = 0; j < kNB; ++j) r[j] = Ajj[tid + (int64_t)j * lda];
-        lu64_wave(r, tid, row0, blockIdx.x == 0 ? info : nullptr);
-#pragma unroll
-        for (int j = 0; j < kNB; ++j) d[tid][j] = r[j];
-        if (nrw == 0) {
-#pragma unroll
-            for (int j = 0; j < kNB; ++j) Ajj[tid + (int64_t)j * lda] = r[j];
+        for (int v = 0; v < 16; ++v) {
+            acc[v] = 0.0f;
+            cv[v] = dp[(jj + dc + 8 * (v >> 2) + 4 * h + (v & 3)) * lda];
         }
     }
-    __syncthreads();
-    diag_recip64(d, rd);
-    if (!act) return;
-    if (rows)
-        runn_all(x, q, d, rd, std::make_integer_sequence<int, kNB>{});
-    else
-        llnu_all(x, q, d, std::make_integer_sequence<int, kNB>{});
+    if (tid == 0) sh.prog = 0;
+    if (upd) {
+        put_u(u2, sh.su, seq);
+        if (cols) put_u(u4, sh.sx, seq);
+    }
+    lds_barrier();
+    if (wave < 4) {
+        if (upd) mfma32(l, &sh.su[dc + l32][32 * h], acc);
 #pragma unroll
-    for (int t = 0; t < 16; ++t) base[(q + 4 * t) * step] = x[t];
+        for (int v = 0; v < 16; ++v) sh.d[dr + l32][dc + 8 * (v >> 2) + 4 * h + (v & 3)] = cv[v] - acc[v];
+    }
+    if (solve) {
+        // the tile's operands, in flight during the factorisation
+        if (upd) load_l(Lp + row, lda, h, seq, l);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            acc[v] = 0.0f;
+            cv[v] = A[row + min(c0 + wc + 8 * (v >> 2) + 4 * h + (v & 3), n - 1) * lda];
+        }
+    }
+    lds_barrier();
+    float r[8], r0[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = r0[k] = sh.d[lane][8 * wave + k];
+    lu_stages<false>(r, lane, wave, sh);
+    // the tile's update, after the wave's own stage
+    if (kUpd && solve) mfma32(l, cols ? &sh.sx[wc + l32][32 * h] : &sh.su[wc + l32][32 * h], acc);
+    lds_barrier();
+    float piv = sh.d[lane][lane];
+    if (__builtin_expect(!__all(pivot_ok(piv)), 0)) {
+        // (every wave sees the same pivots) once more, with divisions
+        lds_barrier();
+        if (tid == 0) sh.prog = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) r[k] = r0[k];
+        lds_barrier();
+        lu_stages<true>(r, lane, wave, sh);
+        lds_barrier();
+        piv = sh.d[lane][lane];
+    }
+    if (wave == 0) sh.rd[lane] = 1.0f / piv;
+    if (bid == 0 && wave == 0 && info) {
+        const uint64_t zero = __ballot(piv == 0.0f);
+        const int b = zero ? (int)jj + (int)__builtin_ctzll(zero) + 1 : 0x7fffffff;
+        if (lane == 0) {
+            if (!kUpd)
+                *info = b;  // the first step sets it
+            else if (zero)
+                atomicMin(info, b);
+        }
+    }
+    if (!solve) {
+        // the previous step's D, or the last one's own
+#pragma unroll
+        for (int k = 0; k < 8; ++k) A[jj + lane + (jj + 8 * wave + k) * lda] = r[k];
+        return;
+    }
+    // the tile into LDS, a line to solve per row of sx; 16 lines a wave
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int rr = wr + l32, cc = wc + 8 * (v >> 2) + 4 * h + (v & 3);
+        sh.sx[cols ? cc : rr][cols ? rr : cc] = cv[v] - acc[v];
+    }
+    lds_barrier();
+    if (cols)
+        tri_solve64<false>(sh.sx + 16 * wave, sh.d, nullptr);
+    else
+        tri_solve64<true>(sh.sx + 16 * wave, sh.d, sh.rd);
+    lds_barrier();
+    // lanes along the matrix rows (of a row-block tile: the wave's own lines)
+    if (cols) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int64_t col = c0 + 16 * wave + c;
+            if (col < n) A[j + lane + col * lda] = sh.sx[16 * wave + c][lane];
+        }
+    } else {
+        const int e = tid & 127, cq = 16 * (tid >> 7);
+        if (i0 + e < n) {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) A[i0 + e + (j + cq + c) * lda] = sh.sx[e][cq + c];
+        }
+    }
 }
 
 // Rows: X(i, :) <- X(i, :) * L^-1 for a 64 x 64 unit lower L (RLNU),
@@ -489,32 +821,30 @@ k_trsm_rows_rlnu64(int64_t m, const float *__restrict__ L, int64_t ldl, float *_
 
 // Inverses of the 64 x 64 diagonal blocks of the factored block D (L unit
 // lower, U upper in one array): workgroup w < nblk writes U_ww^-1 into Xu
-// (row r of it = e_r U_ww^-1, a RUNN row solve of the identity row by a lane
-// quad), workgroup nblk + w writes L_ww^-1 into Xl (column c = L_ww^-1 e_c,
-// an LLNU column solve by a lane quad).
+// (row r of it = e_r U_ww^-1, a row solve of the identity), workgroup nblk + w
+// writes L_ww^-1 into Xl (column c = L_ww^-1 e_c).
 __global__ void __launch_bounds__(256)
 k_tri_inv64(int nblk, const float *__restrict__ D, int64_t ldd, float *__restrict__ Xu, float *__restrict__ Xl,
             int64_t ldx) {
     __shared__ float t[kNB][kNB + 1];
+    __shared__ __align__(16) float xs[kNB][kXS];
     __shared__ float rd[kNB];
     const bool up = (int)blockIdx.x < nblk;
     const int64_t o = (int64_t)(up ? blockIdx.x : blockIdx.x - nblk) * kNB;
-    load_tri64(D + o + o * ldd, ldd, t);
-    const int q = threadIdx.x & 3, r = threadIdx.x >> 2;
-    float v[16];
+    const int lane = threadIdx.x & 63, w0 = 16 * (threadIdx.x >> 6);
 #pragma unroll
-    for (int s = 0; s < 16; ++s) v[s] = (q + 4 * s == r) ? 1.0f : 0.0f;
+    for (int c = 0; c < 16; ++c) xs[w0 + c][lane] = w0 + c == lane ? 1.0f : 0.0f;
+    load_tri64(D + o + o * ldd, ldd, t);
     if (up) {
         diag_recip64(t, rd);
-        runn_all(v, q, t, rd, std::make_integer_sequence<int, kNB>{});
-        float *row = Xu + o + r + o * ldx;
+        tri_solve64<true>(xs + w0, t, rd);
+        __syncthreads();
 #pragma unroll
-        for (int s = 0; s < 16; ++s) row[(q + 4 * s) * ldx] = v[s];
+        for (int c = 0; c < 16; ++c) Xu[o + lane + (o + w0 + c) * ldx] = xs[lane][w0 + c];
     } else {
-        llnu_all(v, q, t, std::make_integer_sequence<int, kNB>{});
-        float *col = Xl + o + (o + r) * ldx;
+        tri_solve64<false>(xs + w0, t, nullptr);
 #pragma unroll
-        for (int s = 0; s < 16; ++s) col[q + 4 * s] = v[s];
+        for (int c = 0; c < 16; ++c) Xl[o + lane + (o + w0 + c) * ldx] = xs[w0 + c][lane];
     }
 }
 
@@ -543,23 +873,11 @@ __global__ void k_copy_block(int64_t m, const float *__restrict__ A, int64_t lda
         B[i + j * ldb] = A[i + j * lda];
 }
 
-__global__ void k_set_int(int *p, int v) { *p = v; }
-
-// The MFMA kernel takes products with at least this many C entries per
-// launch (2^18 = 512 x 512; smaller ones are latency-bound and the 64 x 64
-// VALU tiles spread them over more CUs) when its alignment conditions hold.
-#ifndef OMX_SGEMM_MFMA_T64
-#define OMX_SGEMM_MFMA_T64 1024
-#endif
-#ifndef OMX_SGEMM_MFMA_MIN
-#define OMX_SGEMM_MFMA_MIN (int64_t{1} << 18)
-#endif
-
 bool use_mfma(int64_t m, int64_t n, int64_t k, int64_t batch, const float *A, int64_t lda, const float *B,
               int64_t ldb) {
     const bool aligned = (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (reinterpret_cast<uintptr_t>(B) & 15) == 0 &&
                          (lda & 3) == 0 && (ldb & 3) == 0 && k >= 16 && k % 16 == 0;
-    return aligned && m * n * batch >= OMX_SGEMM_MFMA_MIN;
+    return aligned && mfma_size(m, n, batch);
 }
 
 int sgemm_mfma(int64_t m, int64_t n, int64_t k, float alpha, const float *A, int64_t lda, int64_t sA, const float *B,
@@ -645,22 +963,23 @@ int omx_sgemm_f32(int64_t m, int64_t n, int64_t k, float alpha, const float *A, 
 int omx_getrf_nopiv_f32(int64_t n, float *A, int64_t lda, int *info, void *stream) {
     if (n <= 0 || n % kNB || !A || lda < n) return OMX_ERR_ARG;
     hipStream_t st = omx_stream(stream);
-    if (info) {
-        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, st, info, 0x7fffffff);
-        OMX_LAUNCH_CHECK();
-    }
+    const bool vec = (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (lda & 3) == 0;
     for (int64_t j = 0; j < n; j += kNB) {
-        float *Ajj = A + j + j * lda;
         const int64_t rest = n - j - kNB;
-        const int nrw = (int)omx_cdiv(rest, 64);
-        const int prev = j > 0 ? 1 : 0;  // one more workgroup writes the previous step's factored D
-        hipLaunchKernelGGL(k_getrf_step64, dim3((unsigned)(std::max(1, 2 * nrw) + prev)), dim3(256), 0, st, rest, nrw,
-                           Ajj, lda, j, info, prev);
+        const int64_t np = omx_cdiv(rest, 128);
+        int64_t grid = np > 0 ? 2 * np : 1;
+        if (j > 0) grid += 1 + np * (rest / kNB);  // the previous D's writer, the trailing tiles
+        if (grid >= ((int64_t)1 << 31)) return OMX_ERR_ARG;
+        if (j == 0)  // no update yet: nothing is staged
+            hipLaunchKernelGGL((k_getrf_step64<false, false>), dim3((unsigned)grid), dim3(kGT), 0, st, n, j, (int)np,
+                               A, lda, info);
+        else if (vec)
+            hipLaunchKernelGGL((k_getrf_step64<true, true>), dim3((unsigned)grid), dim3(kGT), 0, st, n, j, (int)np, A,
+                               lda, info);
+        else
+            hipLaunchKernelGGL((k_getrf_step64<true, false>), dim3((unsigned)grid), dim3(kGT), 0, st, n, j, (int)np, A,
+                               lda, info);
         OMX_LAUNCH_CHECK();
-        if (rest <= 0) break;
-        int rc = sgemm(rest, rest, kNB, -1.0f, Ajj + kNB, lda, Ajj + kNB * lda, lda, 1.0f,
-                       Ajj + kNB + kNB * lda, lda, st);
-        if (rc) return rc;
     }
     return OMX_OK;
 }

@@ -49,4 +49,61 @@ def test_mlp_step_chunks(B):
     tol = 4 * (64 * 4 + max(82, B / 256) + 256) * 2.0 ** -24
     g = Pd.grad.numpy()
     assert np.max(np.abs(host(G) - g)) <= tol * np.abs(g).max()
-    assert abs(float(host(loss)[0]) - float(want)) <= tol * max(1.0, abs(float(want)))
+    assert abs(float(host(loss)[0]) - want.item()) <= tol * max(1.0, abs(want.item()))
+
+
+def _dominant(n, seed):
+    rng = np.random.default_rng(seed)
+    A = rng.uniform(-0.5, 0.5, (n, n))
+    A[np.arange(n), np.arange(n)] = n / 4 * (1 + 0.1 * rng.uniform(size=n))
+    return A.astype(np.float32)
+
+
+def _getrf(A, lda):
+    """Factors of A by omx_getrf_nopiv_f32 in a buffer of leading dimension lda whose padding must stay."""
+    torch = torch_cuda()
+    n = A.shape[0]
+    buf = np.full((n, lda), 7.0, np.float32)  # buf[j]: column j
+    buf[:, :n] = A.T
+    d, info = dev(buf), empty(1, torch.int32)
+    assert _L().omx_getrf_nopiv_f32(n, ptr(d), lda, ptr(info), None) == 0
+    out = host(d)
+    assert np.all(out[:, n:] == 7.0)
+    return out[:, :n].T.copy(), int(host(info)[0])
+
+
+# one step, half-empty 128-wide tiles, the order of the update's sums changing
+# at 512 rows, aligned and unaligned leading dimensions
+@pytest.mark.parametrize("pad", [0, 4, 1])
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 448, 512, 576, 640, 1088])
+def test_getrf_steps(n, pad):
+    A = _dominant(n, n + pad)
+    F, info = _getrf(A, n + pad)
+    assert info == 0x7fffffff
+    L, U = np.tril(F.astype(np.float64), -1) + np.eye(n), np.triu(F.astype(np.float64))
+    # each entry: n products summed in FP32, one reciprocal and its product
+    bound = (n + 4) * 2.0 ** -24 * (np.abs(L) @ np.abs(U))
+    assert np.all(np.abs(L @ U - A) <= bound)
+
+
+# pivots outside [2^-123, 2^124) take divisions instead of the refined
+# hardware reciprocal: a power-of-two scaling leaves L as it is, bit for bit,
+# and scales U exactly
+@pytest.mark.parametrize("n", [64, 192, 576])
+def test_getrf_extreme_pivots(n):
+    A = _dominant(n, n)
+    F, _ = _getrf(A, n)
+    e = 126 - int(np.ceil(np.log2(np.abs(np.triu(F)).max())))
+    G, info = _getrf((A * np.float32(2.0) ** e).astype(np.float32), n)
+    assert info == 0x7fffffff and np.abs(np.diag(G)).max() >= 2.0 ** 124
+    low = np.tril(np.ones((n, n), bool), -1)
+    assert np.array_equal(F[low], G[low])
+    assert np.array_equal(F[~low].astype(np.float64) * 2.0 ** e, G[~low].astype(np.float64))
+
+
+@pytest.mark.parametrize("n,k", [(64, 0), (64, 63), (192, 70), (576, 511), (576, 575)])
+def test_getrf_reports_the_first_zero_pivot(n, k):
+    # a block-triangular matrix whose column k is zero from row k on
+    A = np.triu(_dominant(n, k))
+    A[k, k] = 0.0
+    assert _getrf(A, n)[1] == k + 1
