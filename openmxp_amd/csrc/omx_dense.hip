@@ -127,18 +127,15 @@ __host__ __device__ __forceinline__ bool mfma_size(int64_t m, int64_t n, int64_t
 }
 
 template <int kT, bool kOneStage>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict__ A, int64_t lda,
-             const float *__restrict__ B, int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
-             int64_t sA, int64_t sB, int64_t sC) {
+__device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, float alpha,
+                                           const float *__restrict__ A, int64_t lda, const float *__restrict__ B,
+                                           int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
+                                           int64_t k0 = 0) {
     constexpr int kB = kT / 64;       // MFMA blocks per quadrant side
     constexpr int kS = kT / 16;       // float4 loads per thread per operand and stage
     constexpr int kAK = 1024 / kT;    // stage columns between a thread's A loads
     __shared__ float As[kMK][kT];     // As[k][i] = A(i0 + i, k0 + k)
     __shared__ float Bs[kT][kBLd];    // Bs[j][k] = B(k0 + k, j0 + j)
-    A += (int64_t)blockIdx.z * sA;
-    B += (int64_t)blockIdx.z * sB;
-    C += (int64_t)blockIdx.z * sC;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, h = lane >> 5;
     const int64_t i0 = (int64_t)blockIdx.x * kT, j0 = (int64_t)blockIdx.y * kT;
@@ -185,9 +182,8 @@ k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restri
         for (int b = 0; b < kB; ++b)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
-    int64_t k0 = 0;
-    int kc = (int)(K < kMK ? K : kMK);
-    OMX_SGEMM_GLOAD(0, kc);
+    int kc = (int)(K - k0 < kMK ? K - k0 : kMK);
+    OMX_SGEMM_GLOAD(k0, kc);
     // kOneStage (K <= 64): C of the wave's quadrant is read now, with the
     // operands, so that its latency overlaps theirs and the MFMAs (rows /
     // columns past the edge read a clamped entry and are not stored);
@@ -268,6 +264,43 @@ k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restri
             }
         }
     }
+}
+
+template <int kT, bool kOneStage>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict__ A, int64_t lda,
+             const float *__restrict__ B, int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
+             int64_t sA, int64_t sB, int64_t sC) {
+    const int64_t z = blockIdx.z;
+    sgemm_tile<kT, kOneStage>(M, N, K, alpha, A + z * sA, lda, B + z * sB, ldb, beta, C + z * sC, ldc);
+}
+
+// Two independent batches of products C_p = alpha A_p B_p in one launch
+// (blockIdx.z below batch: the first): the merges of the two triangular
+// inverses, which would otherwise wait for each other's launches.  tri: one
+// factor is triangular and the tile's k range ends or begins with it (the
+// products left out are exact zeros): 1 B upper (k below the tile's last
+// column), 2 B lower (from its first column), 3 A upper (from its first row),
+// 4 A lower (below its last row).
+struct SgemmTwin {
+    int64_t M, N, K, lda, ldb, ldc, sA, sB, sC;
+    int tri;
+    const float *A, *B;
+    float *C;
+};
+
+template <int kT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_sgemm_twin(SgemmTwin g0, SgemmTwin g1, float alpha, int batch) {
+    const bool second = (int)blockIdx.z >= batch;
+    const SgemmTwin g = second ? g1 : g0;
+    const int64_t z = second ? blockIdx.z - batch : blockIdx.z;
+    const int64_t i0 = (int64_t)blockIdx.x * kT, j0 = (int64_t)blockIdx.y * kT;
+    if (i0 >= g.M || j0 >= g.N) return;
+    const int64_t k0 = g.tri == 2 ? j0 : (g.tri == 3 ? i0 : 0);
+    const int64_t k1 = g.tri == 1 ? j0 + kT : (g.tri == 4 ? i0 + kT : g.K);
+    sgemm_tile<kT, false>(g.M, g.N, k1 < g.K ? k1 : g.K, alpha, g.A + z * g.sA, g.lda, g.B + z * g.sB, g.ldb, 0.0f,
+                          g.C + z * g.sC, g.ldc, k0);
 }
 
 __device__ __forceinline__ float lane_bcast(float v, int l) {
@@ -822,15 +855,28 @@ k_trsm_rows_rlnu64(int64_t m, const float *__restrict__ L, int64_t ldl, float *_
 // Inverses of the 64 x 64 diagonal blocks of the factored block D (L unit
 // lower, U upper in one array): workgroup w < nblk writes U_ww^-1 into Xu
 // (row r of it = e_r U_ww^-1, a row solve of the identity), workgroup nblk + w
-// writes L_ww^-1 into Xl (column c = L_ww^-1 e_c).
+// writes L_ww^-1 into Xl (column c = L_ww^-1 e_c).  The next 8 nblk workgroups
+// clear what neither these nor the merges write, eight columns each: Xu below
+// and Xl above the columns' diagonal block (a launch of its own took 5 us).
 __global__ void __launch_bounds__(256)
 k_tri_inv64(int nblk, const float *__restrict__ D, int64_t ldd, float *__restrict__ Xu, float *__restrict__ Xl,
             int64_t ldx) {
     __shared__ float t[kNB][kNB + 1];
     __shared__ __align__(16) float xs[kNB][kXS];
     __shared__ float rd[kNB];
-    const bool up = (int)blockIdx.x < nblk;
-    const int64_t o = (int64_t)(up ? blockIdx.x : blockIdx.x - nblk) * kNB;
+    const int role = (int)blockIdx.x / nblk;
+    if (role >= 2) {
+        const int64_t n = (int64_t)nblk * kNB, c0 = (int64_t)((int)blockIdx.x - 2 * nblk) * 8;
+        const int64_t o = c0 / kNB * kNB;
+        for (int64_t c = c0; c < c0 + 8; ++c) {
+            float *u = Xu + c * ldx, *l = Xl + c * ldx;
+            for (int64_t i = o + kNB + threadIdx.x; i < n; i += 256) u[i] = 0.0f;
+            for (int64_t i = threadIdx.x; i < o; i += 256) l[i] = 0.0f;
+        }
+        return;
+    }
+    const int64_t o = (int64_t)((int)blockIdx.x % nblk) * kNB;
+    const bool up = role == 0;
     const int lane = threadIdx.x & 63, w0 = 16 * (threadIdx.x >> 6);
 #pragma unroll
     for (int c = 0; c < 16; ++c) xs[w0 + c][lane] = w0 + c == lane ? 1.0f : 0.0f;
@@ -848,16 +894,90 @@ k_tri_inv64(int nblk, const float *__restrict__ D, int64_t ldd, float *__restric
     }
 }
 
-// The entries of the two inverses that k_tri_inv64 and the merges do not
-// write: in column j, Xu below and Xl above j's diagonal 64 x 64 block (the
-// diagonal blocks are written whole, the merges write every off-diagonal
-// block of the other side).  One workgroup per column.
-__global__ void k_zero_offdiag(int64_t n, float *__restrict__ Xu, float *__restrict__ Xl, int64_t ld) {
-    const int64_t j = blockIdx.x;
-    const int64_t top = (j / kNB) * kNB, bot = top + kNB;
-    float *u = Xu + j * ld, *l = Xl + j * ld;
-    for (int64_t i = bot + threadIdx.x; i < n; i += blockDim.x) u[i] = 0.0f;
-    for (int64_t i = threadIdx.x; i < top; i += blockDim.x) l[i] = 0.0f;
+// One level of merges of the two inverses, ranges of up to kMergeMax rows:
+//   U: X12 = -X1 (U12 X2)      L: X21 = -X2 (L21 X1)
+// A workgroup of 512 threads takes 64 columns of one pair's X12 or X21: the
+// inner product W stays in LDS between the two (as separate products a level
+// took four launches of 14-25 us each; this one takes 23 us on average over
+// the ranges of 64, 128 and 256 rows at n = 2560; beyond, the few workgroups
+// a level has would run longer than two launches of more, k_sgemm_twin:
+// 48 us each where the four took 100).  The triangles' zero blocks of
+// 64 are skipped: their products are exact zeros.  Eight waves, 32 x 32 of
+// a 128-row panel each, operands as in k_getrf_step64 (left operand's rows
+// from global memory, right operand's columns, contiguous along k, from LDS)
+// and sums in the order of the products this replaces (put_u).
+constexpr int64_t kMergeMax = 256;
+
+struct __align__(16) MergeShared {
+    float su[kNB][kUS];                // a 64 x 64 block of the right operand: su[c][k]
+    float sw[kNB][kMergeMax + 4];      // W: sw[c][k], each 64 of k in put_u's order
+};
+
+template <bool kVec>
+__global__ void __launch_bounds__(kGT)
+k_tri_merge(int64_t s1, int64_t s2, int64_t a0, const float *__restrict__ D, int64_t ldd, float *__restrict__ Xu,
+            float *__restrict__ Xl, int64_t ldx, int seq_) {
+    __shared__ MergeShared sh;
+    const bool seq = seq_ != 0;
+    const int nu = (int)(s2 / kNB), nl = (int)(s1 / kNB);  // strips of a pair's X12 and X21
+    const int p = (int)blockIdx.x / (nu + nl), t = (int)blockIdx.x % (nu + nl);
+    const bool up = t < nu;
+    const int strip = up ? t : t - nu;
+    a0 += p * (s1 + s2);
+    const int64_t a1 = a0 + s1;
+    float *X = up ? Xu : Xl;
+    const int64_t ra = up ? a0 : a1, ca = up ? a1 : a0;  // the result's place
+    const int64_t m = up ? s1 : s2;                      // its rows
+    const int nk = (int)((up ? s2 : s1) / kNB);          // blocks of the inner product's k
+    const float *P = X + ra + ra * ldx, *Q = D + ra + ca * ldd;
+    const float *R = X + ca + (ca + (int64_t)strip * kNB) * ldx;  // the right operand's columns
+    float *out = X + ra + (ca + (int64_t)strip * kNB) * ldx;
+    const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wc = 32 * (wave >> 2);
+    f32x32 l;
+    f32x16 acc;
+    // W = Q R: R is triangular with its blocks on the diagonal
+    const int k0 = up ? 0 : strip, k1 = up ? strip + 1 : nk;
+    for (int64_t r0 = 0; r0 < m; r0 += 128) {
+        const int64_t row = r0 + 32 * (wave & 3);
+        const bool act = row < m;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll 1
+        for (int k = k0; k < k1; ++k) {
+            f32x4 u2[2];
+            get_u<kVec>(R + (int64_t)k * kNB, ldx, kNB, u2);
+            if (act) load_l(Q + row + l32 + (int64_t)k * kNB * ldd, ldd, h, seq, l);
+            lds_barrier();  // (the block before is read)
+            put_u(u2, sh.su, seq);
+            lds_barrier();
+            if (act) mfma32(l, &sh.su[wc + l32][32 * h], acc);
+        }
+        if (act) {
+            // row index as the k of the second product
+            const int kk = (int)((row + l32) & 63);
+            const int pos = (int)((row + l32) & ~63) + (seq ? (kk & 1) * 32 + (kk >> 1) : kk);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sh.sw[wc + 8 * (v >> 2) + 4 * h + (v & 3)][pos] = acc[v];
+        }
+    }
+    lds_barrier();
+    // result = -P W
+    for (int64_t r0 = 0; r0 < m; r0 += 128) {
+        const int64_t row = r0 + 32 * (wave & 3);
+        if (row >= m) break;
+        const int rb = (int)(row / kNB), nb = (int)(m / kNB);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+#pragma unroll 1
+        for (int k = up ? rb : 0; k < (up ? nb : rb + 1); ++k) {
+            load_l(P + row + l32 + (int64_t)k * kNB * ldx, ldx, h, seq, l);
+            mfma32(l, &sh.sw[wc + l32][kNB * k + 32 * h], acc);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) out[row + l32 + (int64_t)(wc + 8 * (v >> 2) + 4 * h + (v & 3)) * ldx] = -acc[v];
+    }
 }
 
 __global__ void k_identity(int64_t n, float *__restrict__ A, int64_t lda) {
@@ -933,6 +1053,20 @@ int sgemm_batched(int64_t m, int64_t n, int64_t k, float alpha, const float *A, 
     }
     hipLaunchKernelGGL(k_sgemm_nn, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, sA, sB,
                        sC);
+    OMX_LAUNCH_CHECK();
+    return OMX_OK;
+}
+
+// two batches of batch products each (k_sgemm_twin); tiles as sgemm_mfma
+int sgemm_twin(const SgemmTwin &g0, const SgemmTwin &g1, float alpha, int64_t batch, hipStream_t st) {
+    const int64_t m = std::max(g0.M, g1.M), n = std::max(g0.N, g1.N);
+    const bool small = omx_cdiv(m, 128) * omx_cdiv(n, 128) * batch * 2 < OMX_SGEMM_MFMA_T64;
+    const int t = small ? 64 : 128;
+    const dim3 grid((unsigned)omx_cdiv(m, t), (unsigned)omx_cdiv(n, t), (unsigned)(2 * batch));
+    if (small)
+        hipLaunchKernelGGL(k_sgemm_twin<64>, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
+    else
+        hipLaunchKernelGGL(k_sgemm_twin<128>, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
@@ -1055,16 +1189,18 @@ int omx_trtri_lu_f32(int64_t n, const float *D, int64_t ldd, float *Xu, float *X
     if (n <= 0 || n % kNB || n > 65535 || !D || !Xu || !Xl || !work || ldd < n || ldx < n) return OMX_ERR_ARG;
     hipStream_t st = omx_stream(stream);
     const int nblk = (int)(n / kNB);
-    hipLaunchKernelGGL(k_zero_offdiag, dim3((unsigned)n), dim3(256), 0, st, n, Xu, Xl, ldx);
-    OMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(2 * nblk)), dim3(256), 0, st, nblk, D, ldd, Xu, Xl, ldx);
+    hipLaunchKernelGGL(k_tri_inv64, dim3((unsigned)(10 * nblk)), dim3(256), 0, st, nblk, D, ldd, Xu, Xl, ldx);
     OMX_LAUNCH_CHECK();
     // Merge adjacent ranges of diagonal blocks level by level: ranges of s0
     // blocks pair up (the last, odd one waits for a later level).  For the
     // pair [R1 | R2] with inverses X1, X2 on the diagonal:
     //   U: X12 = -X1 (U12 X2)      L: X21 = -X2 (L21 X1)
-    // with the inner product in work (n x n, leading dimension n, at the
-    // position of the block it becomes).  Pairs of equal sizes run batched.
+    // with the inner product in LDS (k_tri_merge) or in work (n x n, leading
+    // dimension n, at the position of the block it becomes).  Pairs of equal
+    // sizes run batched.
+    const bool vec = ((reinterpret_cast<uintptr_t>(D) | reinterpret_cast<uintptr_t>(Xu) |
+                       reinterpret_cast<uintptr_t>(Xl) | reinterpret_cast<uintptr_t>(work)) & 15) == 0 &&
+                     (ldd & 3) == 0 && (ldx & 3) == 0;
     std::vector<int64_t> sz(nblk, kNB);  // range sizes in rows, in order
     while (sz.size() > 1) {
         std::vector<int64_t> next;
@@ -1080,6 +1216,34 @@ int omx_trtri_lu_f32(int64_t n, const float *D, int64_t ldd, float *Xu, float *X
             }
             const int64_t stride = s1 + s2;  // along the diagonal, per pair
             const int64_t a0 = pos, a1 = pos + s1;
+            for (int64_t c = 0; c < cnt; ++c) next.push_back(stride);
+            pos += cnt * stride;
+            if (std::max(s1, s2) <= kMergeMax) {
+                const dim3 grid((unsigned)(cnt * (stride / kNB)));
+                const int seq = vec && mfma_size(s1, s2, cnt) ? 0 : 1;
+                if (vec)
+                    hipLaunchKernelGGL(k_tri_merge<true>, grid, dim3(kGT), 0, st, s1, s2, a0, D, ldd, Xu, Xl, ldx, seq);
+                else
+                    hipLaunchKernelGGL(k_tri_merge<false>, grid, dim3(kGT), 0, st, s1, s2, a0, D, ldd, Xu, Xl, ldx,
+                                       seq);
+                OMX_LAUNCH_CHECK();
+                continue;
+            }
+            const int64_t dstep = stride * (ldd + 1), xstep = stride * (ldx + 1), wstep = stride * (n + 1);
+            if (vec && mfma_size(s1, s2, cnt) && 2 * cnt <= 65535) {
+                // both sides' inner products, then both results
+                const SgemmTwin wu{s1, s2, s2, ldd, ldx, n, dstep, xstep, wstep, 1, D + a0 + a1 * ldd,
+                                   Xu + a1 + a1 * ldx, work + a0 + a1 * n};
+                const SgemmTwin wl{s2, s1, s1, ldd, ldx, n, dstep, xstep, wstep, 2, D + a1 + a0 * ldd,
+                                   Xl + a0 + a0 * ldx, work + a1 + a0 * n};
+                const SgemmTwin xu{s1, s2, s1, ldx, n, ldx, xstep, wstep, xstep, 3, Xu + a0 + a0 * ldx,
+                                   work + a0 + a1 * n, Xu + a0 + a1 * ldx};
+                const SgemmTwin xl{s2, s1, s2, ldx, n, ldx, xstep, wstep, xstep, 4, Xl + a1 + a1 * ldx,
+                                   work + a1 + a0 * n, Xl + a1 + a0 * ldx};
+                RC(sgemm_twin(wu, wl, 1.0f, cnt, st));
+                RC(sgemm_twin(xu, xl, -1.0f, cnt, st));
+                continue;
+            }
             int rc;
             // U: work(a0.., a1..) = U12 X2;  Xu(a0.., a1..) = -X1 work
             rc = sgemm_batched(s1, s2, s2, 1.0f, D + a0 + a1 * ldd, ldd, stride * (ldd + 1), Xu + a1 + a1 * ldx, ldx,
@@ -1095,8 +1259,6 @@ int omx_trtri_lu_f32(int64_t n, const float *D, int64_t ldd, float *Xu, float *X
             rc = sgemm_batched(s2, s1, s2, -1.0f, Xl + a1 + a1 * ldx, ldx, stride * (ldx + 1), work + a1 + a0 * n, n,
                                stride * (n + 1), 0.0f, Xl + a1 + a0 * ldx, ldx, stride * (ldx + 1), cnt, st);
             if (rc) return rc;
-            for (int64_t c = 0; c < cnt; ++c) next.push_back(stride);
-            pos += cnt * stride;
         }
         if (i < sz.size()) next.push_back(sz[i]);
         sz.swap(next);

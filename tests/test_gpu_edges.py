@@ -107,3 +107,27 @@ def test_getrf_reports_the_first_zero_pivot(n, k):
     A = np.triu(_dominant(n, k))
     A[k, k] = 0.0
     assert _getrf(A, n)[1] == k + 1
+
+
+# ranges that pair up evenly, leave an odd one, and pair unequal sizes; merges
+# in LDS (to 256 rows a side) and beyond; aligned and unaligned
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 320, 448, 576, 640, 704, 1088])
+def test_triangular_inverses(n, pad):
+    torch = torch_cuda()
+    F, _ = _getrf(_dominant(n, n), n)
+    ld = n + pad
+    buf = np.zeros((n, ld), np.float32)
+    buf[:, :n] = F.T
+    D = dev(buf)
+    Xu, Xl = (empty(n * ld, torch.float32).fill_(float("nan")) for _ in range(2))
+    W = empty(n * n, torch.float32).fill_(float("nan"))
+    assert _L().omx_trtri_lu_f32(n, ptr(D), ld, ptr(Xu), ptr(Xl), ld, ptr(W), None) == 0
+    L, U = np.tril(F.astype(np.float64), -1) + np.eye(n), np.triu(F.astype(np.float64))
+    for X, T, tri in ((Xu, U, np.triu), (Xl, L, np.tril)):
+        got = host(X).reshape(n, ld)[:, :n].T.astype(np.float64)
+        assert np.array_equal(got, tri(got))
+        want = np.linalg.inv(T)
+        # products of at most n terms at every one of log2(n / 64) + 1 levels
+        tol = 2 * n * 2.0 ** -24 * (np.log2(n / 64) + 1)
+        assert np.all(np.abs(got - want) <= tol * (np.abs(want) @ np.abs(T) @ np.abs(want)))
