@@ -204,16 +204,18 @@ int omx_lowrank_gemv_f64(int64_t n, int64_t rank, const double *sigma,
                          const double *x, double *y, void *work,
                          size_t work_bytes, void *stream);
 
-/* Bytes of scratch the triangular solves need for order n: 0 (they work in
- * place on x); kept so callers written against a workspace-taking solve
- * keep working.  `work` may be NULL. */
+/* Bytes of scratch with which the triangular solves of order n run as one
+ * launch instead of one per 256 columns (n > 512, A 16-byte aligned, lda % 4
+ * == 0, work 8-byte aligned).  They work in place on x without it: `work` may
+ * be NULL or smaller.  Calls that overlap need a workspace each. */
 size_t omx_trsv_workspace_bytes(int64_t n);
 
 /* x <- L^-1 x with L the unit-lower FP32 factor stored in A (order n), FP64
  * arithmetic.  `b` is the factorisation's block size and only checked
- * (n % b == 0); the solve walks 256-column blocks: per block column the
- * next diagonal block is updated and solved while the rows below receive
- * L_ij x_j, one launch per block column.  Replaces trsvL_h
+ * (n % b == 0); the solve walks blocks of 256: each block row adds up
+ * L_ij x_j over the blocks before it and is then solved with its diagonal
+ * block (with the workspace, by the FP64 inverses of that block's 64 x 64
+ * diagonal sub-blocks).  Replaces trsvL_h
  * (panel_trsv.hpp:308-449: cast_copy_general + rocblas_dtrsv +
  * HPLMXP_gemv + daxpy) for one GPU, without the reference's per-block-column
  * swap of accumulation buffers. */

@@ -149,7 +149,8 @@ __global__ void k_zero(int64_t n, double *__restrict__ y) {
 }
 
 // ---------------------------------------------------------------------------
-// Triangular solves with the FP32 factors, FP64 vector and arithmetic.
+// Triangular solves with the FP32 factors, FP64 vector and arithmetic,
+// without a workspace (or too small, or unaligned): one launch per 256 columns.
 //
 // The matrix is walked in blocks of kTB = 256 rows/columns.  One launch per
 // block column J (solved values x_J final in x), workgroups of 1024
@@ -424,6 +425,348 @@ k_trsv_upper_step(int64_t n, int64_t j0, const float *__restrict__ A, int64_t ld
     if (tid < kTB && r0 + tid < d0) x[r0 + tid] -= t;
 }
 
+// ---------------------------------------------------------------------------
+// The same solves in one launch, with a workspace: rows in blocks of 256,
+// workgroup by workgroup (a ticket each, in solution order: a workgroup only
+// waits for blocks whose tickets were taken before its own, so whatever is
+// resident, the first unfinished block never waits).  For its block row I a
+// workgroup
+//   1. inverts the four 64 x 64 diagonal sub-blocks in FP64 (MFMA, below) and
+//      keeps the six sub-blocks between them in LDS: none of this needs x;
+//   2. adds up M(I, J) x_J in registers for J in solution order as the x_J
+//      appear; the next 256 x 256 tile of M is loaded while it waits;
+//   3. finishes x_I in four stages (a product with an inverse, then with the
+//      sub-blocks beyond it) and publishes it.
+// Published values are their own flags: xs starts as kUnset, a NaN that no
+// result is published as; readers poll it with device-scope loads.
+// The launch per 256 columns it replaces took 14 (lower) and 18 us (upper)
+// however few rows were left: launch, 256 KB through one CU, and 256
+// dependent steps.  A block now takes 4.5 us from x_J to x_I (hand-over
+// between XCDs 0.5, the last tile 0.5, sums 1.0, four stages 2.5), 5-7 while
+// hundreds of workgroups stream their tiles; where the matrix is large the
+// tiles' traffic bounds it (figures at trsv_launch).
+// ---------------------------------------------------------------------------
+constexpr uint64_t kUnset = 0x7FF4A5A5D00D5EEDull;  // a signalling NaN: arithmetic quiets it
+constexpr int kOffSub = kSB * kSB;                  // entries of a sub-block between the diagonal ones
+constexpr int kDiagLd = kSB + 4;                    // column stride of a staged diagonal sub-block
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+struct __align__(16) TrsvPrep {
+    float diag[4][kSB * kDiagLd];  // diag[k][c kDiagLd + r]: sub-block k, masked to its triangle
+    double inv[16][16][17];        // inverses of the 16 x 16 blocks on the diagonal: [block][row][column]
+};
+
+struct __align__(16) TrsvFused {
+    union {
+        TrsvPrep prep;
+        float off[6][kOffSub];     // sub-blocks (t, s) at slot off_slot: [c 64 + (r ^ 16 (c % 4))]
+    };
+    double part[kTW][kTB];         // per-wave sums of step 2
+    double xv[2][kTB];             // x_J, alternating
+    double rd[kTB];                // r_I less what is known
+    double xd[kTB];                // x_I
+    int ticket;
+};
+
+// slot of the sub-block in block row t, block column s (s < t lower, s > t upper)
+__device__ __forceinline__ int off_slot(int t, int s) {
+    const int hi = t > s ? t : s, lo = t > s ? s : t;
+    return hi * (hi - 1) / 2 + lo;
+}
+
+__global__ void __launch_bounds__(256) k_trsv_reset(int64_t n, uint64_t *__restrict__ xs, int *__restrict__ ticket) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) xs[i] = kUnset;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
+}
+
+// v summed over the lanes l, l ^ 16, l ^ 32, l ^ 48, in every one of them:
+// row (16 lanes) and half swaps in the VALU (a shuffle goes through LDS)
+__device__ __forceinline__ double sum_groups(double v) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    uint64_t u = __builtin_bit_cast(uint64_t, v);
+    u32x2 lo = __builtin_amdgcn_permlane16_swap((unsigned)u, (unsigned)u, false, false);
+    u32x2 hi = __builtin_amdgcn_permlane16_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    v = __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]) + __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+    u = __builtin_bit_cast(uint64_t, v);
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)u, (unsigned)u, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)(u >> 32), (unsigned)(u >> 32), false, false);
+    return __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]) +
+           __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+}
+
+// Rows [16 rb, 16 rb + 16) of the inverse of diagonal sub-block k, transposed,
+// as MFMA accumulators: z[b][i] in lane l is the entry (row 16 rb + l % 16,
+// column 16 b + 4 i + l / 16).  v_mfma_f64_16x16x4_f64 leaves row 4 i + l / 16
+// of its result in register i of lane l, which is the lane's share of the
+// second operand's k = 4 i + l / 16: each block of the solution feeds the
+// next products as it is.  Solves T^T Z = I(:, rb) block by block.
+template <bool kUpper>
+__device__ __forceinline__ void inverse_rows(const TrsvPrep &p, int k, int rb, int lane, f64x4 (&z)[4]) {
+    const int i16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[b][i] = (b == rb && 4 * i + g == i16) ? 1.0 : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int b = kUpper ? q : 3 - q;
+        if (kUpper ? b >= rb : b <= rb) {  // (zero elsewhere; rb is the wave's)
+            // z_b <- inv16(T_bb)^T z_b
+            f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p.inv[4 * k + b][4 * i + g][i16], z[b][i], acc, 0, 0, 0);
+            z[b] = acc;
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                if (kUpper ? m <= b : m >= b) continue;
+                // z_m -= T(b, m)^T z_b
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    z[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        -(double)p.diag[k][(16 * m + i16) * kDiagLd + 16 * b + 4 * i + g], z[b][i], z[m], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+}
+
+// Barrier that orders LDS accesses only: __syncthreads() would also wait for
+// the tile loads in flight and, after a publication, for its way to memory
+// (1.5 us a stage).
+__device__ __forceinline__ void lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <bool kUpper>
+__global__ void __launch_bounds__(kTT)
+k_trsv_fused(int64_t n, const float *__restrict__ A, int64_t lda, double *__restrict__ x, uint64_t *xs, int *ticket) {
+    __shared__ TrsvFused sh;
+    const int64_t nb = omx_cdiv(n, kTB);
+    for (;;) {
+        // (opaque: a hundred addresses derived from it, computed once before
+        // the loop, would live through it in scratch memory)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, i16 = lane & 15, g = lane >> 4;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        lds_sync();
+        if (tid == 0) sh.ticket = atomicAdd(ticket, 1);
+        lds_sync();
+        const int64_t t = sh.ticket;
+        if (t >= nb) return;
+        const int64_t I = kUpper ? nb - 1 - t : t;
+        const int64_t d0 = I * kTB;
+        const int dim = (int)min((int64_t)kTB, n - d0);
+        const float *D = A + d0 + d0 * lda;
+        // ---- 1. the diagonal block ----
+        {
+            float v[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int r = kSB * (q >> 2) + lane, c = kSB * (q >> 2) + wave + 16 * (q & 3);
+                v[q] = D[min(r, dim - 1) + (int64_t)min(c, dim - 1) * lda];
+            }
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                // rows and columns past the matrix: the identity
+                const int r = lane, c = wave + 16 * (q & 3), o = kSB * (q >> 2);
+                const bool in = o + r < dim && o + c < dim && (kUpper ? r <= c : r > c);
+                const bool one = r == c && (!kUpper || o + r >= dim);
+                sh.prep.diag[q >> 2][c * kDiagLd + r] = in ? v[q] : (one ? 1.0f : 0.0f);
+            }
+        }
+        lds_sync();
+        {
+            // wave w: 16 x 16 block w % 4 of sub-block w / 4, lane c its column c
+            const float *T = &sh.prep.diag[wave >> 2][(wave & 3) * 16 * (kDiagLd + 1)];
+            double y[16], rec = 1.0;
+            if (kUpper) rec = 1.0 / (double)T[i16 * kDiagLd + i16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int r = kUpper ? 15 - q : q;
+                double s = r == i16 ? 1.0 : 0.0;
+#pragma unroll
+                for (int u = 0; u < q; ++u) {
+                    const int c = kUpper ? 15 - u : u;
+                    s = __builtin_fma(-(double)T[c * kDiagLd + r], y[c], s);
+                }
+                y[r] = kUpper ? s * bcast_lane(rec, r) : s;
+                // (entry by entry: all of T's entries fetched ahead would spill)
+                asm volatile("" : "+v"(y[r]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (lane < 16) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sh.prep.inv[wave][r][lane] = y[r];
+            }
+        }
+        lds_sync();
+        const int k4 = wave >> 2, rb = wave & 3;  // this wave: rows [16 rb, 16 rb + 16) of sub-block k4
+        f64x4 z[4];
+        inverse_rows<kUpper>(sh.prep, k4, rb, lane, z);
+        lds_sync();
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            const int hi = q < 1 ? 1 : (q < 3 ? 2 : 3), lo = q - hi * (hi - 1) / 2;
+            const int rt = kSB * (kUpper ? lo : hi), ct = kSB * (kUpper ? hi : lo);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int c = wave + 16 * e;
+                const bool in = rt + lane < dim && ct + c < dim;
+                const float v = D[min(rt + lane, dim - 1) + (int64_t)min(ct + c, dim - 1) * lda];
+                sh.off[q][c * kSB + (lane ^ ((c & 3) << 4))] = in ? v : 0.0f;
+            }
+        }
+        const double r_in = tid < dim ? x[d0 + tid] : 0.0;
+        // ---- 2. the block row's products ----
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        // (rows past the matrix, in the lower solve's last block, read within
+        // the column's padding; their sums are not used)
+        const float *rows = A + min(d0 + 4 * lane, (n - 1) & ~(int64_t)3);
+        f32x4 v[kTC];
+        auto load_tile = [&](int64_t J) {
+            const int64_t c0 = J * kTB + kTC * wave;
+            const float *p = rows + min(c0, n - 1) * lda;
+            const int64_t cmax = n - 1 - c0;  // (columns past the matrix: the last one, times x = 0)
+            if (cmax >= kTC - 1) {
+#pragma unroll
+                for (int u = 0; u < kTC; ++u) v[u] = *reinterpret_cast<const f32x4 *>(p + u * lda);
+            } else {
+#pragma unroll
+                for (int u = 0; u < kTC; ++u)
+                    v[u] = *reinterpret_cast<const f32x4 *>(p + max(min((int64_t)u, cmax), (int64_t)0) * lda);
+            }
+        };
+        load_tile(kUpper ? nb - 1 : 0);  // (the first block has no use for it)
+        for (int64_t b = 0; b < t; ++b) {
+            const int64_t J = kUpper ? nb - 1 - b : b;
+            double *xv = sh.xv[b & 1];
+            if (tid < kTB) {
+                uint64_t w = 0;
+                if (J * kTB + tid < n) {
+                    const uint64_t *src = xs + J * kTB + tid;
+                    w = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    while (w == kUnset) {
+                        // the further off, the less often
+                        if (t - b > 2) __builtin_amdgcn_s_sleep(24);
+                        else if (t - b > 1) __builtin_amdgcn_s_sleep(6);
+                        w = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+                xv[tid] = __builtin_bit_cast(double, w);
+            }
+            lds_sync();
+            const int64_t Jn = kUpper ? J - 1 : J + 1;
+            const bool more = b + 1 < t;
+#pragma unroll
+            for (int u = 0; u < kTC; ++u) {
+                const double xc = xv[kTC * wave + u];
+                s0 = __builtin_fma((double)v[u].x, xc, s0);
+                s1 = __builtin_fma((double)v[u].y, xc, s1);
+                s2 = __builtin_fma((double)v[u].z, xc, s2);
+                s3 = __builtin_fma((double)v[u].w, xc, s3);
+                if ((u & 3) == 3) {
+                    // (four columns' factors at a time in registers)
+                    asm volatile("" : "+v"(s0), "+v"(s1), "+v"(s2), "+v"(s3)::"memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (more) load_tile(Jn);
+        }
+        sh.part[wave][4 * lane] = s0;
+        sh.part[wave][4 * lane + 1] = s1;
+        sh.part[wave][4 * lane + 2] = s2;
+        sh.part[wave][4 * lane + 3] = s3;
+        lds_sync();
+        if (tid < kTB) {
+            double q[kTW];
+#pragma unroll
+            for (int w = 0; w < kTW; ++w) q[w] = sh.part[w][tid];
+            __builtin_amdgcn_sched_barrier(0);  // (all reads in flight)
+#pragma unroll
+            for (int w = 1; w < kTW; ++w) q[0] += q[w];
+            sh.rd[tid] = tid < dim ? r_in - q[0] : 0.0;
+        }
+        lds_sync();
+        // ---- 3. x_I: stage st solves sub-block st with its inverse, then
+        // takes its products off the next one (the others' sums wait) ----
+        const double r_own = sh.rd[kSB * k4 + 16 * rb + i16];
+        double acc = 0.0;  // this lane's share of what its row loses to solved sub-blocks
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+            const int st = kUpper ? 3 - q : q;
+            const bool later = kUpper ? k4 < st : k4 > st;
+            // (opaque, as above: what is derived from them stays in the loop)
+            int own = 16 * rb + i16, gq = g;
+            asm volatile("" : "+v"(own), "+v"(gq));
+            if (k4 == st) {
+                const double *r = sh.rd + kSB * st + gq;
+                double rc[16], y = 0.0, y2 = 0.0;
+#pragma unroll
+                for (int b = 0; b < 16; ++b) rc[b] = r[4 * b];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < 16; b += 2) {
+                    y = __builtin_fma(z[b >> 2][b & 3], rc[b], y);
+                    y2 = __builtin_fma(z[(b + 1) >> 2][(b + 1) & 3], rc[b + 1], y2);
+                }
+                y = sum_groups(y + y2);
+                if (__builtin_expect(!__all(fabs(y) < __builtin_inf()), 0)) {
+                    // an infinity or NaN may have met the inverse's zeros:
+                    // once more with the row's own triangle only
+                    y = 0.0;
+#pragma unroll
+                    for (int b = 0; b < 16; ++b) {
+                        const int c = 4 * b + gq;
+                        y = __builtin_fma(z[b >> 2][b & 3], (kUpper ? c >= own : c <= own) ? rc[b] : 0.0, y);
+                    }
+                    y = sum_groups(y);
+                }
+                if (gq == 0) {
+                    const int row = kSB * st + own;
+                    sh.xd[row] = y;
+                    if (row < dim) {
+                        uint64_t w = __builtin_bit_cast(uint64_t, y);
+                        if (w == kUnset) w |= 1ull << 51;  // (quiet)
+                        __hip_atomic_store(xs + d0 + row, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        x[d0 + row] = y;
+                    }
+                }
+                lds_sync();
+            } else if (later) {
+                // (barriers in each branch: the waves' roles share no registers)
+                const float *src = sh.off[off_slot(k4, st)] + (own ^ (gq << 4)) + gq * kSB;
+                const double *xd = sh.xd + kSB * st + gq;
+                float o[16];
+                double xc[16], a2 = 0.0;
+#pragma unroll
+                for (int b = 0; b < 16; ++b) o[b] = src[4 * b * kSB];
+                lds_sync();
+#pragma unroll
+                for (int b = 0; b < 16; ++b) xc[b] = xd[4 * b];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int b = 0; b < 16; b += 2) {
+                    acc = __builtin_fma((double)o[b], xc[b], acc);
+                    a2 = __builtin_fma((double)o[b + 1], xc[b + 1], a2);
+                }
+                acc += a2;
+                if (kUpper ? k4 == st - 1 : k4 == st + 1) {
+                    const double d = sum_groups(acc);
+                    if (gq == 0) sh.rd[kSB * k4 + own] = r_own - d;
+                }
+            } else {
+                lds_sync();
+            }
+            lds_sync();
+        }
+    }
+}
+
 int grid_for(int64_t n, int threads) {
     int64_t g = omx_cdiv(n, threads);
     if (g > 65536) g = 65536;
@@ -535,8 +878,8 @@ int omx_axpy_f64(int64_t n, double alpha, const double *x, double *y, void *stre
 }
 
 size_t omx_trsv_workspace_bytes(int64_t n) {
-    (void)n;
-    return 0;
+    if (n <= 0) return 0;
+    return ((size_t)omx_cdiv(n, kTB) * kTB + 32) * sizeof(double);
 }
 
 static int trsv_args(int64_t n, int64_t b, const float *A, int64_t lda, double *x) {
@@ -548,13 +891,44 @@ static bool trsv_vec(const float *A, int64_t lda) {
     return (reinterpret_cast<uintptr_t>(A) & 15) == 0 && (lda & 3) == 0;
 }
 
+// The solve in one launch when the caller gives the workspace; OMX_OK and
+// *done = true if it was queued.  From three blocks on: with two the launch
+// and the inversion of the diagonal blocks cost what they save (n = 512:
+// lower 25 us against 19, upper 26 against 28; n = 768: 28 against 30 and 30
+// against 44).  us, one launch against one per block, lower / upper:
+//   n = 1024    33 /   41    35 /    59      n =  61440  1674 /  3640   1697 /  4821
+//   n = 10240  190 /  467   205 /   648      n = 122880  5664 /  8534   5668 / 10740
+//   n = 20480  453 / 1131   464 /  1526      n = 204800 14471 / 18635  14501 / 21080
+// (5.8 TB/s of factor entries at n = 204800: the tiles' traffic).
+static int trsv_launch(bool upper, int64_t n, const float *A, int64_t lda, double *x, void *work, size_t work_bytes,
+                       hipStream_t st, bool *done) {
+    *done = false;
+    const int64_t nb = omx_cdiv(n, kTB);
+    if (nb < 3 || !trsv_vec(A, lda) || !work || work_bytes < omx_trsv_workspace_bytes(n) ||
+        (reinterpret_cast<uintptr_t>(work) & 7))
+        return OMX_OK;
+    uint64_t *xs = static_cast<uint64_t *>(work);
+    int *ticket = reinterpret_cast<int *>(xs + nb * kTB);
+    hipLaunchKernelGGL(k_trsv_reset, dim3(grid_for(nb * kTB, 256)), dim3(256), 0, st, nb * kTB, xs, ticket);
+    OMX_LAUNCH_CHECK();
+    const dim3 grid((unsigned)(nb < 256 ? nb : 256));  // one workgroup per CU
+    if (upper)
+        hipLaunchKernelGGL(k_trsv_fused<true>, grid, dim3(kTT), 0, st, n, A, lda, x, xs, ticket);
+    else
+        hipLaunchKernelGGL(k_trsv_fused<false>, grid, dim3(kTT), 0, st, n, A, lda, x, xs, ticket);
+    OMX_LAUNCH_CHECK();
+    *done = true;
+    return OMX_OK;
+}
+
 int omx_trsv_lower_unit_f32f64(int64_t n, int64_t b, const float *A, int64_t lda, double *x,
                                void *work, size_t work_bytes, void *stream) {
-    (void)work;
-    (void)work_bytes;
     int rc = trsv_args(n, b, A, lda, x);
     if (rc) return rc;
     hipStream_t st = omx_stream(stream);
+    bool done;
+    rc = trsv_launch(false, n, A, lda, x, work, work_bytes, st, &done);
+    if (rc || done) return rc;
     const bool vec = trsv_vec(A, lda);
     for (int64_t j0 = -kTB; j0 + kTB < n; j0 += kTB) {
         const int64_t d0 = j0 + kTB;
@@ -571,11 +945,12 @@ int omx_trsv_lower_unit_f32f64(int64_t n, int64_t b, const float *A, int64_t lda
 
 int omx_trsv_upper_f32f64(int64_t n, int64_t b, const float *A, int64_t lda, double *x,
                           void *work, size_t work_bytes, void *stream) {
-    (void)work;
-    (void)work_bytes;
     int rc = trsv_args(n, b, A, lda, x);
     if (rc) return rc;
     hipStream_t st = omx_stream(stream);
+    bool done;
+    rc = trsv_launch(true, n, A, lda, x, work, work_bytes, st, &done);
+    if (rc || done) return rc;
     const bool vec = trsv_vec(A, lda);
     const int64_t last0 = ((n - 1) / kTB) * kTB;
     // j0 = n: the last block alone; then J = each block from the last down

@@ -131,3 +131,45 @@ def test_triangular_inverses(n, pad):
         # products of at most n terms at every one of log2(n / 64) + 1 levels
         tol = 2 * n * 2.0 ** -24 * (np.log2(n / 64) + 1)
         assert np.all(np.abs(got - want) <= tol * (np.abs(want) @ np.abs(T) @ np.abs(want)))
+
+
+# with the workspace (one launch): one block and a bit, exact blocks, ragged
+# last blocks, more blocks than workgroups (n > 65536 is left to the solver's
+# tests), against LAPACK; x and the workspace are not written beyond n
+@pytest.mark.parametrize("n,lda", [(257, 260), (300, 300), (512, 512), (575, 576), (777, 780), (1024, 1028),
+                                   (2303, 2304), (4096, 4096)])
+def test_trsv_with_workspace(n, lda):
+    import scipy.linalg as sla
+    torch = torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    F = (np.tril(rng.uniform(-1, 1, (n, n)) / n, -1) + np.triu(rng.uniform(-1, 1, (n, n)) / n, 1)
+         + np.diag(rng.uniform(1, 2, n))).astype(np.float32)
+    store = np.full((n, lda), np.nan, np.float32)
+    store[:, :n] = F.T
+    Ad = dev(store)
+    r = rng.uniform(-1, 1, n)
+    wb = L.omx_trsv_workspace_bytes(n)
+    W = empty(wb + 64, torch.uint8).fill_(255)
+    xd = dev(np.concatenate([r, np.full(8, 3.0)]))
+    F64 = F.astype(np.float64)
+    y = sla.solve_triangular(np.tril(F64, -1) + np.eye(n), r, lower=True, unit_diagonal=True)
+    z = sla.solve_triangular(np.triu(F64), y, lower=False)
+    for rep in range(3):  # the workspace as the last call left it
+        xd[:n] = dev(r)
+        assert L.omx_trsv_lower_unit_f32f64(n, n, ptr(Ad), lda, ptr(xd), ptr(W), wb, None) == 0
+        yg = host(xd)
+        assert np.max(np.abs(yg[:n] - y)) <= 1e-13 * np.max(np.abs(y)) and np.all(yg[n:] == 3.0)
+        assert L.omx_trsv_upper_f32f64(n, n, ptr(Ad), lda, ptr(xd), ptr(W), wb, None) == 0
+        zg = host(xd)
+        assert np.max(np.abs(zg[:n] - z)) <= 1e-13 * np.max(np.abs(z)) and np.all(zg[n:] == 3.0)
+    assert bool((W[wb:] == 255).all())
+    # a NaN spreads as in a substitution: to every later entry, to none before
+    k = 300 % n
+    r[k] = np.nan
+    for solve, before, after in ((L.omx_trsv_lower_unit_f32f64, slice(0, k), slice(k, n)),
+                                 (L.omx_trsv_upper_f32f64, slice(k + 1, n), slice(0, k + 1))):
+        xd[:n] = dev(r)
+        assert solve(n, n, ptr(Ad), lda, ptr(xd), ptr(W), wb, None) == 0
+        g = host(xd)[:n]
+        assert np.all(np.isfinite(g[before])) and np.all(np.isnan(g[after]))
