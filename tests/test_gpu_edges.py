@@ -175,3 +175,24 @@ def test_trsv_with_workspace(n, lda):
         assert solve(n, n, ptr(Ad), lda, ptr(xd), ptr(W), wb, None) == 0
         g = host(xd)[:n]
         assert np.all(np.isfinite(g[before])) and np.all(np.isnan(g[after]))
+
+
+# one workgroup's rows, one more, ragged ends; the largest entries at either
+# end of the sums
+@pytest.mark.parametrize("n", [2, 63, 64, 1023, 1024, 1025, 2048, 5000])
+def test_higham_gemv_running_sums(n):
+    torch = torch_cuda()
+    rng = np.random.default_rng(n)
+    a, b = -0.5 / n, 1.0 / n
+    i = np.arange(n, dtype=np.float64)
+    A = np.where(i[:, None] < i[None, :], -b + a * b * i[:, None], -a + a * b * i[None, :])
+    A[np.arange(n), np.arange(n)] = 1.0 + a * b * i
+    for x in (rng.uniform(-1, 1, n), np.exp(-20 * i / n), np.exp(20 * (i / n - 1))):
+        y0 = rng.uniform(-1, 1, n)
+        xd, yd = dev(x), dev(np.concatenate([y0, [5.0]]))
+        assert _L().omx_higham_gemv_f64(n, a, b, 1.5, ptr(xd), ptr(yd), None) == 0
+        got = host(yd)
+        assert got[n] == 5.0
+        want = y0 + 1.5 * (A @ x)
+        # |u_i| sum_{j>i} |x_j| and the like: n terms, each rounded a few times
+        assert np.all(np.abs(got[:n] - want) <= 4 * n * 2.0 ** -53 * (np.abs(A) @ np.abs(x) * 1.5 + np.abs(y0)))
