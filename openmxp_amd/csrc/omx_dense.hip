@@ -24,10 +24,10 @@ constexpr int kNB = 64;
         if (rc_) return rc_;   \
     } while (0)
 
-// The triangular solves (omx_trsm_f32) go 64 columns at a time inside
-// blocks of kOB: the 64-wide steps update only the rest of their block, and
-// each block updates everything beyond it in one product of depth kOB, so
-// the large products read and write their C a quarter as often.
+// The triangular solves (omx_trsm_f32) go in blocks of kOB: a block is solved
+// in one launch (RLNU: 64 columns at a time) and updates everything beyond it
+// in one product of depth kOB, so the large products read and write their C a
+// quarter as often as with 64.
 constexpr int64_t kOB = 256;
 
 // ---------------------------------------------------------------------------
@@ -365,8 +365,8 @@ __device__ __forceinline__ void tri16_steps(float (&x)[4], int q, const float (&
     (tri16_step<J, kUp>(x, q, e, r), ...);
 }
 
-template <bool kUp>
-__device__ __forceinline__ void tri_solve64(float (*xs)[kXS], const float (*t)[kNB + 1], const float *rd) {
+template <bool kUp, int kLd>
+__device__ __forceinline__ void tri_solve64(float (*xs)[kLd], const float (*t)[kNB + 1], const float *rd) {
     const int lane = threadIdx.x & 63, q = lane & 3;
     const int i16 = lane & 15, g = lane >> 4;
 #pragma unroll 1
@@ -440,35 +440,12 @@ k_trsm_rows_runn64(int64_t m, const float *__restrict__ U, int64_t ldu, float *_
 #pragma unroll
     for (int c = 0; c < 16; ++c) xs[r][c0 + c] = v[c];
     diag_recip64(u, rd);
-    tri_solve64<true>(xs + c0, u, rd);
+    tri_solve64<true, kXS>(xs + c0, u, rd);
     __syncthreads();
     if (i < m) {
 #pragma unroll
         for (int c = 0; c < 16; ++c) row[c * ldx] = xs[r][c0 + c];
     }
-}
-
-// 64 columns per workgroup, 16 per wave: Y(:, j) <- L^-1 Y(:, j).  Columns
-// past n are read as column n - 1 and not stored.
-__global__ void __launch_bounds__(256)
-k_trsm_cols_llnu64(int64_t n, const float *__restrict__ L, int64_t ldl, float *__restrict__ Y,
-                   int64_t ldy) {
-    __shared__ float l[kNB][kNB + 1];
-    __shared__ __align__(16) float ys[kNB][kXS];
-    const int r = threadIdx.x & 63, c0 = 16 * (threadIdx.x >> 6);
-    const int64_t j = (int64_t)blockIdx.x * 64 + c0;
-    float v[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) v[c] = Y[r + min(j + c, n - 1) * ldy];
-    load_tri64(L, ldl, l);
-    // (the wave's own columns: no barrier before it solves them)
-#pragma unroll
-    for (int c = 0; c < 16; ++c) ys[c0 + c][r] = v[c];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    tri_solve64<false>(ys + c0, l, nullptr);
-#pragma unroll
-    for (int c = 0; c < 16; ++c)
-        if (j + c < n) Y[r + (j + c) * ldy] = ys[c0 + c][r];
 }
 
 // ---------------------------------------------------------------------------
@@ -809,9 +786,9 @@ k_getrf_step64(int64_t n, int64_t j, int np, float *__restrict__ A, int64_t lda,
     }
     lds_barrier();
     if (cols)
-        tri_solve64<false>(sh.sx + 16 * wave, sh.d, nullptr);
+        tri_solve64<false, kXS>(sh.sx + 16 * wave, sh.d, nullptr);
     else
-        tri_solve64<true>(sh.sx + 16 * wave, sh.d, sh.rd);
+        tri_solve64<true, kXS>(sh.sx + 16 * wave, sh.d, sh.rd);
     lds_barrier();
     // lanes along the matrix rows (of a row-block tile: the wave's own lines)
     if (cols) {
@@ -852,6 +829,143 @@ k_trsm_rows_rlnu64(int64_t m, const float *__restrict__ L, int64_t ldl, float *_
     for (int j = 0; j < kNB; ++j) X[i + j * ldx] = x[j];
 }
 
+// One block of kOB columns (RUNN, kUp) or rows (LLNU) of the triangular solves
+// in one launch: a workgroup of 256 threads takes 64 lines (rows of X, columns
+// of Y) of w = 64, 128, 192 or 256 entries.  64 entries at a time are read,
+// lose their products with the lines' solved entries (each block of 64 summed
+// by itself and subtracted, in the order of the product that a launch of its
+// own would run: put_u), are solved (tri_solve64) and written; the solved
+// entries stay in LDS.  As launches of 64 entries each (solve, then a depth-64
+// product over the rest of the block) the lines went to memory and back four
+// times: 110 us a block for 30000 lines of 256, now 46; bound by the chain of
+// four solves and their operands' latency.
+struct __align__(16) TrsmShared {
+    float xs[kNB][kOB + 4];    // the lines: xs[line][entry]
+    float t[kNB][kNB + 1];     // the 64 x 64 triangle
+    float su[kNB][kUS];        // a block between: su[c][k] for entry c, solved entry k
+    float rd[kNB];
+};
+
+// the block for solved entries [64 i, +64) and entries [64 j, +64): element
+// (c, k) is U(64 i + k, 64 j + c) (kUp) or L(64 j + c, 64 i + k)
+template <bool kUp, bool kVec>
+__device__ __forceinline__ void trsm_block_get(const float *__restrict__ T, int64_t ldt, int i, int j, f32x4 (&v)[4]) {
+    // four consecutive k (kUp) or c of a column: 16 threads a column
+    const float *g = T + (kUp ? i : j) * kNB + 4 * (threadIdx.x & 15) +
+                     (int64_t)((kUp ? j : i) * kNB + (threadIdx.x >> 4)) * ldt;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float *p = g + (int64_t)(16 * q) * ldt;
+        v[q] = kVec ? *reinterpret_cast<const f32x4 *>(p) : f32x4{p[0], p[1], p[2], p[3]};
+    }
+}
+
+template <bool kUp>
+__device__ __forceinline__ void trsm_block_put(const f32x4 (&v)[4], float (*su)[kUS], bool seq) {
+    const int a = 4 * (threadIdx.x & 15);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int b = (threadIdx.x >> 4) + 16 * q;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int c = kUp ? b : a + e, k = kUp ? a + e : b;
+            su[c][seq ? (k & 1) * 32 + (k >> 1) : k] = v[q][e];
+        }
+    }
+}
+
+template <bool kUp, bool kVec>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_trsm_block(int64_t lines, int w, const float *__restrict__ T, int64_t ldt, float *__restrict__ X, int64_t ldx) {
+    __shared__ TrsmShared sh;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t e0 = (int64_t)blockIdx.x * kNB;
+    const int nb = w / kNB;
+    // a thread's 16 values of a 64 x 64 piece: memory rows along the lanes;
+    // lines past the end are read as the last one and not stored
+    const int64_t le = min(e0 + lane, lines - 1) - e0;
+    auto addr = [&](int j, int q) -> float * {
+        return kUp ? X + e0 + le + (int64_t)(kNB * j + 16 * wave + q) * ldx
+                   : X + kNB * j + lane + min(e0 + 16 * wave + q, lines - 1) * ldx;
+    };
+    float v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = *addr(0, q);
+#pragma unroll 1
+    for (int j = 0; j < nb; ++j) {
+        // the update's order of sums: the product over the rest of the block
+        // that followed solved block i
+        f32x4 u[4];
+        if (j > 0) trsm_block_get<kUp, kVec>(T, ldt, 0, j, u);
+        lds_barrier();  // (the last piece's triangle and lines are read)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int line = kUp ? lane : 16 * wave + q, c = kUp ? 16 * wave + q : lane;
+            sh.xs[line][kNB * j + c] = v[q];
+        }
+        {
+            const float *tj = T + (kNB * j + lane) + (int64_t)(kNB * j + 16 * wave) * ldt;
+            float d[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) d[q] = tj[(int64_t)q * ldt];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) sh.t[lane][16 * wave + q] = d[q];
+        }
+        if (j + 1 < nb) {  // the next piece, in flight during this one
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = *addr(j + 1, q);
+        }
+        // 32 lines x 32 entries a wave
+        const int wl = 32 * (wave & 1), wc = 32 * (wave >> 1);
+#pragma unroll 1
+        for (int i = 0; i < j; ++i) {
+            const int64_t inner = w - kNB * (i + 1);
+            const bool seq = !kVec || !mfma_size(kUp ? lines : inner, kUp ? inner : lines, 1);
+            trsm_block_put<kUp>(u, sh.su, seq);
+            lds_barrier();
+            if (i + 1 < j) trsm_block_get<kUp, kVec>(T, ldt, i + 1, j, u);
+            const float *x = &sh.xs[wl + l32][kNB * i + (seq ? h : 32 * h)];
+            f32x16 acc;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+            for (int g = 0; g < 8; ++g) {
+                const f32x4 y = *reinterpret_cast<const f32x4 *>(&sh.su[wc + l32][32 * h + 4 * g]);
+                f32x4 xv;
+                if (seq)
+                    xv = f32x4{x[8 * g], x[8 * g + 2], x[8 * g + 4], x[8 * g + 6]};
+                else
+                    xv = *reinterpret_cast<const f32x4 *>(x + 4 * g);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[s], xv[s], acc, 0, 0, 0);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                f32x4 *d = reinterpret_cast<f32x4 *>(&sh.xs[wl + l32][kNB * j + wc + 8 * r + 4 * h]);
+                f32x4 o = *d;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) o[s] -= acc[4 * r + s];
+                *d = o;
+            }
+            lds_barrier();
+        }
+        lds_barrier();
+        if (kUp) {
+            if (tid < kNB) sh.rd[tid] = 1.0f / sh.t[tid][tid];
+            lds_barrier();
+        }
+        float (*lines16)[kOB + 4] = reinterpret_cast<float (*)[kOB + 4]>(&sh.xs[16 * wave][kNB * j]);
+        tri_solve64<kUp, kOB + 4>(lines16, sh.t, sh.rd);
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int line = kUp ? lane : 16 * wave + q, c = kUp ? 16 * wave + q : lane;
+            if (e0 + line < lines) *addr(j, q) = sh.xs[line][kNB * j + c];
+        }
+    }
+}
+
 // Inverses of the 64 x 64 diagonal blocks of the factored block D (L unit
 // lower, U upper in one array): workgroup w < nblk writes U_ww^-1 into Xu
 // (row r of it = e_r U_ww^-1, a row solve of the identity), workgroup nblk + w
@@ -883,12 +997,12 @@ k_tri_inv64(int nblk, const float *__restrict__ D, int64_t ldd, float *__restric
     load_tri64(D + o + o * ldd, ldd, t);
     if (up) {
         diag_recip64(t, rd);
-        tri_solve64<true>(xs + w0, t, rd);
+        tri_solve64<true, kXS>(xs + w0, t, rd);
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < 16; ++c) Xu[o + lane + (o + w0 + c) * ldx] = xs[lane][w0 + c];
     } else {
-        tri_solve64<false>(xs + w0, t, nullptr);
+        tri_solve64<false, kXS>(xs + w0, t, nullptr);
 #pragma unroll
         for (int c = 0; c < 16; ++c) Xl[o + lane + (o + w0 + c) * ldx] = xs[w0 + c][lane];
     }
@@ -1071,6 +1185,22 @@ int sgemm_twin(const SgemmTwin &g0, const SgemmTwin &g1, float alpha, int64_t ba
     return OMX_OK;
 }
 
+// one block of the triangular solves (k_trsm_block); the order of its sums
+// goes by the operands' alignment as in the products it replaces
+template <bool kUp>
+int trsm_block(int64_t lines, int64_t w, const float *T, int64_t ldt, float *X, int64_t ldx, hipStream_t st) {
+    const bool vec = ((reinterpret_cast<uintptr_t>(T) | reinterpret_cast<uintptr_t>(X)) & 15) == 0 && (ldt & 3) == 0 &&
+                     (ldx & 3) == 0;
+    const dim3 grid((unsigned)omx_cdiv(lines, kNB));
+    if (omx_cdiv(lines, kNB) >= ((int64_t)1 << 31)) return OMX_ERR_ARG;
+    if (vec)
+        hipLaunchKernelGGL((k_trsm_block<kUp, true>), grid, dim3(256), 0, st, lines, (int)w, T, ldt, X, ldx);
+    else
+        hipLaunchKernelGGL((k_trsm_block<kUp, false>), grid, dim3(256), 0, st, lines, (int)w, T, ldt, X, ldx);
+    OMX_LAUNCH_CHECK();
+    return OMX_OK;
+}
+
 // sgemm with n split into chunks of at most 65535*64 columns
 int sgemm_big(int64_t m, int64_t n, int64_t k, float alpha, const float *A, int64_t lda, const float *B,
               int64_t ldb, float beta, float *C, int64_t ldc, hipStream_t st, int64_t msel = -1) {
@@ -1128,17 +1258,9 @@ int omx_trsm_f32(int variant, int64_t m, int64_t n, const float *T, int64_t ldt,
         if (n % kNB || ldt < n) return OMX_ERR_ARG;
         const unsigned g = (unsigned)omx_cdiv(m, 256);
         if (variant == OMX_TRSM_RUNN) {
-            const unsigned g4 = (unsigned)omx_cdiv(m, 64);  // a lane quad per row
             for (int64_t J0 = 0; J0 < n; J0 += kOB) {
                 const int64_t w = std::min(kOB, n - J0);
-                for (int64_t j = J0; j < J0 + w; j += kNB) {
-                    hipLaunchKernelGGL(k_trsm_rows_runn64, dim3(g4), dim3(256), 0, st, m, T + j + j * ldt, ldt,
-                                       B + j * ldb, ldb);
-                    OMX_LAUNCH_CHECK();
-                    const int64_t inner = J0 + w - j - kNB;
-                    if (inner > 0) RC(sgemm_big(m, inner, kNB, -1.0f, B + j * ldb, ldb, T + j + (j + kNB) * ldt, ldt, 1.0f,
-                                                B + (j + kNB) * ldb, ldb, st));
-                }
+                RC(trsm_block<true>(m, w, T + J0 + J0 * ldt, ldt, B + J0 * ldb, ldb, st));
                 const int64_t rest = n - J0 - w;
                 if (rest > 0) RC(sgemm_big(m, rest, w, -1.0f, B + J0 * ldb, ldb, T + J0 + (J0 + w) * ldt, ldt, 1.0f,
                                            B + (J0 + w) * ldb, ldb, st));
@@ -1161,20 +1283,9 @@ int omx_trsm_f32(int variant, int64_t m, int64_t n, const float *T, int64_t ldt,
     if (variant == OMX_TRSM_LLNU) {
         // inverse of an m x m unit lower triangle times B (m x n), m % 64 == 0
         if (m % kNB || ldt < m) return OMX_ERR_ARG;
-        const int64_t nmax = (int64_t)65535 * 64;  // a lane quad per column
         for (int64_t I0 = 0; I0 < m; I0 += kOB) {
             const int64_t w = std::min(kOB, m - I0);
-            for (int64_t i = I0; i < I0 + w; i += kNB) {
-                for (int64_t c = 0; c < n; c += nmax) {
-                    const int64_t nn = (n - c < nmax) ? n - c : nmax;
-                    hipLaunchKernelGGL(k_trsm_cols_llnu64, dim3((unsigned)omx_cdiv(nn, 64)), dim3(256), 0, st, nn,
-                                       T + i + i * ldt, ldt, B + i + c * ldb, ldb);
-                    OMX_LAUNCH_CHECK();
-                }
-                const int64_t inner = I0 + w - i - kNB;
-                if (inner > 0) RC(sgemm_big(inner, n, kNB, -1.0f, T + (i + kNB) + i * ldt, ldt, B + i, ldb, 1.0f,
-                                            B + i + kNB, ldb, st));
-            }
+            RC(trsm_block<false>(n, w, T + I0 + I0 * ldt, ldt, B + I0, ldb, st));
             const int64_t rest = m - I0 - w;
             if (rest > 0) RC(sgemm_big(rest, n, w, -1.0f, T + (I0 + w) + I0 * ldt, ldt, B + I0, ldb, 1.0f,
                                        B + I0 + w, ldb, st));

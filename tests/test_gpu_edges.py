@@ -196,3 +196,35 @@ def test_higham_gemv_running_sums(n):
         want = y0 + 1.5 * (A @ x)
         # |u_i| sum_{j>i} |x_j| and the like: n terms, each rounded a few times
         assert np.all(np.abs(got[:n] - want) <= 4 * n * 2.0 ** -53 * (np.abs(A) @ np.abs(x) * 1.5 + np.abs(y0)))
+
+
+# blocks of one to four pieces and a ragged last one, one line, full and
+# ragged workgroups, both orders of sums (2^18 entries), unaligned operands
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("w,lines", [(64, 1), (128, 63), (192, 64), (256, 65), (320, 200), (448, 1500), (576, 4097)])
+@pytest.mark.parametrize("variant", [0, 1])
+def test_trsm_blocks(variant, w, lines, pad):
+    import scipy.linalg as sla
+    torch = torch_cuda()
+    rng = np.random.default_rng(w + lines)
+    T = np.triu(rng.uniform(-0.5, 0.5, (w, w)), 1) + np.tril(rng.uniform(-0.5, 0.5, (w, w)) * 4 / w, -1) \
+        + np.diag(w / 4 * (1 + 0.1 * rng.uniform(size=w)))
+    T = T.astype(np.float32)
+    m, n = (lines, w) if variant == 0 else (w, lines)
+    B = rng.uniform(-0.5, 0.5, (m, n)).astype(np.float32)
+    ldt, ldb = w + pad, (m + 3) // 4 * 4 + pad
+    tb, bb = np.zeros((w, ldt), np.float32), np.full((n, ldb), 7.0, np.float32)
+    tb[:, :w], bb[:, :m] = T.T, B.T
+    Td, Bd = dev(tb), dev(bb)
+    assert _L().omx_trsm_f32(variant, m, n, ptr(Td), ldt, ptr(Bd), ldb, None) == 0
+    out = host(Bd)
+    assert np.all(out[:, m:] == 7.0)
+    X = out[:, :m].T.astype(np.float64)
+    T64 = T.astype(np.float64)
+    # residual of substitution: w products a entry, rounded one by one
+    if variant == 0:
+        U = np.triu(T64)
+        assert np.all(np.abs(X @ U - B) <= (w + 4) * 2.0 ** -24 * (np.abs(X) @ np.abs(U) + np.abs(B)))
+    else:
+        L = np.tril(T64, -1) + np.eye(w)
+        assert np.all(np.abs(L @ X - B) <= (w + 4) * 2.0 ** -24 * (np.abs(L) @ np.abs(X) + np.abs(B)))
