@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "omx_common.hpp"
+#include "omx_internal.hpp"
 #include "omx_layout.hpp"
 
 #ifndef OMX_GEMM_NBUF
@@ -309,6 +310,21 @@ __device__ __forceinline__ void epilogue_lds(floatx16 (&acc)[4][4], float alpha,
     }
 }
 
+// Two products of one kind in one launch (kPair: a step's column and row
+// panel): workgroups below split take the kernel's own arguments, the others
+// j1.  Where a product has few tiles its
+// launch lasts as long as one tile, so two of them wait for each other:
+// 10 + 10 us as two -alt panel products at b = 256 and 10000 rows, 12 as one.
+struct GemmJob {
+    int64_t M, N, K;
+    const char *X, *Y;
+    const int32_t *xexp, *yexp;  // FP8
+    float *C;
+    int64_t ldc, xstrip, ystrip, xet, yet;
+    int tiles_m, tiles_n, ktri, tmax_tr;
+    float *tmax;
+};
+
 // ---------------------------------------------------------------------------
 // FP16: LDS stages of 32 columns (16 KB per operand), kNbuf of them in a
 // ring, kNbuf-1 in flight.  Stage s of a 256-row strip is half (s & 1) of
@@ -319,18 +335,38 @@ __device__ __forceinline__ void epilogue_lds(floatx16 (&acc)[4][4], float alpha,
 // previous stage and reads the next stage's first fragments, which then
 // arrive while the second 16 MFMAs run.
 // ---------------------------------------------------------------------------
-template <bool kBetaZero, int kNbuf, bool kTmax = false>
+template <bool kBetaZero, int kNbuf, bool kTmax = false, bool kPair = false>
 __global__ void __launch_bounds__(kThreads, 1)
 k_gemm_f16(int64_t M, int64_t N, int64_t K, float alpha, float beta, const char *__restrict__ X,
            const char *__restrict__ Y, float *__restrict__ C, int64_t ldc, int tiles_m, int tiles_n,
            const int32_t *__restrict__ xsexp, const int32_t *__restrict__ ysexp, int64_t xstrip,
-           int64_t ystrip, int ktri, float *__restrict__ tmax, int tmax_tr) {
+           int64_t ystrip, int ktri, float *__restrict__ tmax, int tmax_tr, GemmJob j1, int split) {
+    int bid = blockIdx.x;
+    if constexpr (kPair) {
+        if (bid >= split) {
+            bid -= split;
+            M = j1.M;
+            N = j1.N;
+            K = j1.K;
+            X = j1.X;
+            Y = j1.Y;
+            C = j1.C;
+            ldc = j1.ldc;
+            tiles_m = j1.tiles_m;
+            tiles_n = j1.tiles_n;
+            xstrip = j1.xstrip;
+            ystrip = j1.ystrip;
+            ktri = j1.ktri;
+            tmax = j1.tmax;
+            tmax_tr = j1.tmax_tr;
+        }
+    }
     __shared__ __attribute__((aligned(1024))) char smem[kNbuf][2][16384];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar tile offsets
     const int wm = wave & 1, wn = wave >> 1;
     int tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_of(bid, tiles_m, tiles_n, tm, tn);
     int nks = (int)(K / 32);
     // a triangular factor (ktri 1: Y(j, l) = 0 for l > j; 2: X(i, l) = 0
     // for l > i): the tile's products past its diagonal 256-column k tile
@@ -492,18 +528,39 @@ k_gemm_f16(int64_t M, int64_t N, int64_t K, float alpha, float beta, const char 
 // blocks rr*2 + (s&1) (2 KB each, two 1 KB halves) of packed chunk s/2.  One
 // k-step of 16 scaled MFMAs per stage, split 8 + 8 around the barrier.
 // ---------------------------------------------------------------------------
-template <bool kBetaZero, int kNbuf>
+template <bool kBetaZero, int kNbuf, bool kPair = false>
 __global__ void __launch_bounds__(kThreads, 1)
 k_gemm_f8(int64_t M, int64_t N, int64_t K, float alpha, float beta, const char *__restrict__ X,
           const int32_t *__restrict__ xexp, const char *__restrict__ Y, const int32_t *__restrict__ yexp,
           float *__restrict__ C, int64_t ldc, int tiles_m, int tiles_n, int64_t xstrip, int64_t ystrip,
-          int64_t xet, int64_t yet) {
+          int64_t xet, int64_t yet, GemmJob j1, int split) {
+    int bid = blockIdx.x;
+    if constexpr (kPair) {
+        if (bid >= split) {
+            bid -= split;
+            M = j1.M;
+            N = j1.N;
+            K = j1.K;
+            X = j1.X;
+            xexp = j1.xexp;
+            Y = j1.Y;
+            yexp = j1.yexp;
+            C = j1.C;
+            ldc = j1.ldc;
+            tiles_m = j1.tiles_m;
+            tiles_n = j1.tiles_n;
+            xstrip = j1.xstrip;
+            ystrip = j1.ystrip;
+            xet = j1.xet;
+            yet = j1.yet;
+        }
+    }
     __shared__ __attribute__((aligned(1024))) char smem[kNbuf][2][16384];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: scalar tile offsets
     const int wm = wave & 1, wn = wave >> 1;
     int tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    tile_of(bid, tiles_m, tiles_n, tm, tn);
     const int nks = (int)(K / 64);
     // strips xstrip / ystrip bytes apart; xet / yet exponents per strip
     const char *xs = X + (int64_t)tm * xstrip;
@@ -1050,13 +1107,13 @@ int gemm_f16_launch(int64_t m, int64_t n, int64_t k, float alpha, const uint16_t
     if (beta == 0.0f && tile_max)
         hipLaunchKernelGGL((k_gemm_f16<true, kNbuf, true>), grid, dim3(kThreads), 0, omx_stream(stream), m, n, k,
                            alpha, beta, xp, yp, C, ldc, tiles_m, tiles_n, xe, ye, xstrip, ystrip, tri, tile_max,
-                           tri == 2 ? 1 : 0);
+                           tri == 2 ? 1 : 0, GemmJob{}, 0);
     else if (beta == 0.0f)
         hipLaunchKernelGGL((k_gemm_f16<true, kNbuf>), grid, dim3(kThreads), 0, omx_stream(stream), m, n, k, alpha,
-                           beta, xp, yp, C, ldc, tiles_m, tiles_n, xe, ye, xstrip, ystrip, tri, nullptr, 0);
+                           beta, xp, yp, C, ldc, tiles_m, tiles_n, xe, ye, xstrip, ystrip, tri, nullptr, 0, GemmJob{}, 0);
     else
         hipLaunchKernelGGL((k_gemm_f16<false, kNbuf>), grid, dim3(kThreads), 0, omx_stream(stream), m, n, k, alpha,
-                           beta, xp, yp, C, ldc, tiles_m, tiles_n, xe, ye, xstrip, ystrip, tri, nullptr, 0);
+                           beta, xp, yp, C, ldc, tiles_m, tiles_n, xe, ye, xstrip, ystrip, tri, nullptr, 0, GemmJob{}, 0);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
@@ -1126,10 +1183,10 @@ int omx_gemm_f8_packed_window(int64_t m, int64_t n, int64_t k, float alpha, cons
     dim3 grid((unsigned)(tiles_m * tiles_n));
     if (beta == 0.0f)
         hipLaunchKernelGGL((k_gemm_f8<true, kNbuf>), grid, dim3(kThreads), 0, omx_stream(stream), m, n, k, alpha,
-                           beta, xp, xe, yp, ye, C, ldc, tiles_m, tiles_n, xstrip, ystrip, xet, yet);
+                           beta, xp, xe, yp, ye, C, ldc, tiles_m, tiles_n, xstrip, ystrip, xet, yet, GemmJob{}, 0);
     else
         hipLaunchKernelGGL((k_gemm_f8<false, kNbuf>), grid, dim3(kThreads), 0, omx_stream(stream), m, n, k, alpha,
-                           beta, xp, xe, yp, ye, C, ldc, tiles_m, tiles_n, xstrip, ystrip, xet, yet);
+                           beta, xp, xe, yp, ye, C, ldc, tiles_m, tiles_n, xstrip, ystrip, xet, yet, GemmJob{}, 0);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
@@ -1142,3 +1199,100 @@ int omx_gemm_f8_packed(int64_t m, int64_t n, int64_t k, float alpha, const uint8
 }
 
 }  // extern "C"
+
+namespace {
+
+// j with its operands' addresses resolved (es: columns per 32 KB chunk)
+int resolve_job(const omx_gemm_job &q, int64_t es, bool fp8, GemmJob &j) {
+    const int64_t align = fp8 ? OMX_SCALE_TILE : OMX_KSTAGE16;
+    const int rc = gemm_args(q.m, q.n, q.k, align, q.X, q.x_row0, q.Y, q.y_row0, q.C, q.ldc);
+    if (rc) return rc;
+    if (!window_ok(q.k, q.x_ldk, q.x_k0, align) || !window_ok(q.k, q.y_ldk, q.y_k0, align)) return OMX_ERR_ARG;
+    j.M = q.m;
+    j.N = q.n;
+    j.K = q.k;
+    j.xstrip = (q.x_ldk / es) * kChunk;
+    j.ystrip = (q.y_ldk / es) * kChunk;
+    j.X = static_cast<const char *>(q.X) + (q.x_row0 / OMX_STRIP) * j.xstrip + (q.x_k0 / es) * kChunk;
+    j.Y = static_cast<const char *>(q.Y) + (q.y_row0 / OMX_STRIP) * j.ystrip + (q.y_k0 / es) * kChunk;
+    j.C = q.C;
+    j.ldc = q.ldc;
+    j.tiles_m = (int)omx_cdiv(q.m, OMX_STRIP);
+    j.tiles_n = (int)omx_cdiv(q.n, OMX_STRIP);
+    j.ktri = q.tri;
+    j.tmax = q.tile_max;
+    j.tmax_tr = q.tri == 2 ? 1 : 0;
+    if (fp8) {
+        if (!q.xexp || !q.yexp) return OMX_ERR_ARG;
+        j.xet = q.x_ldk / OMX_SCALE_TILE;
+        j.yet = q.y_ldk / OMX_SCALE_TILE;
+        j.xexp = q.xexp + (q.x_row0 / OMX_STRIP) * j.xet + q.x_k0 / OMX_SCALE_TILE;
+        j.yexp = q.yexp + (q.y_row0 / OMX_STRIP) * j.yet + q.y_k0 / OMX_SCALE_TILE;
+    }
+    return OMX_OK;
+}
+
+bool pair_splits(const omx_gemm_job *q) {
+    // a product without rows or columns, or the other kernel family
+    return use_half_tiles() || q[0].m == 0 || q[0].n == 0 || q[1].m == 0 || q[1].n == 0;
+}
+
+}  // namespace
+
+int omx_gemm_f16_pair(const omx_gemm_job *q, float alpha, float beta, void *stream) {
+    if (pair_splits(q)) {
+        for (int i = 0; i < 2; ++i) {
+            const int rc = gemm_f16_launch(q[i].m, q[i].n, q[i].k, alpha, static_cast<const uint16_t *>(q[i].X), nullptr,
+                                           q[i].x_row0, q[i].x_ldk, q[i].x_k0, static_cast<const uint16_t *>(q[i].Y),
+                                           nullptr, q[i].y_row0, q[i].y_ldk, q[i].y_k0, beta, q[i].C, q[i].ldc,
+                                           q[i].tri, q[i].tile_max, stream);
+            if (rc) return rc;
+        }
+        return OMX_OK;
+    }
+    GemmJob j[2] = {};
+    for (int i = 0; i < 2; ++i) {
+        const int rc = resolve_job(q[i], OMX_KSTAGE16, false, j[i]);
+        if (rc) return rc;
+    }
+    const bool tmax = q[0].tile_max && q[1].tile_max;
+    if ((q[0].tile_max || q[1].tile_max) && (!tmax || beta != 0.0f)) return OMX_ERR_ARG;
+    const int64_t split = (int64_t)j[0].tiles_m * j[0].tiles_n, total = split + (int64_t)j[1].tiles_m * j[1].tiles_n;
+    if (total >= ((int64_t)1 << 31)) return OMX_ERR_ARG;
+    const dim3 grid((unsigned)total);
+#define OMX_PAIR_F16(BZ, TM)                                                                                      \
+    hipLaunchKernelGGL((k_gemm_f16<BZ, kNbuf, TM, true>), grid, dim3(kThreads), 0, omx_stream(stream), j[0].M, j[0].N, \
+                       j[0].K, alpha, beta, j[0].X, j[0].Y, j[0].C, j[0].ldc, j[0].tiles_m, j[0].tiles_n, nullptr, \
+                       nullptr, j[0].xstrip, j[0].ystrip, j[0].ktri, j[0].tmax, j[0].tmax_tr, j[1], (int)split)
+    if (tmax) OMX_PAIR_F16(true, true);
+    else if (beta == 0.0f) OMX_PAIR_F16(true, false);
+    else OMX_PAIR_F16(false, false);
+#undef OMX_PAIR_F16
+    OMX_LAUNCH_CHECK();
+    return OMX_OK;
+}
+
+int omx_gemm_f8_pair(const omx_gemm_job *q, float alpha, float beta, void *stream) {
+    if (pair_splits(q) || beta == 0.0f) {
+        for (int i = 0; i < 2; ++i) {
+            const int rc = omx_gemm_f8_packed_window(q[i].m, q[i].n, q[i].k, alpha, static_cast<const uint8_t *>(q[i].X),
+                                                     q[i].xexp, q[i].x_row0, q[i].x_ldk, q[i].x_k0,
+                                                     static_cast<const uint8_t *>(q[i].Y), q[i].yexp, q[i].y_row0,
+                                                     q[i].y_ldk, q[i].y_k0, beta, q[i].C, q[i].ldc, stream);
+            if (rc) return rc;
+        }
+        return OMX_OK;
+    }
+    GemmJob j[2] = {};
+    for (int i = 0; i < 2; ++i) {
+        const int rc = resolve_job(q[i], OMX_KSTAGE8, true, j[i]);
+        if (rc) return rc;
+    }
+    const int64_t split = (int64_t)j[0].tiles_m * j[0].tiles_n, total = split + (int64_t)j[1].tiles_m * j[1].tiles_n;
+    if (total >= ((int64_t)1 << 31)) return OMX_ERR_ARG;
+    hipLaunchKernelGGL((k_gemm_f8<false, kNbuf, true>), dim3((unsigned)total), dim3(kThreads), 0, omx_stream(stream),
+                       j[0].M, j[0].N, j[0].K, alpha, beta, j[0].X, j[0].xexp, j[0].Y, j[0].yexp, j[0].C, j[0].ldc,
+                       j[0].tiles_m, j[0].tiles_n, j[0].xstrip, j[0].ystrip, j[0].xet, j[0].yet, j[1], (int)split);
+    OMX_LAUNCH_CHECK();
+    return OMX_OK;
+}

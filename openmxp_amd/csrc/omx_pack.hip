@@ -8,6 +8,7 @@
 // half_conversion_left / half_conversion_right_trans
 // (fp16_gpu_kernels.cpp:11-36, :157-211).  Rows past R are packed as zeros.
 #include "omx_common.hpp"
+#include "omx_internal.hpp"
 #include "omx_layout.hpp"
 
 namespace {
@@ -53,30 +54,69 @@ __device__ __forceinline__ void load_run(const float *__restrict__ src, int64_t 
     }
 }
 
+// A launch packs up to kPackJobs panels of equal K (a step's inverses and
+// panels: as single launches, 7 us each where the panels are small); their
+// row strips follow each other in blockIdx.y.
+constexpr int kPackJobs = 4;
+
+struct PackJob {
+    const float *src;
+    int64_t R, rs, ls;
+    void *P;
+    int64_t pchunks, pk0;     // packed chunks per strip; the panel's first
+    float *chunk_max;         // FP16, optional
+    const int32_t *sexp;      // FP16, optional: per-strip scales
+    const float *tmax;        // FP8: tile maxima
+    int32_t *exps;            // FP8
+    int64_t ekt, ek0;         // FP8: exponents per strip; the panel's first
+    int mask, headroom;
+};
+
+struct PackJobs {
+    PackJob job[kPackJobs];
+    int64_t end[kPackJobs];   // strips of the jobs up to and with this one
+};
+
+// the workgroup's job and row strip
+__device__ __forceinline__ const PackJob &pack_job(const PackJobs &p, int64_t &strip) {
+    int q = 0;
+    int64_t first = 0;
+#pragma unroll
+    for (int i = 0; i + 1 < kPackJobs; ++i) {
+        if ((int64_t)blockIdx.y >= p.end[i]) {
+            q = i + 1;
+            first = p.end[i];
+        }
+    }
+    strip = (int64_t)blockIdx.y - first;
+    return p.job[q];
+}
+
 // One workgroup per (row strip, 64-column stage): 32 KB of packed output.
 // Each thread writes 8 of the stage's 2048 16-byte units (8 consecutive k of
 // one row); all 64 of its source values are loaded, straight from the panel,
 // before the first is converted, so a workgroup's 64 KB arrive in one round
 // trip.
 __global__ void __launch_bounds__(kPackThreads)
-k_pack_f16(int64_t R, int64_t K, const float *__restrict__ src, int64_t rs, int64_t ls,
-           int mask, _Float16 *__restrict__ P, float *__restrict__ chunk_max,
-           const int32_t *__restrict__ sexp, int64_t pchunks, int64_t pk0) {
+k_pack_f16(int64_t K, PackJobs jobs) {
     __shared__ float red[kPackThreads / 64];
+    int64_t rsb;                     // row strip
+    const PackJob j = pack_job(jobs, rsb);
     const int64_t ks = blockIdx.x;   // K-stage
-    const int64_t rsb = blockIdx.y;  // row strip
+    const int64_t R = j.R;
     const int64_t r0 = rsb * OMX_STRIP, k0 = ks * kTileK;
     // the packed panel has pchunks 64-column chunks per strip; this panel's
     // columns start at chunk pk0
-    _Float16 *out = P + (rsb * pchunks + pk0 + ks) * 16384;
+    _Float16 *out = static_cast<_Float16 *>(j.P) + (rsb * j.pchunks + j.pk0 + ks) * 16384;
     const int t = threadIdx.x;
-    const float scale = sexp ? ldexpf(1.0f, sexp[rsb]) : 1.0f;
+    const float scale = j.sexp ? ldexpf(1.0f, j.sexp[rsb]) : 1.0f;
     float v[8][8];
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         const int oidx = t + kPackThreads * q;  // 16-byte unit, 0..2047
         const int fb = oidx >> 6, lane = oidx & 63;
-        load_run<8>(src, rs, ls, R, r0 + (fb >> 2) * 32 + (lane & 31), k0 + (fb & 3) * 16 + (lane >> 5) * 8, v[q]);
+        load_run<8>(j.src, j.rs, j.ls, R, r0 + (fb >> 2) * 32 + (lane & 31), k0 + (fb & 3) * 16 + (lane >> 5) * 8,
+                    v[q]);
     }
     float mx = 0.0f;
 #pragma unroll
@@ -89,18 +129,18 @@ k_pack_f16(int64_t R, int64_t K, const float *__restrict__ src, int64_t rs, int6
         half8 h;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float x = (r < R) ? apply_mask(v[q][e], r, kb + e, mask) : 0.0f;
+            const float x = (r < R) ? apply_mask(v[q][e], r, kb + e, j.mask) : 0.0f;
             mx = fmaxf(mx, fabsf(x));
             h[e] = (_Float16)(x * scale);
         }
         *reinterpret_cast<half8 *>(out + oidx * 8) = h;
     }
-    if (chunk_max) {
+    if (j.chunk_max) {
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
         if ((t & 63) == 0) red[t >> 6] = mx;
         __syncthreads();
         if (t == 0)
-            chunk_max[rsb * (K >> 6) + ks] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            j.chunk_max[rsb * (K >> 6) + ks] = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     }
 }
 
@@ -155,15 +195,10 @@ __device__ __forceinline__ int pow2_exp_448(float maxabs) {
     return e > 100 ? 100 : (e < -100 ? -100 : e);
 }
 
-// exps[strip * ekt + ek0 + t] from tmax[strip * KT + t] (the exponent array
-// may span a wider packed panel than the tile maxima)
-__global__ void k_tile_exps(int64_t n, int64_t KT, const float *__restrict__ tmax, int headroom,
-                            int32_t *__restrict__ exps, int64_t ekt, int64_t ek0) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const int e = pow2_exp_448(tmax[i]);
-        exps[(i / KT) * ekt + ek0 + i % KT] = (tmax[i] > 0.0f) ? (e - headroom < -100 ? -100 : e - headroom) : 0;
-    }
+// the exponent of a scale tile with maximum m, `headroom` bits below
+__device__ __forceinline__ int tile_exp(float m, int headroom) {
+    const int e = pow2_exp_448(m);
+    return (m > 0.0f) ? (e - headroom < -100 ? -100 : e - headroom) : 0;
 }
 
 // Per-strip FP16 scale: the largest e with max|strip| * 2^e <= 2^15 (half the
@@ -186,19 +221,25 @@ __global__ void k_strip_exps16(int64_t nstrips, int64_t KT, const float *__restr
 
 // FP8 pack: one workgroup per (row strip, 64-column half of a 128 stage);
 // each thread writes 4 16-byte units (16 consecutive k of one row), its 64
-// source values loaded straight from the panel first.
+// source values loaded straight from the panel first.  Every workgroup forms
+// its scale tile's exponent from the tile maximum; the tile's first one
+// stores it (a launch of its own before each pack took 8 us).
 __global__ void __launch_bounds__(kPackThreads)
-k_pack_f8(int64_t R, int64_t K, const float *__restrict__ src, int64_t rs, int64_t ls,
-          const int32_t *__restrict__ exps, uint8_t *__restrict__ P, int64_t pchunks, int64_t pk0,
-          int64_t ekt, int64_t ek0) {
+k_pack_f8(int64_t K, PackJobs jobs) {
+    int64_t rsb;
+    const PackJob j = pack_job(jobs, rsb);
     const int64_t k64 = blockIdx.x;  // 64-column block
-    const int64_t rsb = blockIdx.y;
+    const int64_t R = j.R, rs = j.rs, ls = j.ls;
+    const float *src = j.src;
     const int64_t r0 = rsb * OMX_STRIP, k0 = k64 * kTileK;
-    const float scale = ldexpf(1.0f, exps[rsb * ekt + ek0 + k0 / OMX_SCALE_TILE]);
+    const int64_t kt = k0 / OMX_SCALE_TILE;
+    const int e = tile_exp(j.tmax[rsb * (K / OMX_SCALE_TILE) + kt], j.headroom);
+    if (k0 % OMX_SCALE_TILE == 0 && threadIdx.x == 0) j.exps[rsb * j.ekt + j.ek0 + kt] = e;
+    const float scale = ldexpf(1.0f, e);
     const int64_t ks = k64 >> 1;
     const int kk = (int)(k64 & 1);
     // pchunks 128-column chunks per strip; this panel starts at chunk pk0
-    uint8_t *chunk = P + (rsb * pchunks + pk0 + ks) * 32768;
+    uint8_t *chunk = static_cast<uint8_t *>(j.P) + (rsb * j.pchunks + j.pk0 + ks) * 32768;
     const int t = threadIdx.x;
     float v[4][16];
 #pragma unroll
@@ -226,6 +267,63 @@ k_pack_f8(int64_t R, int64_t K, const float *__restrict__ src, int64_t rs, int64
     }
 }
 
+bool pack_source_ok(const float *src, int64_t rows, int64_t k, int64_t rs, int64_t ls) {
+    if (!((rs == 1 && ls >= rows) || (ls == 1 && rs >= k))) return false;
+    return !(ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15)));
+}
+
+// one launch of k_pack_f16 / k_pack_f8 over count jobs of k columns
+int launch_pack(bool fp8, int64_t k, int count, const PackJob *job, hipStream_t st) {
+    PackJobs p{};
+    int64_t strips = 0;
+    for (int i = 0; i < kPackJobs; ++i) {
+        if (i < count) {
+            p.job[i] = job[i];
+            strips += omx_strips(job[i].R);
+        }
+        p.end[i] = strips;
+    }
+    const dim3 grid((unsigned)(k / kTileK), (unsigned)strips);
+    if (fp8)
+        hipLaunchKernelGGL(k_pack_f8, grid, dim3(kPackThreads), 0, st, k, p);
+    else
+        hipLaunchKernelGGL(k_pack_f16, grid, dim3(kPackThreads), 0, st, k, p);
+    OMX_LAUNCH_CHECK();
+    return OMX_OK;
+}
+
+PackJob job_f16(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int mask, void *P, int64_t ldk,
+                int64_t k0) {
+    PackJob j{};
+    j.src = src;
+    j.R = rows;
+    j.rs = rs;
+    j.ls = ls;
+    j.P = P;
+    j.pchunks = ldk / OMX_KSTAGE16;
+    j.pk0 = k0 / OMX_KSTAGE16;
+    j.mask = mask;
+    return j;
+}
+
+PackJob job_f8(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int headroom, void *P,
+               int32_t *exps, const float *tmax, int64_t ldk, int64_t k0) {
+    PackJob j{};
+    j.src = src;
+    j.R = rows;
+    j.rs = rs;
+    j.ls = ls;
+    j.P = P;
+    j.pchunks = ldk / OMX_KSTAGE8;
+    j.pk0 = k0 / OMX_KSTAGE8;
+    j.tmax = tmax;
+    j.exps = exps;
+    j.ekt = ldk / OMX_SCALE_TILE;
+    j.ek0 = k0 / OMX_SCALE_TILE;
+    j.headroom = headroom;
+    return j;
+}
+
 }  // namespace
 
 extern "C" {
@@ -243,20 +341,16 @@ size_t omx_panel_exps_count(int64_t rows, int64_t k) {
 int omx_pack_f16(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int mask,
                  uint16_t *P, float *chunk_max, void *stream) {
     if (rows <= 0 || k <= 0 || k % OMX_KSTAGE16 || !src || !P || mask < 0 || mask > 3) return OMX_ERR_ARG;
-    if (!((rs == 1 && ls >= rows) || (ls == 1 && rs >= k))) return OMX_ERR_ARG;
-    if (ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15))) return OMX_ERR_ARG;
-    dim3 grid((unsigned)(k / kTileK), (unsigned)omx_strips(rows));
-    hipLaunchKernelGGL(k_pack_f16, grid, dim3(kPackThreads), 0, omx_stream(stream), rows, k, src, rs,
-                       ls, mask, reinterpret_cast<_Float16 *>(P), chunk_max, nullptr, k / 64, (int64_t)0);
-    OMX_LAUNCH_CHECK();
-    return OMX_OK;
+    if (!pack_source_ok(src, rows, k, rs, ls)) return OMX_ERR_ARG;
+    PackJob j = job_f16(rows, k, src, rs, ls, mask, P, k, 0);
+    j.chunk_max = chunk_max;
+    return launch_pack(false, k, 1, &j, omx_stream(stream));
 }
 
 int omx_pack_f16_scaled(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int have_max,
                         uint16_t *P, int32_t *sexp, float *tile_max, void *stream) {
     if (rows <= 0 || k <= 0 || k % OMX_SCALE_TILE || !src || !P || !sexp || !tile_max) return OMX_ERR_ARG;
-    if (!((rs == 1 && ls >= rows) || (ls == 1 && rs >= k))) return OMX_ERR_ARG;
-    if (ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15))) return OMX_ERR_ARG;
+    if (!pack_source_ok(src, rows, k, rs, ls)) return OMX_ERR_ARG;
     hipStream_t st = omx_stream(stream);
     const int64_t strips = omx_strips(rows), KT = omx_cdiv(k, OMX_SCALE_TILE);
     if (!have_max) {
@@ -267,11 +361,9 @@ int omx_pack_f16_scaled(int64_t rows, int64_t k, const float *src, int64_t rs, i
     hipLaunchKernelGGL(k_strip_exps16, dim3((unsigned)omx_cdiv(strips, 256)), dim3(256), 0, st, strips, KT, tile_max,
                        sexp);
     OMX_LAUNCH_CHECK();
-    dim3 grid((unsigned)(k / kTileK), (unsigned)strips);
-    hipLaunchKernelGGL(k_pack_f16, grid, dim3(kPackThreads), 0, st, rows, k, src, rs, ls, (int)OMX_MASK_NONE,
-                       reinterpret_cast<_Float16 *>(P), nullptr, sexp, k / 64, (int64_t)0);
-    OMX_LAUNCH_CHECK();
-    return OMX_OK;
+    PackJob j = job_f16(rows, k, src, rs, ls, OMX_MASK_NONE, P, k, 0);
+    j.sexp = sexp;
+    return launch_pack(false, k, 1, &j, st);
 }
 
 int omx_pack_f8_window(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int headroom, int have_max,
@@ -279,8 +371,7 @@ int omx_pack_f8_window(int64_t rows, int64_t k, const float *src, int64_t rs, in
     if (rows <= 0 || k <= 0 || k % OMX_SCALE_TILE || !src || !P || !exps || !tile_max) return OMX_ERR_ARG;
     if (ldk <= 0 || ldk % OMX_SCALE_TILE || k0 < 0 || k0 % OMX_SCALE_TILE || k0 + k > ldk) return OMX_ERR_ARG;
     if (headroom < 0 || headroom > 3) return OMX_ERR_ARG;
-    if (!((rs == 1 && ls >= rows) || (ls == 1 && rs >= k))) return OMX_ERR_ARG;
-    if (ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15))) return OMX_ERR_ARG;
+    if (!pack_source_ok(src, rows, k, rs, ls)) return OMX_ERR_ARG;
     hipStream_t st = omx_stream(stream);
     const int64_t strips = omx_strips(rows), KT = omx_cdiv(k, OMX_SCALE_TILE);
     if (!have_max) {
@@ -288,15 +379,8 @@ int omx_pack_f8_window(int64_t rows, int64_t k, const float *src, int64_t rs, in
                            rows, k, src, rs, ls, tile_max);
         OMX_LAUNCH_CHECK();
     }
-    const int64_t nt = strips * KT;
-    const int64_t ekt = ldk / OMX_SCALE_TILE, ek0 = k0 / OMX_SCALE_TILE;
-    hipLaunchKernelGGL(k_tile_exps, dim3((unsigned)omx_cdiv(nt, 256)), dim3(256), 0, st, nt, KT, tile_max, headroom,
-                       exps, ekt, ek0);
-    OMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_pack_f8, dim3((unsigned)(k / kTileK), (unsigned)strips), dim3(kPackThreads), 0,
-                       st, rows, k, src, rs, ls, exps, P, ldk / OMX_KSTAGE8, k0 / OMX_KSTAGE8, ekt, ek0);
-    OMX_LAUNCH_CHECK();
-    return OMX_OK;
+    const PackJob j = job_f8(rows, k, src, rs, ls, headroom, P, exps, tile_max, ldk, k0);
+    return launch_pack(true, k, 1, &j, st);
 }
 
 int omx_pack_f8_ex(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int headroom, int have_max,
@@ -309,8 +393,7 @@ int omx_pack_f16_window(int64_t rows, int64_t k, const float *src, int64_t rs, i
     if (rows <= 0 || k <= 0 || k % OMX_KSTAGE16 || !src || !P) return OMX_ERR_ARG;
     if (ldk <= 0 || ldk % OMX_KSTAGE16 || k0 < 0 || k0 % OMX_KSTAGE16 || k0 + k > ldk) return OMX_ERR_ARG;
     if (sexp && (!tile_max || k % OMX_SCALE_TILE)) return OMX_ERR_ARG;
-    if (!((rs == 1 && ls >= rows) || (ls == 1 && rs >= k))) return OMX_ERR_ARG;
-    if (ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15))) return OMX_ERR_ARG;
+    if (!pack_source_ok(src, rows, k, rs, ls)) return OMX_ERR_ARG;
     hipStream_t st = omx_stream(stream);
     const int64_t strips = omx_strips(rows);
     if (sexp) {
@@ -324,11 +407,9 @@ int omx_pack_f16_window(int64_t rows, int64_t k, const float *src, int64_t rs, i
                            tile_max, sexp);
         OMX_LAUNCH_CHECK();
     }
-    dim3 grid((unsigned)(k / kTileK), (unsigned)strips);
-    hipLaunchKernelGGL(k_pack_f16, grid, dim3(kPackThreads), 0, st, rows, k, src, rs, ls, (int)OMX_MASK_NONE,
-                       reinterpret_cast<_Float16 *>(P), nullptr, sexp, ldk / 64, k0 / 64);
-    OMX_LAUNCH_CHECK();
-    return OMX_OK;
+    PackJob j = job_f16(rows, k, src, rs, ls, OMX_MASK_NONE, P, ldk, k0);
+    j.sexp = sexp;
+    return launch_pack(false, k, 1, &j, st);
 }
 
 int omx_pack_f8(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, uint8_t *P,
@@ -348,3 +429,29 @@ int omx_panel_tile_maxabs(int64_t rows, int64_t k, const float *src, int64_t rs,
 }
 
 }  // extern "C"
+
+int omx_pack_f16_jobs(int count, const omx_pack_job *jobs, void *stream) {
+    if (count < 1 || count > kPackJobs) return OMX_ERR_ARG;
+    PackJob j[kPackJobs];
+    for (int i = 0; i < count; ++i) {
+        const omx_pack_job &q = jobs[i];
+        if (q.rows <= 0 || q.k <= 0 || q.k != jobs[0].k || q.k % OMX_KSTAGE16 || !q.src || !q.P ||
+            !pack_source_ok(q.src, q.rows, q.k, q.rs, q.ls))
+            return OMX_ERR_ARG;
+        j[i] = job_f16(q.rows, q.k, q.src, q.rs, q.ls, q.mask, q.P, q.ldk, q.k0);
+    }
+    return launch_pack(false, jobs[0].k, count, j, omx_stream(stream));
+}
+
+int omx_pack_f8_jobs(int count, const omx_pack_job *jobs, void *stream) {
+    if (count < 1 || count > kPackJobs) return OMX_ERR_ARG;
+    PackJob j[kPackJobs];
+    for (int i = 0; i < count; ++i) {
+        const omx_pack_job &q = jobs[i];
+        if (q.rows <= 0 || q.k <= 0 || q.k != jobs[0].k || q.k % OMX_SCALE_TILE || !q.src || !q.P || !q.exps ||
+            !q.tile_max || q.headroom < 0 || q.headroom > 3 || !pack_source_ok(q.src, q.rows, q.k, q.rs, q.ls))
+            return OMX_ERR_ARG;
+        j[i] = job_f8(q.rows, q.k, q.src, q.rs, q.ls, q.headroom, q.P, q.exps, q.tile_max, q.ldk, q.k0);
+    }
+    return launch_pack(true, jobs[0].k, count, j, omx_stream(stream));
+}

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "omx_common.hpp"
+#include "omx_internal.hpp"
 #include "omx_layout.hpp"
 
 #define RC(x)                  \
@@ -159,7 +160,7 @@ struct omx_solver {
     hipStream_t crit = nullptr, bulk = nullptr;
     std::vector<hipEvent_t> ev_panel, ev_t0, ev_t1;
     int64_t G = 2;                      // panels per trailing update (group)
-    DevBuf Lp[2], Rp[2], Tp;            // FP16 group buffers (K = G b) and the -alt temporary
+    DevBuf Lp[2], Rp[2], Tp;            // FP16 group buffers (K = G b) and the -alt temporaries (column, row panel)
     DevBuf L8[2], R8[2], Le[2], Re[2];  // FP8 group buffers and their exponents
     DevBuf L8max, R8max;                // tile max-abs scratch
     int scale16 = 0;                    // FP16 Schur panels with per-strip scales
@@ -370,7 +371,7 @@ int omx_solver_create(int64_t n, int64_t b, int alt, int flags, omx_solver **out
     s->last_sched.assign(nb, 0);
     s->prec.assign(nb, 0);
     s->last_feat.assign((size_t)nb * OMX_MLP_NFEATURES, 0.0f);
-    if ((rc = dalloc(s->Tp, omx_panel_bytes(rows, b, 0)))) return fail(rc);
+    if ((rc = dalloc(s->Tp, 2 * omx_panel_bytes(rows, b, 0)))) return fail(rc);
     if ((rc = dalloc(s->Wup, (size_t)b * b * 4)) || (rc = dalloc(s->Wlo, (size_t)b * b * 4)) ||
         (rc = dalloc(s->Wtmp, (size_t)b * b * 4)) ||
         (rc = dalloc(s->Wup_h, omx_panel_bytes(b, b, 0))) || (rc = dalloc(s->Wlo_h, omx_panel_bytes(b, b, 0))))
@@ -427,24 +428,44 @@ static inline int64_t pwin(int64_t i, int64_t b, int64_t G) { return (i % G) * b
 
 // A(r0:r0+m, c0:c0+nn) -= L R^T over K window [k0, k0 + k) of panel i's
 // group buffer (the panels whose windows it spans, from panel i on).
-static int schur_window(omx_solver *s, int64_t i, int64_t k, int64_t k0, int64_t r0, int64_t c0, int64_t m,
-                        int64_t nn, float *A, int64_t lda, hipStream_t st) {
+static omx_gemm_job schur_job(omx_solver *s, int64_t i, int64_t k, int64_t k0, int64_t r0, int64_t c0, int64_t m,
+                              int64_t nn, float *A, int64_t lda) {
     const int64_t b = s->b, G = s->G, ldk = G * b;
     const int buf = pbuf(i, G);
-    const int64_t xr0 = r0 - porigin(i, b, G), yr0 = c0 - porigin(i, b, G);
-    float *C = A + r0 + c0 * lda;
-    if (s->prec[i])
-        return omx_gemm_f8_packed_window(m, nn, k, -1.0f, static_cast<uint8_t *>(s->L8[buf].p),
-                                         static_cast<int32_t *>(s->Le[buf].p), xr0, ldk, k0,
-                                         static_cast<uint8_t *>(s->R8[buf].p), static_cast<int32_t *>(s->Re[buf].p),
-                                         yr0, ldk, k0, 1.0f, C, lda, st);
-    const int32_t *xe = nullptr, *ye = nullptr;
-    if (s->scale16) {
-        xe = static_cast<int32_t *>(s->Lse[G * buf + i % G].p);
-        ye = static_cast<int32_t *>(s->Rse[G * buf + i % G].p);
+    omx_gemm_job q{};
+    q.m = m;
+    q.n = nn;
+    q.k = k;
+    q.x_row0 = r0 - porigin(i, b, G);
+    q.y_row0 = c0 - porigin(i, b, G);
+    q.x_ldk = q.y_ldk = ldk;
+    q.x_k0 = q.y_k0 = k0;
+    q.C = A + r0 + c0 * lda;
+    q.ldc = lda;
+    if (s->prec[i]) {
+        q.X = s->L8[buf].p;
+        q.Y = s->R8[buf].p;
+        q.xexp = static_cast<int32_t *>(s->Le[buf].p);
+        q.yexp = static_cast<int32_t *>(s->Re[buf].p);
+        return q;
     }
-    return omx_gemm_f16_packed_window(m, nn, k, -1.0f, static_cast<uint16_t *>(s->Lp[buf].p), xe, xr0, ldk, k0,
-                                      static_cast<uint16_t *>(s->Rp[buf].p), ye, yr0, ldk, k0, 1.0f, C, lda, st);
+    q.X = s->Lp[buf].p;
+    q.Y = s->Rp[buf].p;
+    if (s->scale16) {
+        q.xexp = static_cast<int32_t *>(s->Lse[G * buf + i % G].p);
+        q.yexp = static_cast<int32_t *>(s->Rse[G * buf + i % G].p);
+    }
+    return q;
+}
+
+static int schur_window(omx_solver *s, int64_t i, const omx_gemm_job &q, hipStream_t st) {
+    if (s->prec[i])
+        return omx_gemm_f8_packed_window(q.m, q.n, q.k, -1.0f, static_cast<const uint8_t *>(q.X), q.xexp, q.x_row0,
+                                         q.x_ldk, q.x_k0, static_cast<const uint8_t *>(q.Y), q.yexp, q.y_row0, q.y_ldk,
+                                         q.y_k0, 1.0f, q.C, q.ldc, st);
+    return omx_gemm_f16_packed_window(q.m, q.n, q.k, -1.0f, static_cast<const uint16_t *>(q.X), q.xexp, q.x_row0,
+                                      q.x_ldk, q.x_k0, static_cast<const uint16_t *>(q.Y), q.yexp, q.y_row0, q.y_ldk,
+                                      q.y_k0, 1.0f, q.C, q.ldc, st);
 }
 
 // A(r0.., c0..) (m x nn) -= the panels i0 .. i1 (all in one group), in
@@ -452,25 +473,46 @@ static int schur_window(omx_solver *s, int64_t i, int64_t k, int64_t k0, int64_t
 // its K windows (scaled FP16 panels, whose scales are per panel, one by one).
 static int prec_class(int p) { return p > 0 ? 1 : (p < 0 ? -1 : 0); }
 
-static int apply_panels(omx_solver *s, int64_t i0, int64_t i1, int64_t r0, int64_t c0, int64_t m, int64_t nn,
-                        float *A, int64_t lda, hipStream_t st) {
-    if (m <= 0 || nn <= 0) return OMX_OK;
+struct Target {
+    int64_t r0, c0, m, nn;
+};
+
+// The same to one or two disjoint targets (a block row and column: in one
+// launch).
+static int apply_panels(omx_solver *s, int64_t i0, int64_t i1, const Target *t, int nt, float *A, int64_t lda,
+                        hipStream_t st) {
     const int64_t b = s->b, G = s->G;
     for (int64_t i = i0; i <= i1;) {
         int64_t j = i;
         const int cls = prec_class(s->prec[i]);
         if (cls != 0 || !s->scale16)
             while (j + 1 <= i1 && (j + 1) / G == i / G && prec_class(s->prec[j + 1]) == cls) ++j;
-        if (cls < 0) {
-            // FP32 class: C -= A(r0.., ib..jb+b) A(ib..jb+b, c0..), the
-            // panels as factored (column panels side by side, row panels
-            // stacked), on the FP32 matrix cores
-            const int64_t ib = i * b, k = (j - i + 1) * b;
-            RC(omx_sgemm_f32(m, nn, k, -1.0f, A + r0 + ib * lda, lda, A + ib + c0 * lda, lda, 1.0f,
-                             A + r0 + c0 * lda, lda, st));
-        } else {
-            RC(schur_window(s, i, (j - i + 1) * b, pwin(i, b, G), r0, c0, m, nn, A, lda, st));
+        const int64_t ib = i * b, k = (j - i + 1) * b;
+        omx_gemm_job q[2];
+        int nq = 0;
+        for (int u = 0; u < nt; ++u) {
+            if (t[u].m <= 0 || t[u].nn <= 0) continue;
+            if (cls < 0) {
+                // FP32 class: C -= A(r0.., ib..jb+b) A(ib..jb+b, c0..), the
+                // panels as factored (column panels side by side, row panels
+                // stacked), on the FP32 matrix cores
+                RC(omx_sgemm_f32(t[u].m, t[u].nn, k, -1.0f, A + t[u].r0 + ib * lda, lda, A + ib + t[u].c0 * lda, lda,
+                                 1.0f, A + t[u].r0 + t[u].c0 * lda, lda, st));
+            } else {
+                q[nq++] = schur_job(s, i, k, pwin(i, b, G), t[u].r0, t[u].c0, t[u].m, t[u].nn, A, lda);
+            }
         }
+        // one launch where the first product has at most a tile per CU (its
+        // launch lasts as long as a tile; n = 10240, b = 256: LU 8.0 -> 7.0
+        // ms); larger ones gain nothing side by side and lose the cache
+        // (n = 61440, b = 2560: 116.6 ms by themselves, 120 in one launch)
+        const bool pair = nq == 2 && q[0].m * q[0].n <= (int64_t)256 * OMX_STRIP * OMX_STRIP;
+        if (pair && cls > 0)
+            RC(omx_gemm_f8_pair(q, -1.0f, 1.0f, st));
+        else if (pair && !s->scale16)
+            RC(omx_gemm_f16_pair(q, -1.0f, 1.0f, st));
+        else
+            for (int u = 0; u < nq; ++u) RC(schur_window(s, i, q[u], st));
         i = j + 1;
     }
     return OMX_OK;
@@ -483,8 +525,8 @@ static int update_block(omx_solver *s, int64_t t, int64_t i0, int64_t i1, float 
     const double fl = 2.0 * (double)(i1 - i0 + 1) * b * b * (2.0 * (n - tb) - b);
     long sp;
     RC(s->timers.beg(kT_GEMM_UPDATE, st, &sp));
-    RC(apply_panels(s, i0, i1, tb, tb, n - tb, b, A, lda, st));
-    RC(apply_panels(s, i0, i1, tb, tb + b, b, n - tb - b, A, lda, st));
+    const Target tg[2] = {{tb, tb, n - tb, b}, {tb, tb + b, b, n - tb - b}};
+    RC(apply_panels(s, i0, i1, tg, 2, A, lda, st));
     RC(s->timers.end(sp, st, fl));
     s->crit_flops += fl;
     return OMX_OK;
@@ -506,6 +548,12 @@ static int pack_panel(omx_solver *s, int64_t i, int have_max, int64_t rest, cons
         uint8_t *R8 = static_cast<uint8_t *>(s->R8[buf].p) + rstrip * sb8;
         int32_t *Le = static_cast<int32_t *>(s->Le[buf].p) + rstrip * ne;
         int32_t *Re = static_cast<int32_t *>(s->Re[buf].p) + rstrip * ne;
+        if (have_max && !s->timers.on) {  // (the phase timers time the two by themselves)
+            omx_pack_job q[2] = {};
+            q[0] = {rest, b, Acol, 1, lda, 0, L8, ldk, k0, h, Le, static_cast<float *>(s->L8max.p)};
+            q[1] = {rest, b, Arow, lda, 1, 0, R8, ldk, k0, h, Re, static_cast<float *>(s->R8max.p)};
+            return omx_pack_f8_jobs(2, q, st);
+        }
         TIMED(s->timers, kT_CONV_L, st, (double)rest * b,
               omx_pack_f8_window(rest, b, Acol, 1, lda, h, have_max, L8, Le, ldk, k0,
                                  static_cast<float *>(s->L8max.p), st));
@@ -517,6 +565,12 @@ static int pack_panel(omx_solver *s, int64_t i, int have_max, int64_t rest, cons
     const size_t sb16 = (size_t)(ldk / OMX_KSTAGE16) * 16384;  // uint16 per strip
     uint16_t *Lp = static_cast<uint16_t *>(s->Lp[buf].p) + rstrip * sb16;
     uint16_t *Rp = static_cast<uint16_t *>(s->Rp[buf].p) + rstrip * sb16;
+    if (!s->scale16 && !s->timers.on) {
+        omx_pack_job q[2] = {};
+        q[0] = {rest, b, Acol, 1, lda, OMX_MASK_NONE, Lp, ldk, k0, 0, nullptr, nullptr};
+        q[1] = {rest, b, Arow, lda, 1, OMX_MASK_NONE, Rp, ldk, k0, 0, nullptr, nullptr};
+        return omx_pack_f16_jobs(2, q, st);
+    }
     int32_t *xe = nullptr, *ye = nullptr;
     if (s->scale16) {
         xe = static_cast<int32_t *>(s->Lse[G * buf + i % G].p) + rstrip;
@@ -621,7 +675,7 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
     const bool learned = !sched && s->has_policy;
     const bool stats = s->fp8 != 0;
     int *info = static_cast<int *>(s->info.p);  // one slot per diagonal block
-    uint16_t *Tp = static_cast<uint16_t *>(s->Tp.p);
+    uint16_t *Tp = static_cast<uint16_t *>(s->Tp.p), *Tr = Tp + s->Tp.bytes / 4;
     float *Wup = static_cast<float *>(s->Wup.p), *Wlo = static_cast<float *>(s->Wlo.p);
     uint16_t *Wup_h = static_cast<uint16_t *>(s->Wup_h.p), *Wlo_h = static_cast<uint16_t *>(s->Wlo_h.p);
     s->bulk_count = 0;
@@ -677,29 +731,40 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
                 // U^-1 and L^-1 of the factored diagonal block
                 TIMED(T, kT_DIAG_LU, cs, 2.0 / 3.0 * b * (double)b * b,
                       omx_trtri_lu_f32(b, Akk, lda, Wup, Wlo, b, static_cast<float *>(s->Wtmp.p), cs));
-                // Y(j, l) = W(l, j), upper part only for -alt 2
-                long sp;
-                RC(T.beg(kT_CONV_L, cs, &sp));
-                RC(omx_pack_f16(b, b, Wup, b, 1, s->alt == 2 ? OMX_MASK_K_LE_R : OMX_MASK_NONE, Wup_h, nullptr, cs));
-                RC(omx_pack_f16(rest, b, Acol, 1, lda, OMX_MASK_NONE, Tp, nullptr, cs));
-                RC(T.end(sp, cs, (double)(rest + b) * b));
-                // U^-1 is upper triangular: each output column tile stops
-                // at its diagonal k tile (the rest of its products are
-                // zero).  With the statistics on, the product also leaves
-                // the column panel's tile maxima (no separate pass over it).
+                // Y(j, l) = W(l, j), upper part only for -alt 2; X(i, l) =
+                // W(i, l), strict lower + unit diagonal for -alt 2.  U^-1 is
+                // upper triangular: each output column tile stops at its
+                // diagonal k tile (the rest of its products are zero); L^-1
+                // lower: each output row tile likewise.  With the statistics
+                // on, the products also leave the panels' tile maxima (no
+                // separate pass over them).
+                const int mu = s->alt == 2 ? OMX_MASK_K_LE_R : OMX_MASK_NONE;
+                const int ml = s->alt == 2 ? OMX_MASK_R_GT_K_UNIT : OMX_MASK_NONE;
                 float *lmax = stats ? static_cast<float *>(s->L8max.p) : nullptr;
                 float *rmax = stats ? static_cast<float *>(s->R8max.p) : nullptr;
-                TIMED(T, kT_TRSM_L, cs, 2.0 * rb2,
-                      omx_gemm_f16_packed_tri(rest, b, b, 1.0f, Tp, Wup_h, 1, 0.0f, Acol, lda, lmax, cs));
-                // X(i, l) = W(i, l), strict lower + unit diagonal for -alt 2
-                RC(T.beg(kT_CONV_R, cs, &sp));
-                RC(omx_pack_f16(b, b, Wlo, 1, b, s->alt == 2 ? OMX_MASK_R_GT_K_UNIT : OMX_MASK_NONE, Wlo_h, nullptr,
-                                cs));
-                RC(omx_pack_f16(rest, b, Arow, lda, 1, OMX_MASK_NONE, Tp, nullptr, cs));
-                RC(T.end(sp, cs, (double)(rest + b) * b));
-                // L^-1 lower triangular: each output row tile likewise
-                TIMED(T, kT_TRSM_R, cs, 2.0 * rb2,
-                      omx_gemm_f16_packed_tri(b, rest, b, 1.0f, Wlo_h, Tp, 2, 0.0f, Arow, lda, rmax, cs));
+                const omx_pack_job pk[4] = {
+                    {b, b, Wup, b, 1, mu, Wup_h, b, 0, 0, nullptr, nullptr},
+                    {rest, b, Acol, 1, lda, OMX_MASK_NONE, Tp, b, 0, 0, nullptr, nullptr},
+                    {b, b, Wlo, 1, b, ml, Wlo_h, b, 0, 0, nullptr, nullptr},
+                    {rest, b, Arow, lda, 1, OMX_MASK_NONE, Tr, b, 0, 0, nullptr, nullptr}};
+                const omx_gemm_job pr[2] = {
+                    {rest, b, b, Tp, nullptr, 0, b, 0, Wup_h, nullptr, 0, b, 0, Acol, lda, 1, lmax},
+                    {b, rest, b, Wlo_h, nullptr, 0, b, 0, Tr, nullptr, 0, b, 0, Arow, lda, 2, rmax}};
+                if (!T.on) {
+                    // one launch for the four packs, one for the two products
+                    // (LU at n = 10240, b = 256: 10 launches of a step's
+                    // chain become 4; n = 61440, b = 2560: 117.0 -> 116.5 ms)
+                    RC(omx_pack_f16_jobs(4, pk, cs));
+                    RC(omx_gemm_f16_pair(pr, 1.0f, 0.0f, cs));
+                } else {
+                    // column, then row panel, each phase by itself
+                    TIMED(T, kT_CONV_L, cs, (double)(rest + b) * b, omx_pack_f16_jobs(2, pk, cs));
+                    TIMED(T, kT_TRSM_L, cs, 2.0 * rb2,
+                          omx_gemm_f16_packed_tri(rest, b, b, 1.0f, Tp, Wup_h, 1, 0.0f, Acol, lda, lmax, cs));
+                    TIMED(T, kT_CONV_R, cs, (double)(rest + b) * b, omx_pack_f16_jobs(2, pk + 2, cs));
+                    TIMED(T, kT_TRSM_R, cs, 2.0 * rb2,
+                          omx_gemm_f16_packed_tri(b, rest, b, 1.0f, Wlo_h, Tr, 2, 0.0f, Arow, lda, rmax, cs));
+                }
                 have_max = stats;
             }
             s->crit_flops += 4.0 * rest * (double)b * b;
@@ -737,9 +802,10 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
         const int64_t f = G * (g + 2);
         if (f < nb && !(s->skip & OMX_SKIP_GEMM)) {
             const int64_t m = n - f * b;
+            const Target tg{f * b, f * b, m, m};
             OMX_HIP_CHECK(hipEventRecord(s->ev_t0[s->bulk_count], bs));
             TIMED(T, kT_GEMM_UPDATE, bs, 2.0 * (double)m * m * (double)((i1 - i0 + 1) * b),
-                  apply_panels(s, i0, i1, f * b, f * b, m, m, A, lda, bs));
+                  apply_panels(s, i0, i1, &tg, 1, A, lda, bs));
             OMX_HIP_CHECK(hipEventRecord(s->ev_t1[s->bulk_count], bs));
             s->bulk_flops += 2.0 * (double)m * m * (double)((i1 - i0 + 1) * b);
             ++s->bulk_count;

@@ -228,3 +228,31 @@ def test_trsm_blocks(variant, w, lines, pad):
     else:
         L = np.tril(T64, -1) + np.eye(w)
         assert np.all(np.abs(L @ X - B) <= (w + 4) * 2.0 ** -24 * (np.abs(L) @ np.abs(X) + np.abs(B)))
+
+
+def _lu(n, b, alt, flags, sched, seed=3):
+    """Factors of the generated system; flags of omx_solver_create."""
+    import ctypes as C
+    torch = torch_cuda()
+    L = _L()
+    A, d = empty(n * n, torch.float32), empty(n, torch.float64)
+    assert L.omx_matgen_f32(n, seed, ptr(A), n, ptr(d), None) == 0
+    h = C.c_void_p()
+    assert L.omx_solver_create(n, b, alt, flags, C.byref(h)) == 0
+    s = np.ascontiguousarray(sched, np.int32)
+    assert L.omx_lu_factor(h, ptr(A), n, s.ctypes.data, None) == 0
+    L.omx_solver_destroy(h)
+    return host(A)
+
+
+# the solver with phase timers (flag 8) runs every pack and product of a step
+# as a launch of its own; without them a step's are merged: same factors, bit
+# for bit, for every panel method, precision and grouping
+@pytest.mark.parametrize("n,b,alt,flags,prec", [
+    (256, 256, 1, 0, 0), (512, 256, 1, 0, 0), (1536, 256, 1, 0, 0), (2560, 512, 2, 0, 0), (1280, 256, 0, 0, 0),
+    (1536, 256, 1, 1, 1), (2304, 256, 2, 5, 2), (3072, 768, 1, 5, 1), (2048, 256, 1, 2, 0), (1536, 256, 1, 0, -1),
+    (2560, 256, 1, 5, None)])
+def test_merged_launches_leave_the_factors_alone(n, b, alt, flags, prec):
+    nb = n // b
+    sched = [0, 1, -1, 2][:4] * nb if prec is None else [prec] * nb
+    assert np.array_equal(_lu(n, b, alt, flags, sched[:nb]), _lu(n, b, alt, flags | 8, sched[:nb]))
