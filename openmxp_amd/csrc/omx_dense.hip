@@ -96,28 +96,39 @@ k_sgemm_nn(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict
 
 // ---------------------------------------------------------------------------
 // The same product on the matrix cores (v_mfma_f32_32x32x2_f32), for the
-// large updates: a kT x kT tile (128, or 64 where 128-tiles would leave CUs
-// idle) per workgroup of four waves (a kT/2 square quadrant each, made of
-// 32 x 32 MFMA blocks), k staged through LDS up to 64 at a time, the next stage's global loads in flight during the current
-// stage's MFMAs.  The MFMA's first operand takes B (lane l: column l % 32),
-// the second A (lane l: row l % 32), so every accumulator register of lane l
-// belongs to row l % 32 of its block and a half-wave's C access is 32
-// consecutive rows of one column (one 128-byte line).  In a stage of kc
-// columns, lanes 0-31 carry k in [0, kc/2) and lanes 32-63 k in [kc/2, kc);
-// the MFMA adds the two halves.  Needs A and B 16-byte aligned with lda and
-// ldb multiples of 4, and k % 16 == 0 (so kc is a multiple of 16).
+// large updates: a 64 x 64 tile per workgroup of four waves (a 32 x 32 MFMA
+// block each), k staged through LDS up to 64 at a time, the next stage's
+// global loads in flight during the current stage's MFMAs.  The MFMA's first
+// operand takes B (lane l: column l % 32), the second A (lane l: row l % 32),
+// so every accumulator register of lane l belongs to row l % 32 of its block
+// and a half-wave's C access is 32 consecutive rows of one column (one
+// 128-byte line).  In a stage of kc columns, lanes 0-31 carry k in [0, kc/2)
+// and lanes 32-63 k in [kc/2, kc); the MFMA adds the two halves.  Needs A and
+// B 16-byte aligned with lda and ldb multiples of 4, and k % 16 == 0 (so kc
+// is a multiple of 16).
+//
+// Bound by the MFMAs where k is deep and by C's traffic where it is not; what
+// stood between was the time from a stage's loads to the next's.  A product
+// of whole groups of 64 and whole float4s of rows therefore steps pointers
+// and has no bounds in its loop: with the clamps the compiler put waits
+// between a stage's own loads, and a tile of four waves alone on its CU paid
+// for every address instruction.  Its last stage stands outside the loop, so
+// that C's old values are on their way during that stage's MFMAs.  Edge of 64
+// for every size: four workgroups a CU hide one another's loads and C better
+// than two of 128 x 128 did, whose operands are read half as often.  Measured
+// (128 x 128 or 64 x 64 tiles with bounds in the loop -> now), C -= A B:
+// 30000 x 2304 x 256 420 -> 355 us, 7680 x 7680 x 512 588 -> 523, 2048 x 2048 x
+// 512 47.5 -> 41.7, 30000 x 256 x 256 54.4 -> 46, 512 x 512 x 512 17.6 -> 13.5,
+// 4096 x 4096 x 8192 2190 -> 2150 (128 TFLOP/s; 128-tiles in this form 2045),
+// 60000 x 2304 x 64 289 -> 270.  The tiles in an order that gives each XCD
+// neighbouring ones: within 2 % either way.
 // ---------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kMK = 64;         // k per LDS stage
-constexpr int kBLd = kMK + 4;   // row stride of Bs: conflict-free 16-byte reads
 
 // The MFMA kernel takes products with at least this many C entries per
 // launch (2^18 = 512 x 512; smaller ones are latency-bound and the 64 x 64
 // VALU tiles spread them over more CUs) when its alignment conditions hold.
-#ifndef OMX_SGEMM_MFMA_T64
-#define OMX_SGEMM_MFMA_T64 1024
-#endif
 #ifndef OMX_SGEMM_MFMA_MIN
 #define OMX_SGEMM_MFMA_MIN (int64_t{1} << 18)
 #endif
@@ -126,153 +137,163 @@ __host__ __device__ __forceinline__ bool mfma_size(int64_t m, int64_t n, int64_t
     return m * n * batch >= OMX_SGEMM_MFMA_MIN;
 }
 
-template <int kT, bool kOneStage>
+constexpr int kT = 64;          // tile edge
+constexpr int kMG = 64;         // k per group
+constexpr int kQ = 32;          // a stage's k in each half of a group
+constexpr int kBLd = 2 * kQ + 4;  // row stride of Bs: conflict-free 16-byte reads
+
 __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, float alpha,
                                            const float *__restrict__ A, int64_t lda, const float *__restrict__ B,
                                            int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
                                            int64_t k0 = 0) {
-    constexpr int kB = kT / 64;       // MFMA blocks per quadrant side
-    constexpr int kS = kT / 16;       // float4 loads per thread per operand and stage
-    constexpr int kAK = 1024 / kT;    // stage columns between a thread's A loads
-    __shared__ float As[kMK][kT];     // As[k][i] = A(i0 + i, k0 + k)
-    __shared__ float Bs[kT][kBLd];    // Bs[j][k] = B(k0 + k, j0 + j)
+    constexpr int kS = kT * kQ / 512;  // float4 loads per thread per operand and stage
+    constexpr int kAK = 1024 / kT;     // stage columns between a thread's A loads
+    constexpr int kBJ = 512 / kQ;      // columns between a thread's B loads
+    __shared__ float As[2 * kQ][kT];   // As[q][i], As[kQ + q][i] = A(i0 + i, p0 + q), A(i0 + i, p1 + q)
+    __shared__ float Bs[kT][kBLd];     // Bs[j][q], Bs[j][kQ + q] = B(p0 + q, j0 + j), B(p1 + q, j0 + j)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, h = lane >> 5;
     const int64_t i0 = (int64_t)blockIdx.x * kT, j0 = (int64_t)blockIdx.y * kT;
     const int wi = (wave & 1) * (kT / 2), wj = (wave >> 1) * (kT / 2);
     // global -> LDS: A rows ar .. ar+3 at stage columns ak + kAK s; B column
-    // bj + 16 s, stage rows bk .. bk+3.  Rows (columns) past M (N) are
-    // clamped: their products land only in results that are not stored.
+    // bj + kBJ s, stage rows bk .. bk+3 of half bh.  Rows (columns) past M
+    // (N) are clamped: their products land only in results that are not
+    // stored.
     const int ar = 4 * (tid % (kT / 4)), ak = tid / (kT / 4);
-    const int bk = 4 * (tid & 15), bj = tid >> 4;
+    const int bk = 4 * (tid % (kQ / 4)), bh = tid / (kQ / 4) & 1, bj = tid / (kQ / 2);
     const int64_t arow = i0 + ar;
-    const bool afull = arow + 3 < M;
-    int64_t ar1 = arow + 1, ar2 = arow + 2, ar3 = arow + 3;
-    const int64_t arow0 = arow < M ? arow : M - 1;
-    if (ar1 >= M) ar1 = M - 1;
-    if (ar2 >= M) ar2 = M - 1;
-    if (ar3 >= M) ar3 = M - 1;
     const float *Bcol[kS];
 #pragma unroll
-    for (int s = 0; s < kS; ++s) {
-        int64_t j = j0 + bj + 16 * s;
-        if (j >= N) j = N - 1;
-        Bcol[s] = B + j * ldb;
-    }
+    for (int s = 0; s < kS; ++s) Bcol[s] = B + min(j0 + bj + kBJ * s, N - 1) * ldb;
     f32x4 ra[kS], rb[kS];
-    // stage k0 .. k0 + kc into ra / rb.  Every load is unconditional: stage
-    // columns (rows) at or past kc read column (row) kc - 1 (kc - 4) instead,
-    // and are not stored to LDS.
-#define OMX_SGEMM_GLOAD(k0, kc)                                                                            \
-    {                                                                                                      \
-        _Pragma("unroll") for (int s = 0; s < kS; ++s) {                                                   \
-            const int kk = ak + kAK * s < (kc) ? ak + kAK * s : (kc) - 1;                                  \
-            const float *p = A + ((k0) + kk) * lda;                                                        \
-            ra[s] = afull ? *reinterpret_cast<const f32x4 *>(p + arow)                                    \
-                          : f32x4{p[arow0], p[ar1], p[ar2], p[ar3]};                                 \
-        }                                                                                                  \
-        const int kb4 = bk < (kc) ? bk : (kc) - 4;                                                         \
-        _Pragma("unroll") for (int s = 0; s < kS; ++s)                                                     \
-            rb[s] = *reinterpret_cast<const f32x4 *>(Bcol[s] + (k0) + kb4);                               \
-    }
-    f32x16 acc[kB][kB];
+    f32x16 acc;
 #pragma unroll
-    for (int a = 0; a < kB; ++a)
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    // the products of a stage's first hc columns of each half
+    auto products = [&](int hc) {
+        for (int s = 0; s < hc; s += 4) {
+            const f32x4 y = *reinterpret_cast<const f32x4 *>(&Bs[wj + l32][kQ * h + s]);
 #pragma unroll
-        for (int b = 0; b < kB; ++b)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
-    int kc = (int)(K - k0 < kMK ? K - k0 : kMK);
-    OMX_SGEMM_GLOAD(k0, kc);
-    // kOneStage (K <= 64): C of the wave's quadrant is read now, with the
-    // operands, so that its latency overlaps theirs and the MFMAs (rows /
-    // columns past the edge read a clamped entry and are not stored);
-    // cv[a][b][v] sits where acc[a][b][v] does (see below).  With several
-    // stages the staging registers are live through the loop and C is read
-    // in the epilogue.
-    float cv[kB][kB][16];
-    if (kOneStage && beta != 0.0f) {
-#pragma unroll
-        for (int a = 0; a < kB; ++a) {
-            int64_t i = i0 + wi + 32 * a + l32;
-            if (i >= M) i = M - 1;
-#pragma unroll
-            for (int b = 0; b < kB; ++b)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    int64_t j = j0 + wj + 32 * b + 4 * h + 8 * (v >> 2) + (v & 3);
-                    if (j >= N) j = N - 1;
-                    cv[a][b][v] = C[i + j * ldc];
-                }
+            for (int u = 0; u < 4; ++u)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[u], As[kQ * h + s + u][wi + l32], acc, 0, 0, 0);
         }
-    }
-    for (;;) {
+    };
+    // acc[v] and cv[v]: row i, column j + 8 (v / 4) + v % 4.  C's columns are
+    // walked by one pointer, opaque to the compiler, which otherwise forms all
+    // the addresses beforehand; a column past N repeats the one before it.
+    const int64_t i = i0 + wi + l32, j = j0 + wj + 4 * h;
+    const int ncols = (int)max(min(N - j, (int64_t)kT), (int64_t)0);
+    float cv[16];
+    auto load_c = [&] {
+        if (beta == 0.0f) return;
+        const float *c = C + min(i, M - 1) + min(j, N - 1) * ldc;
 #pragma unroll
-        for (int s = 0; s < kS; ++s)
-            if (ak + kAK * s < kc) *reinterpret_cast<f32x4 *>(&As[ak + kAK * s][ar]) = ra[s];
-        if (bk < kc) {
-#pragma unroll
-            for (int s = 0; s < kS; ++s) *reinterpret_cast<f32x4 *>(&Bs[bj + 16 * s][bk]) = rb[s];
+        for (int v = 0; v < 16; ++v) {
+            cv[v] = *c;
+            const int step = v % 4 < 3 ? 1 : 5;
+            c += 8 * (v >> 2) + (v & 3) + step < ncols ? step * ldc : 0;
+            asm volatile("" : "+v"(c));
         }
+    };
+    if (K - k0 >= kMG && (K - k0) % kMG == 0 && (M % 4 == 0 || i0 + kT <= M)) {
+        // whole groups and whole float4s: pointers that step, no bounds
+        const float *Ap = A + min(arow, M - 4) + (k0 + ak) * lda;
+#pragma unroll
+        for (int s = 0; s < kS; ++s) Bcol[s] += k0 + bk + kMG / 2 * bh;
+        int t = 0;
+        auto load = [&] {
+#pragma unroll
+            for (int s = 0; s < kS; ++s)
+                ra[s] = *reinterpret_cast<const f32x4 *>(
+                    Ap + (kAK * s < kQ ? kAK * s : kMG / 2 + kAK * s - kQ) * lda);
+#pragma unroll
+            for (int s = 0; s < kS; ++s) rb[s] = *reinterpret_cast<const f32x4 *>(Bcol[s]);
+            t += kQ;
+            const int step = t < kMG / 2 ? kQ : kMG / 2 + kQ;
+            if (t == kMG / 2) t = 0;
+            Ap += step * lda;
+#pragma unroll
+            for (int s = 0; s < kS; ++s) Bcol[s] += step;
+        };
+        auto put = [&] {
+#pragma unroll
+            for (int s = 0; s < kS; ++s) *reinterpret_cast<f32x4 *>(&As[ak + kAK * s][ar]) = ra[s];
+#pragma unroll
+            for (int s = 0; s < kS; ++s) *reinterpret_cast<f32x4 *>(&Bs[bj + kBJ * s][kQ * bh + bk]) = rb[s];
+        };
+        load();
+        for (int64_t left = (K - k0) / (2 * kQ); left > 1; --left) {
+            put();
+            __syncthreads();
+            load();
+            products(kQ);
+            __syncthreads();
+        }
+        put();
         __syncthreads();
-        const int64_t kn = k0 + kc;
-        const int kcn = (!kOneStage && kn < K) ? (int)(K - kn < kMK ? K - kn : kMK) : 0;
-        if (kcn) OMX_SGEMM_GLOAD(kn, kcn);
-        const int half = kc >> 1, kb = h * half;
-        for (int s = 0; s < half; s += 4) {
-            f32x4 y[kB];
+        load_c();   // its latency passes behind the last stage's products
+        products(kQ);
+    } else {
+        int half = (int)min(K - k0, (int64_t)kMG) >> 1, t = 0;
+        int hh = min(half, kQ);
+        // columns p0 .. p0 + hh and p1 .. p1 + hh into ra / rb.  Every load
+        // is unconditional: what lies past hh reads the last column (rows)
+        // before it instead and is not stored to LDS.
+        auto load = [&](int64_t p0, int64_t p1) {
 #pragma unroll
-            for (int b = 0; b < kB; ++b) y[b] = *reinterpret_cast<const f32x4 *>(&Bs[wj + 32 * b + l32][kb + s]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                float x[kB];
-#pragma unroll
-                for (int a = 0; a < kB; ++a) x[a] = As[kb + s + u][wi + 32 * a + l32];
-#pragma unroll
-                for (int a = 0; a < kB; ++a)
-#pragma unroll
-                    for (int b = 0; b < kB; ++b)
-                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[b][u], x[a], acc[a][b], 0, 0, 0);
+            for (int s = 0; s < kS; ++s) {
+                const int q = min((ak + kAK * s) % kQ, hh - 1);
+                const float *p = A + ((kAK * s < kQ ? p0 : p1) + q) * lda;
+                ra[s] = arow + 3 < M ? *reinterpret_cast<const f32x4 *>(p + arow)
+                                     : f32x4{p[min(arow, M - 1)], p[min(arow + 1, M - 1)], p[min(arow + 2, M - 1)],
+                                             p[min(arow + 3, M - 1)]};
             }
+            const int64_t kb4 = (bh ? p1 : p0) + min(bk, hh - 4);
+#pragma unroll
+            for (int s = 0; s < kS; ++s) rb[s] = *reinterpret_cast<const f32x4 *>(Bcol[s] + kb4);
+        };
+        load(k0, k0 + half);
+        for (;;) {
+#pragma unroll
+            for (int s = 0; s < kS; ++s)
+                if ((ak + kAK * s) % kQ < hh) *reinterpret_cast<f32x4 *>(&As[ak + kAK * s][ar]) = ra[s];
+            if (bk < hh) {
+#pragma unroll
+                for (int s = 0; s < kS; ++s) *reinterpret_cast<f32x4 *>(&Bs[bj + kBJ * s][kQ * bh + bk]) = rb[s];
+            }
+            __syncthreads();
+            const int hc = hh;
+            t += kQ;
+            if (t >= half) {
+                k0 += 2 * half;
+                half = (int)min(K - k0, (int64_t)kMG) >> 1;
+                t = 0;
+            }
+            hh = min(half - t, kQ);
+            if (hh > 0) load(k0 + t, k0 + half + t);
+            products(hc);
+            if (hh <= 0) break;
+            __syncthreads();
         }
-        __syncthreads();
-        if (!kcn) break;
-        k0 = kn;
-        kc = kcn;
+        load_c();
     }
-#undef OMX_SGEMM_GLOAD
-    // acc[a][b][v]: row i0 + wi + 32 a + l32, column j0 + wj + 32 b + 8 (v / 4) + 4 h + v % 4
+    if (i >= M) return;
+    float *c = C + i + j * ldc;
 #pragma unroll
-    for (int a = 0; a < kB; ++a) {
-        const int64_t i = i0 + wi + 32 * a + l32;
-        if (i >= M) continue;
-#pragma unroll
-        for (int b = 0; b < kB; ++b) {
-            const int64_t jb = j0 + wj + 32 * b + 4 * h;
-            if (!kOneStage && beta != 0.0f) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int64_t j = jb + 8 * (v >> 2) + (v & 3);
-                    cv[a][b][v] = j < N ? C[i + j * ldc] : 0.0f;
-                }
-            }
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t j = jb + 8 * (v >> 2) + (v & 3);
-                if (j < N)
-                    C[i + j * ldc] = (beta == 0.0f) ? alpha * acc[a][b][v] : beta * cv[a][b][v] + alpha * acc[a][b][v];
-            }
-        }
+    for (int v = 0; v < 16; ++v) {
+        const float r = beta == 0.0f ? alpha * acc[v] : beta * cv[v] + alpha * acc[v];
+        if (8 * (v >> 2) + (v & 3) < ncols) *c = r;
+        c += (v % 4 < 3 ? 1 : 5) * ldc;
+        asm volatile("" : "+v"(c));
     }
 }
 
-template <int kT, bool kOneStage>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict__ A, int64_t lda,
              const float *__restrict__ B, int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
              int64_t sA, int64_t sB, int64_t sC) {
     const int64_t z = blockIdx.z;
-    sgemm_tile<kT, kOneStage>(M, N, K, alpha, A + z * sA, lda, B + z * sB, ldb, beta, C + z * sC, ldc);
+    sgemm_tile(M, N, K, alpha, A + z * sA, lda, B + z * sB, ldb, beta, C + z * sC, ldc);
 }
 
 // Two independent batches of products C_p = alpha A_p B_p in one launch
@@ -289,8 +310,7 @@ struct SgemmTwin {
     float *C;
 };
 
-template <int kT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 k_sgemm_twin(SgemmTwin g0, SgemmTwin g1, float alpha, int batch) {
     const bool second = (int)blockIdx.z >= batch;
     const SgemmTwin g = second ? g1 : g0;
@@ -299,7 +319,7 @@ k_sgemm_twin(SgemmTwin g0, SgemmTwin g1, float alpha, int batch) {
     if (i0 >= g.M || j0 >= g.N) return;
     const int64_t k0 = g.tri == 2 ? j0 : (g.tri == 3 ? i0 : 0);
     const int64_t k1 = g.tri == 1 ? j0 + kT : (g.tri == 4 ? i0 + kT : g.K);
-    sgemm_tile<kT, false>(g.M, g.N, k1 < g.K ? k1 : g.K, alpha, g.A + z * g.sA, g.lda, g.B + z * g.sB, g.ldb, 0.0f,
+    sgemm_tile(g.M, g.N, k1 < g.K ? k1 : g.K, alpha, g.A + z * g.sA, g.lda, g.B + z * g.sB, g.ldb, 0.0f,
                           g.C + z * g.sC, g.ldc, k0);
 }
 
@@ -1116,24 +1136,8 @@ bool use_mfma(int64_t m, int64_t n, int64_t k, int64_t batch, const float *A, in
 
 int sgemm_mfma(int64_t m, int64_t n, int64_t k, float alpha, const float *A, int64_t lda, int64_t sA, const float *B,
                int64_t ldb, int64_t sB, float beta, float *C, int64_t ldc, int64_t sC, int64_t batch, hipStream_t st) {
-    // 64-tiles where 128-tiles would give fewer than 1024 workgroups (four
-    // per CU): the inverse merges (few tiles, deep k) and the mid-size LU
-    // updates finish sooner on four times as many, smaller workgroups
-    const bool small = omx_cdiv(m, 128) * omx_cdiv(n, 128) * batch < OMX_SGEMM_MFMA_T64;
-    const int t = small ? 64 : 128;
-    const dim3 grid((unsigned)omx_cdiv(m, t), (unsigned)omx_cdiv(n, t), (unsigned)batch);
-    const bool one = k <= kMK;
-#define OMX_SGEMM_LAUNCH(T, ONE)                                                                              \
-    hipLaunchKernelGGL((k_sgemm_mfma<T, ONE>), grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, \
-                       ldc, sA, sB, sC)
-    if (small) {
-        if (one) OMX_SGEMM_LAUNCH(64, true);
-        else OMX_SGEMM_LAUNCH(64, false);
-    } else {
-        if (one) OMX_SGEMM_LAUNCH(128, true);
-        else OMX_SGEMM_LAUNCH(128, false);
-    }
-#undef OMX_SGEMM_LAUNCH
+    const dim3 grid((unsigned)omx_cdiv(m, kT), (unsigned)omx_cdiv(n, kT), (unsigned)batch);
+    hipLaunchKernelGGL(k_sgemm_mfma, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, sA, sB, sC);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
@@ -1171,16 +1175,11 @@ int sgemm_batched(int64_t m, int64_t n, int64_t k, float alpha, const float *A, 
     return OMX_OK;
 }
 
-// two batches of batch products each (k_sgemm_twin); tiles as sgemm_mfma
+// two batches of batch products each (k_sgemm_twin)
 int sgemm_twin(const SgemmTwin &g0, const SgemmTwin &g1, float alpha, int64_t batch, hipStream_t st) {
     const int64_t m = std::max(g0.M, g1.M), n = std::max(g0.N, g1.N);
-    const bool small = omx_cdiv(m, 128) * omx_cdiv(n, 128) * batch * 2 < OMX_SGEMM_MFMA_T64;
-    const int t = small ? 64 : 128;
-    const dim3 grid((unsigned)omx_cdiv(m, t), (unsigned)omx_cdiv(n, t), (unsigned)(2 * batch));
-    if (small)
-        hipLaunchKernelGGL(k_sgemm_twin<64>, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
-    else
-        hipLaunchKernelGGL(k_sgemm_twin<128>, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
+    const dim3 grid((unsigned)omx_cdiv(m, kT), (unsigned)omx_cdiv(n, kT), (unsigned)(2 * batch));
+    hipLaunchKernelGGL(k_sgemm_twin, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }

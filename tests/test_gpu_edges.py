@@ -256,3 +256,29 @@ def test_merged_launches_leave_the_factors_alone(n, b, alt, flags, prec):
     nb = n // b
     sched = [0, 1, -1, 2][:4] * nb if prec is None else [prec] * nb
     assert np.array_equal(_lu(n, b, alt, flags, sched[:nb]), _lu(n, b, alt, flags | 8, sched[:nb]))
+
+
+# FP32 product on the matrix cores: with whole groups of 64 in k and whole
+# float4s of rows (or none, in the last row tile) and without either; one,
+# two and many groups; last columns and rows of a tile; nothing else written
+@pytest.mark.parametrize("m,n,k,beta", [(1024, 257, 64, 1.0), (1023, 320, 128, 1.0), (513, 513, 192, 0.5),
+                                        (4097, 65, 256, 0.0), (516, 1027, 48, 1.0), (1025, 256, 80, 1.0),
+                                        (524288, 1, 64, 1.0), (2, 131072, 64, 1.0), (2048, 129, 1040, 0.0)])
+def test_sgemm_stage_and_tile_edges(m, n, k, beta):
+    torch = torch_cuda()
+    print(f"sgemm edges m={m} n={n} k={k} beta={beta}", flush=True)
+    L = _L()
+    rng = np.random.default_rng(m + n + k)
+    lda, ldb, ldc = (m + 3) // 4 * 4 + 4, k + 4, m + 3
+    A = rng.uniform(-1, 1, (k, lda)).astype(np.float32)
+    B = rng.uniform(-1, 1, (n, ldb)).astype(np.float32)
+    C = np.full((n + 1, ldc), 7.0, np.float32)
+    C[:n, :m] = rng.uniform(-1, 1, (n, m)) if beta else np.nan
+    Ad, Bd, Cd = dev(A.ravel()), dev(B.ravel()), dev(C.ravel())
+    assert L.omx_sgemm_f32(m, n, k, -1.0, ptr(Ad), lda, ptr(Bd), ldb, beta, ptr(Cd), ldc, None) == 0
+    out = host(Cd).reshape(n + 1, ldc)
+    assert np.all(out[n] == 7.0) and np.all(out[:n, m:] == 7.0)
+    A64, B64 = A[:, :m].astype(np.float64), B[:, :k].astype(np.float64)
+    c0 = beta * C[:n, :m].astype(np.float64) if beta else np.zeros((n, m))
+    bound = (k + 2) * 2.0 ** -24 * (np.abs(c0) + np.abs(B64) @ np.abs(A64))
+    assert np.all(np.abs(out[:n, :m] - (c0 - B64 @ A64)) <= bound)
