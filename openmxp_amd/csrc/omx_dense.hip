@@ -854,44 +854,68 @@ k_trsm_rows_rlnu64(int64_t m, const float *__restrict__ L, int64_t ldl, float *_
 // of Y) of w = 64, 128, 192 or 256 entries.  64 entries at a time are read,
 // lose their products with the lines' solved entries (each block of 64 summed
 // by itself and subtracted, in the order of the product that a launch of its
-// own would run: put_u), are solved (tri_solve64) and written; the solved
-// entries stay in LDS.  As launches of 64 entries each (solve, then a depth-64
-// product over the rest of the block) the lines went to memory and back four
-// times: 110 us a block for 30000 lines of 256, now 46; bound by the chain of
-// four solves and their operands' latency.
+// own would run: trsm_block_y), are solved (tri_solve64) and written; the
+// solved entries stay in LDS.  As launches of 64 entries each (solve, then a
+// depth-64 product over the rest of the block) the lines went to memory and
+// back four times: 110 us a block for 30000 lines of 256.  Bound by the chain
+// of four solves and their operands' latency, so what counts is how many
+// workgroups a CU holds: two, with 70 KB of LDS each - the triangle lies in
+// the piece's buffer that is free (the next one's, or the first's, whose
+// products are then done), and the factor's blocks between go from memory to
+// the registers of the lanes that multiply them.  RUNN blocks of 256 x 30000
+// lines 61 -> 44 us, 58880 115 -> 80 (LLNU 55 -> 40, 106 -> 74) against the form
+// with one workgroup a CU (100 KB); 16384 lines and below, where no CU has two,
+// 32 (28).
+constexpr int kXT = kNB + 4;
 struct __align__(16) TrsmShared {
-    float xs[kNB][kOB + 4];    // the lines: xs[line][entry]
-    float t[kNB][kNB + 1];     // the 64 x 64 triangle
-    float su[kNB][kUS];        // a block between: su[c][k] for entry c, solved entry k
+    float xs[kOB / kNB][kNB][kXT];  // the lines, a piece each: xs[piece][line][entry]
     float rd[kNB];
 };
 
-// the block for solved entries [64 i, +64) and entries [64 j, +64): element
-// (c, k) is U(64 i + k, 64 j + c) (kUp) or L(64 j + c, 64 i + k)
+// a lane's factor entries for solved entries [64 i, +64) and its entry c of
+// [64 j, +64): y[g][s] is U(64 i + k, 64 j + c) (kUp) or L(64 j + c, 64 i + k)
+// with k = 32 h + 4 g + s, or 8 g + 2 s + h (seq: sums in the order of k)
 template <bool kUp, bool kVec>
-__device__ __forceinline__ void trsm_block_get(const float *__restrict__ T, int64_t ldt, int i, int j, f32x4 (&v)[4]) {
-    // four consecutive k (kUp) or c of a column: 16 threads a column
-    const float *g = T + (kUp ? i : j) * kNB + 4 * (threadIdx.x & 15) +
-                     (int64_t)((kUp ? j : i) * kNB + (threadIdx.x >> 4)) * ldt;
+__device__ __forceinline__ void trsm_block_y(const float *__restrict__ T, int64_t ldt, int i, int j, int c, int h,
+                                             bool seq, f32x4 (&y)[8]) {
+    if constexpr (kUp) {
+        const float *p = T + i * kNB + (int64_t)(j * kNB + c) * ldt;
+        if (kVec) {  // always the first form: trsm_block_order makes the second of it
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float *p = g + (int64_t)(16 * q) * ldt;
-        v[q] = kVec ? *reinterpret_cast<const f32x4 *>(p) : f32x4{p[0], p[1], p[2], p[3]};
+            for (int g = 0; g < 8; ++g) y[g] = *reinterpret_cast<const f32x4 *>(p + 32 * h + 4 * g);
+        } else {
+#pragma unroll
+            for (int g = 0; g < 8; ++g)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) y[g][s] = p[8 * g + 2 * s + h];
+        }
+    } else {
+        const float *p = T + j * kNB + c + (int64_t)(i * kNB + (seq ? h : 32 * h)) * ldt;
+        const int64_t step = (seq ? 2 : 1) * ldt;
+#pragma unroll
+        for (int g = 0; g < 8; ++g)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) y[g][s] = p[(4 * g + s) * step];
     }
 }
 
-template <bool kUp>
-__device__ __forceinline__ void trsm_block_put(const f32x4 (&v)[4], float (*su)[kUS], bool seq) {
-    const int a = 4 * (threadIdx.x & 15);
+// y's k = 32 h + 4 g + s to k = 8 g + 2 s + h: of an even and the following odd
+// k the two halves of the wave trade places (at the use, not at the load,
+// where it would wait for it)
+__device__ __forceinline__ void trsm_block_order(f32x4 (&y)[8]) {
+    f32x4 o[8];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int b = (threadIdx.x >> 4) + 16 * q;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = kUp ? b : a + e, k = kUp ? a + e : b;
-            su[c][seq ? (k & 1) * 32 + (k >> 1) : k] = v[q][e];
-        }
+    for (int p = 0; p < 16; ++p) {
+        // (through scalars: __builtin_bit_cast of a vector's element takes its first)
+        const float a = y[p / 2][2 * p % 4], b = y[p / 2][2 * p % 4 + 1];
+        const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                        false, false);
+        const unsigned lo = r[0], hi = r[1];
+        o[p / 4][p % 4] = __builtin_bit_cast(float, lo);
+        o[p / 4 + 4][p % 4] = __builtin_bit_cast(float, hi);
     }
+#pragma unroll
+    for (int g = 0; g < 8; ++g) y[g] = o[g];
 }
 
 template <bool kUp, bool kVec>
@@ -902,6 +926,14 @@ k_trsm_block(int64_t lines, int w, const float *__restrict__ T, int64_t ldt, flo
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t e0 = (int64_t)blockIdx.x * kNB;
     const int nb = w / kNB;
+    // 32 lines x 32 entries a wave
+    const int wl = 32 * (wave & 1), wc = 32 * (wave >> 1);
+    // the update's order of sums: that of the product over the rest of the
+    // block that followed solved piece i
+    auto in_order = [&](int i) {
+        const int64_t inner = w - kNB * (i + 1);
+        return !kVec || !mfma_size(kUp ? lines : inner, kUp ? inner : lines, 1);
+    };
     // a thread's 16 values of a 64 x 64 piece: memory rows along the lanes;
     // lines past the end are read as the last one and not stored
     const int64_t le = min(e0 + lane, lines - 1) - e0;
@@ -910,78 +942,75 @@ k_trsm_block(int64_t lines, int w, const float *__restrict__ T, int64_t ldt, flo
                    : X + kNB * j + lane + min(e0 + 16 * wave + q, lines - 1) * ldx;
     };
     float v[16];
+    f32x4 y[8];
 #pragma unroll
     for (int q = 0; q < 16; ++q) v[q] = *addr(0, q);
 #pragma unroll 1
     for (int j = 0; j < nb; ++j) {
-        // the update's order of sums: the product over the rest of the block
-        // that followed solved block i
-        f32x4 u[4];
-        if (j > 0) trsm_block_get<kUp, kVec>(T, ldt, 0, j, u);
-        lds_barrier();  // (the last piece's triangle and lines are read)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int line = kUp ? lane : 16 * wave + q, c = kUp ? 16 * wave + q : lane;
-            sh.xs[line][kNB * j + c] = v[q];
+            sh.xs[j][line][c] = v[q];
         }
-        {
-            const float *tj = T + (kNB * j + lane) + (int64_t)(kNB * j + 16 * wave) * ldt;
-            float d[16];
+        const float *tj = T + (kNB * j + lane) + (int64_t)(kNB * j + 16 * wave) * ldt;
+        float d[16];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) d[q] = tj[(int64_t)q * ldt];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) sh.t[lane][16 * wave + q] = d[q];
-        }
+        for (int q = 0; q < 16; ++q) d[q] = tj[(int64_t)q * ldt];
         if (j + 1 < nb) {  // the next piece, in flight during this one
 #pragma unroll
             for (int q = 0; q < 16; ++q) v[q] = *addr(j + 1, q);
         }
-        // 32 lines x 32 entries a wave
-        const int wl = 32 * (wave & 1), wc = 32 * (wave >> 1);
+        if (j > 0) lds_barrier();
 #pragma unroll 1
         for (int i = 0; i < j; ++i) {
-            const int64_t inner = w - kNB * (i + 1);
-            const bool seq = !kVec || !mfma_size(kUp ? lines : inner, kUp ? inner : lines, 1);
-            trsm_block_put<kUp>(u, sh.su, seq);
-            lds_barrier();
-            if (i + 1 < j) trsm_block_get<kUp, kVec>(T, ldt, i + 1, j, u);
-            const float *x = &sh.xs[wl + l32][kNB * i + (seq ? h : 32 * h)];
+            const bool seq = in_order(i);
+            const float *x = &sh.xs[i][wl + l32][seq ? h : 32 * h];
+            f32x4 yn[8];
+            if (i + 1 < j) trsm_block_y<kUp, kVec>(T, ldt, i + 1, j, wc + l32, h, in_order(i + 1), yn);
+            if (kUp && kVec && seq) trsm_block_order(y);
             f32x16 acc;
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
 #pragma unroll
             for (int g = 0; g < 8; ++g) {
-                const f32x4 y = *reinterpret_cast<const f32x4 *>(&sh.su[wc + l32][32 * h + 4 * g]);
                 f32x4 xv;
                 if (seq)
                     xv = f32x4{x[8 * g], x[8 * g + 2], x[8 * g + 4], x[8 * g + 6]};
                 else
                     xv = *reinterpret_cast<const f32x4 *>(x + 4 * g);
 #pragma unroll
-                for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[s], xv[s], acc, 0, 0, 0);
+                for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[g][s], xv[s], acc, 0, 0, 0);
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                f32x4 *d = reinterpret_cast<f32x4 *>(&sh.xs[wl + l32][kNB * j + wc + 8 * r + 4 * h]);
-                f32x4 o = *d;
+                f32x4 *o = reinterpret_cast<f32x4 *>(&sh.xs[j][wl + l32][wc + 8 * r + 4 * h]);
+                f32x4 n = *o;
 #pragma unroll
-                for (int s = 0; s < 4; ++s) o[s] -= acc[4 * r + s];
-                *d = o;
+                for (int s = 0; s < 4; ++s) n[s] -= acc[4 * r + s];
+                *o = n;
             }
-            lds_barrier();
+#pragma unroll
+            for (int g = 0; g < 8; ++g) y[g] = yn[g];
         }
+        // the triangle over the next piece's buffer, or the first's: neither
+        // is read by now (the last solve is past a barrier, and so, below, are
+        // the products)
+        if (j > 0) lds_barrier();
+        float (*t)[kNB + 1] = reinterpret_cast<float (*)[kNB + 1]>(&sh.xs[(j + 1) % (kOB / kNB)][0][0]);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            t[lane][16 * wave + q] = d[q];
+            if (kUp && lane == 16 * wave + q) sh.rd[lane] = 1.0f / d[q];
+        }
+        // (the next piece's first factor block, in flight during the solve)
+        if (j + 1 < nb) trsm_block_y<kUp, kVec>(T, ldt, 0, j + 1, wc + l32, h, in_order(0), y);
         lds_barrier();
-        if (kUp) {
-            if (tid < kNB) sh.rd[tid] = 1.0f / sh.t[tid][tid];
-            lds_barrier();
-        }
-        float (*lines16)[kOB + 4] = reinterpret_cast<float (*)[kOB + 4]>(&sh.xs[16 * wave][kNB * j]);
-        tri_solve64<kUp, kOB + 4>(lines16, sh.t, sh.rd);
+        tri_solve64<kUp, kXT>(&sh.xs[j][16 * wave], t, sh.rd);
         lds_barrier();
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int line = kUp ? lane : 16 * wave + q, c = kUp ? 16 * wave + q : lane;
-            if (e0 + line < lines) *addr(j, q) = sh.xs[line][kNB * j + c];
+            if (e0 + line < lines) *addr(j, q) = sh.xs[j][line][c];
         }
     }
 }
