@@ -24,12 +24,16 @@ constexpr int kGemvTargetWG = 16384;
 constexpr int kGemvMaxSeg = 64;
 
 // Number of column segments of the residual GEMV for order n: enough
-// workgroups to fill the 256 CUs several times, each segment >= 256 columns.
+// workgroups to fill the 256 CUs several times, each segment >= 64 columns
+// (the jump to a segment's first column costs about as much as 30 columns'
+// steps).  At n = 1024 segments of 256 columns left 15 of 16 SIMDs without a
+// wave, and the columns of the diagonal, a load and a step at a time,
+// took longer than all others: 22.4 us, 10.6 now; 5120 29.0 -> 20, 10240 48 -> 39.
 int gemv_segments(int64_t n) {
     const int64_t nrb = omx_cdiv(n, kGemvRows);
     int64_t s = omx_cdiv(kGemvTargetWG, nrb);
     if (s > kGemvMaxSeg) s = kGemvMaxSeg;
-    const int64_t smax = omx_cdiv(n, 256);
+    const int64_t smax = omx_cdiv(n, 64);
     if (s > smax) s = smax;
     if (s < 1) s = 1;
     return (int)s;
@@ -53,24 +57,32 @@ __device__ __forceinline__ double otf_int(uint64_t t) {
 // at half the rate, and an FMA.  Four columns per trip with a 32-bit trip
 // count: the loop test is scalar, the state copies amortised.
 // n = 40960, with the copy and the norm of a refinement step: 468 us with
-// converted and scaled entries, 394 now (and a rounding less per entry).
+// converted and scaled entries, 379 now (and a rounding less per entry).
+// kDiag: column j0 + skip (the row's diagonal, where it is one of these) is
+// left out.
+template <bool kDiag>
 __device__ __forceinline__ void otf_columns(uint64_t &t, double &acc, omx_map jn, const double *__restrict__ x,
-                                            int64_t j0, int64_t j1) {
+                                            int64_t j0, int64_t j1, int skip = -1) {
     const double *__restrict__ xp = x + j0;
     const int cnt = (int)(j1 - j0);
+    auto add = [&](int c, uint64_t tc, double xc) {
+        const double sum = __builtin_fma(otf_int(tc), xc, acc);
+        acc = kDiag && c == skip ? acc : sum;
+    };
     int c = 0;
     for (; c + 4 <= cnt; c += 4) {
         const uint64_t t1 = omx_apply(jn, t);
         const uint64_t t2 = omx_apply(jn, t1);
         const uint64_t t3 = omx_apply(jn, t2);
-        acc = __builtin_fma(otf_int(t), xp[c], acc);
-        acc = __builtin_fma(otf_int(t1), xp[c + 1], acc);
-        acc = __builtin_fma(otf_int(t2), xp[c + 2], acc);
-        acc = __builtin_fma(otf_int(t3), xp[c + 3], acc);
+        const double x0 = xp[c], x1 = xp[c + 1], x2 = xp[c + 2], x3 = xp[c + 3];
+        add(c, t, x0);
+        add(c + 1, t1, x1);
+        add(c + 2, t2, x2);
+        add(c + 3, t3, x3);
         t = omx_apply(jn, t3);
     }
     for (; c < cnt; ++c) {
-        acc = __builtin_fma(otf_int(t), xp[c], acc);
+        add(c, t, xp[c]);
         t = omx_apply(jn, t);
     }
 }
@@ -98,14 +110,9 @@ k_otf_gemv(int64_t n, uint64_t x00, omx_map jn, const double *__restrict__ diag,
     // c0 <= lo <= hi <= c1
     const int64_t lo = c0 > d0 ? c0 : (d0 < c1 ? d0 : c1);
     const int64_t hi = c1 < d1 ? (c1 > lo ? c1 : lo) : (d1 > lo ? d1 : lo);
-    otf_columns(t, acc, jn, x, c0, lo);
-    for (int64_t j = lo; j < hi; ++j) {
-        const double xj = x[j];
-        const double sum = __builtin_fma(otf_int(t), xj, acc);
-        acc = j == i ? acc : sum;
-        t = omx_apply(jn, t);
-    }
-    otf_columns(t, acc, jn, x, hi, c1);
+    otf_columns<false>(t, acc, jn, x, c0, lo);
+    otf_columns<true>(t, acc, jn, x, lo, hi, (int)(i - lo));
+    otf_columns<false>(t, acc, jn, x, hi, c1);
     acc *= 0x1.fffffffffffffp-65;  // RandStat's scale (omx_lcg_value)
     if (i >= lo && i < hi) acc = __builtin_fma(diag[i], x[i], acc);
     if (part)
@@ -118,8 +125,17 @@ __global__ void k_gemv_reduce(int64_t n, int nseg, const double *__restrict__ pa
                               double *__restrict__ y, double alpha) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    // eight loads in flight: one after the other 64 segments took 12 us
     double s = part[i];
-    for (int q = 1; q < nseg; ++q) s += part[(int64_t)q * n + i];
+    int q = 1;
+    for (; q + 8 <= nseg; q += 8) {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = part[(int64_t)(q + e) * n + i];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += v[e];
+    }
+    for (; q < nseg; ++q) s += part[(int64_t)q * n + i];
     y[i] = y[i] + alpha * s;
 }
 

@@ -282,3 +282,21 @@ def test_sgemm_stage_and_tile_edges(m, n, k, beta):
     c0 = beta * C[:n, :m].astype(np.float64) if beta else np.zeros((n, m))
     bound = (k + 2) * 2.0 ** -24 * (np.abs(c0) + np.abs(B64) @ np.abs(A64))
     assert np.all(np.abs(out[:n, :m] - (c0 - B64 @ A64)) <= bound)
+
+
+# residual GEMV at the edges of its row blocks (256), column segments (64 and
+# up, 4 columns a trip) and of the segments that hold a row block's diagonal
+@pytest.mark.parametrize("n", [1, 63, 65, 129, 255, 257, 515, 1151, 4097, 4161])
+def test_otf_gemv_segment_edges(orc, n):
+    torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    d, x, y0 = rng.uniform(n, 2 * n, n), rng.standard_normal(n), rng.standard_normal(n)
+    wb = L.omx_otf_gemv_workspace_bytes(n)
+    D, X, Y, W = dev(d), dev(x), dev(y0), dev(np.full(wb // 8 + 8, np.nan))
+    assert L.omx_otf_gemv_f64(n, 42, ptr(D), -1.0, ptr(X), ptr(Y), ptr(W), wb, None) == 0
+    assert np.all(np.isnan(host(W)[wb // 8:]))
+    ref = orc.otf_gemv(n, 42, d, -1.0, x, y0)
+    # both sides: n rounded additions of terms of at most |x| / 2, and d x
+    bound = (2 * n + 8) * 2.0 ** -53 * (np.abs(y0) + d * np.abs(x) + 0.5 * np.abs(x).sum())
+    assert np.all(np.abs(host(Y) - ref) <= bound)
