@@ -1369,8 +1369,10 @@ int omx_trtri_lu_f32(int64_t n, const float *D, int64_t ldd, float *Xu, float *X
                 continue;
             }
             const int64_t dstep = stride * (ldd + 1), xstep = stride * (ldx + 1), wstep = stride * (n + 1);
-            if (vec && mfma_size(s1, s2, cnt) && 2 * cnt <= 65535) {
-                // both sides' inner products, then both results
+            if (vec && 2 * cnt <= 65535) {
+                // both sides' inner products, then both results, on the matrix
+                // cores however few the tiles: the 512 + 256 of n = 768 took
+                // 190 us as four products of 64 x 64 VALU tiles, now 35
                 const SgemmTwin wu{s1, s2, s2, ldd, ldx, n, dstep, xstep, wstep, 1, D + a0 + a1 * ldd,
                                    Xu + a1 + a1 * ldx, work + a0 + a1 * n};
                 const SgemmTwin wl{s2, s1, s1, ldd, ldx, n, dstep, xstep, wstep, 2, D + a1 + a0 * ldd,
