@@ -72,17 +72,20 @@ struct PackJob {
     int mask, headroom;
 };
 
+// (kJobs = 1: a panel by itself starts without the look-up, 0.4 us sooner)
+template <int kJobs>
 struct PackJobs {
-    PackJob job[kPackJobs];
-    int64_t end[kPackJobs];   // strips of the jobs up to and with this one
+    PackJob job[kJobs];
+    int64_t end[kJobs];       // strips of the jobs up to and with this one
 };
 
 // the workgroup's job and row strip
-__device__ __forceinline__ const PackJob &pack_job(const PackJobs &p, int64_t &strip) {
+template <int kJobs>
+__device__ __forceinline__ const PackJob &pack_job(const PackJobs<kJobs> &p, int64_t &strip) {
     int q = 0;
     int64_t first = 0;
 #pragma unroll
-    for (int i = 0; i + 1 < kPackJobs; ++i) {
+    for (int i = 0; i + 1 < kJobs; ++i) {
         if ((int64_t)blockIdx.y >= p.end[i]) {
             q = i + 1;
             first = p.end[i];
@@ -97,8 +100,9 @@ __device__ __forceinline__ const PackJob &pack_job(const PackJobs &p, int64_t &s
 // one row); all 64 of its source values are loaded, straight from the panel,
 // before the first is converted, so a workgroup's 64 KB arrive in one round
 // trip.
+template <int kJobs>
 __global__ void __launch_bounds__(kPackThreads)
-k_pack_f16(int64_t K, PackJobs jobs) {
+k_pack_f16(int64_t K, PackJobs<kJobs> jobs) {
     __shared__ float red[kPackThreads / 64];
     int64_t rsb;                     // row strip
     const PackJob j = pack_job(jobs, rsb);
@@ -224,8 +228,9 @@ __global__ void k_strip_exps16(int64_t nstrips, int64_t KT, const float *__restr
 // source values loaded straight from the panel first.  Every workgroup forms
 // its scale tile's exponent from the tile maximum; the tile's first one
 // stores it (a launch of its own before each pack took 8 us).
+template <int kJobs>
 __global__ void __launch_bounds__(kPackThreads)
-k_pack_f8(int64_t K, PackJobs jobs) {
+k_pack_f8(int64_t K, PackJobs<kJobs> jobs) {
     int64_t rsb;
     const PackJob j = pack_job(jobs, rsb);
     const int64_t k64 = blockIdx.x;  // 64-column block
@@ -272,11 +277,11 @@ bool pack_source_ok(const float *src, int64_t rows, int64_t k, int64_t rs, int64
     return !(ls == 1 && (rs % 4 || (reinterpret_cast<uintptr_t>(src) & 15)));
 }
 
-// one launch of k_pack_f16 / k_pack_f8 over count jobs of k columns
-int launch_pack(bool fp8, int64_t k, int count, const PackJob *job, hipStream_t st) {
-    PackJobs p{};
+template <int kJobs>
+int launch_pack_jobs(bool fp8, int64_t k, int count, const PackJob *job, hipStream_t st) {
+    PackJobs<kJobs> p{};
     int64_t strips = 0;
-    for (int i = 0; i < kPackJobs; ++i) {
+    for (int i = 0; i < kJobs; ++i) {
         if (i < count) {
             p.job[i] = job[i];
             strips += omx_strips(job[i].R);
@@ -285,11 +290,17 @@ int launch_pack(bool fp8, int64_t k, int count, const PackJob *job, hipStream_t 
     }
     const dim3 grid((unsigned)(k / kTileK), (unsigned)strips);
     if (fp8)
-        hipLaunchKernelGGL(k_pack_f8, grid, dim3(kPackThreads), 0, st, k, p);
+        hipLaunchKernelGGL(k_pack_f8<kJobs>, grid, dim3(kPackThreads), 0, st, k, p);
     else
-        hipLaunchKernelGGL(k_pack_f16, grid, dim3(kPackThreads), 0, st, k, p);
+        hipLaunchKernelGGL(k_pack_f16<kJobs>, grid, dim3(kPackThreads), 0, st, k, p);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
+}
+
+// one launch of k_pack_f16 / k_pack_f8 over count jobs of k columns
+int launch_pack(bool fp8, int64_t k, int count, const PackJob *job, hipStream_t st) {
+    return count == 1 ? launch_pack_jobs<1>(fp8, k, count, job, st)
+                      : launch_pack_jobs<kPackJobs>(fp8, k, count, job, st);
 }
 
 PackJob job_f16(int64_t rows, int64_t k, const float *src, int64_t rs, int64_t ls, int mask, void *P, int64_t ldk,
