@@ -100,12 +100,10 @@ __device__ __forceinline__ void gl_lds16(const char *g, char *l) {
 // C update of one wave's 128 x 128 block.  acc[mi][ni][r] is
 //   C(i0 + 32 mi + lane%32, j0 + 32 ni + 8 (r/4) + 4 (lane/32) + r%4),
 // so each lane owns 16 columns of one row per 32 x 32 block and every load or
-// store instruction covers 32 consecutive rows of two columns.  Interior
-// tiles go through buffer instructions, one resource per 32-column block
-// (wave-uniform 64-bit base in SGPRs, 16 per-lane 32-bit column offsets, the
-// row block in the immediate), pipelined over ni: the 64 old values of
-// column block ni + 1 are in flight while column block ni is combined and
-// stored.
+// store instruction covers 32 consecutive rows of two columns.  They are
+// buffer instructions, one resource per 32-column block (wave-uniform 64-bit base in SGPRs, 16 per-lane 32-bit column offsets, the
+// row block in the immediate), in units of two row blocks of one column block:
+// the next unit's 32 old values are in flight while one is combined and stored.
 // Cache policy of the C loads and stores (buffer aux operand): NT (bit 1),
 // non-temporal.  Each C element is read and written once per launch, while
 // the packed panels are re-read by many workgroups through L2; streaming C
@@ -113,10 +111,28 @@ __device__ __forceinline__ void gl_lds16(const char *g, char *l) {
 // 61440 x 61440 x 2560: 1404 -> 1548 TFLOP/s, FP16 unchanged).
 constexpr int kCPolicy = 2;
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t colblock_rsrc(float *p, int64_t ldc) {
-    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)(ldc * 32 * 4), 0x00020000);
+// That holds where a half-wave's 32 rows are one 128-byte line.  Where they lie
+// across two, each store writes parts of lines that a later one completes, and
+// without a cache between the parts go to memory by themselves: there C goes
+// through L2.  C -= X Y at 7936 x 12544 x 2560: FP16 605 -> 526 us (ldc 7937),
+// 531 -> 505 (ldc 7940); FP8 437 -> 325, 317 -> 304; on whole lines (ldc 7936)
+// without this 3 to 5 % slower in FP8.
+__device__ __forceinline__ bool whole_lines(const float *C, int64_t ldc) {
+    return ldc % 32 == 0 && (reinterpret_cast<uintptr_t>(C) & 127) == 0;
 }
 
+// p: the first of cols (at most 32) columns that exist; the hardware leaves
+// out accesses to those beyond
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t colblock_rsrc(float *p, int64_t ldc, int64_t cols = 32) {
+    const int n = cols < 0 ? 0 : (cols > 32 ? 32 : (int)cols);
+    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)(ldc * 4) * n, 0x00020000);
+}
+
+// Tiles cut by C's edge run the same way: rows are left out by the lanes,
+// columns by the resource's size.  (Checked one by one, 16 old values in flight
+// at a time, a cut tile held its launch up by 35 us: C -= X Y in FP16 / FP8 at
+// 1000 x 1000 x 256 53 -> 16 / 51 -> 15 us, 5001 x 5001 x 1024 159 -> 82 / 138 ->
+// 59.)
 // mx (beta = 0): max |value stored| by this lane, folded into what it holds.
 template <bool kBetaZero>
 __device__ __forceinline__ void epilogue(floatx16 (&acc)[4][4], int64_t M, int64_t N, float alpha,
@@ -124,25 +140,32 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[4][4], int64_t M, int64
                                          int tn, int wm, int wn, int lane, float &mx) {
     const int64_t i0 = (int64_t)tm * OMX_STRIP + wm * 128;
     const int64_t j0 = (int64_t)tn * OMX_STRIP + wn * 128;
-    if ((int64_t)(tm + 1) * OMX_STRIP <= M && (int64_t)(tn + 1) * OMX_STRIP <= N &&
-        ldc * 32 * 4 < ((int64_t)1 << 31)) {
+    // (opaque: the offsets below are not to be formed ahead of the branch that
+    // leads here, and spilled)
+    asm volatile("" : "+v"(lane));
+    if (ldc * 32 * 4 < ((int64_t)1 << 31)) {
+        // this lane's rows of the four row blocks that exist
+        const int rows = (int)min(max(M - i0 - (lane & 31) + 31, (int64_t)0) >> 5, (int64_t)4);
         int voff[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             voff[r] = (int)(((8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * ldc + (lane & 31)) * 4);
         if (kBetaZero) {
+            const int64_t cols = N - j0 - 4 * (lane >> 5);
 #pragma unroll
             for (int ni = 0; ni < 4; ++ni) {
-                const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc);
+                const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc, N - j0 - 32 * ni);
 #pragma unroll
-                for (int mi = 0; mi < 4; ++mi)
+                for (int mi = 0; mi < 4; ++mi) {
+                    if (mi >= rows) continue;
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const float v = alpha * acc[mi][ni][r];
-                        mx = fmaxf(mx, fabsf(v));
+                        if (8 * (r >> 2) + (r & 3) < cols - 32 * ni) mx = fmaxf(mx, fabsf(v));
                         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, voff[r] + mi * 128,
                                                               0, kCPolicy);
                     }
+                }
             }
             return;
         }
@@ -151,31 +174,35 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[4][4], int64_t M, int64
         float old[2][2][16];
         auto fetch = [&](float(&o)[2][16], int u) {
             const int ni = u >> 1, m0 = 2 * (u & 1);
-            const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc);
+            const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc, N - j0 - 32 * ni);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                if (m0 + h >= rows) continue;
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     o[h][r] = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff[r] + (m0 + h) * 128, 0, kCPolicy));
+                        float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff[r] + (m0 + h) * 128, 0, 0));
+            }
         };
         fetch(old[0], 0);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             if (u + 1 < 8) fetch(old[(u + 1) & 1], u + 1);
             const int ni = u >> 1, m0 = 2 * (u & 1);
-            const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc);
+            const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc, N - j0 - 32 * ni);
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h) {
+                if (m0 + h >= rows) continue;
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     __builtin_amdgcn_raw_buffer_store_b32(
                         __builtin_bit_cast(uint32_t, beta * old[u & 1][h][r] + alpha * acc[m0 + h][ni][r]), rs,
-                        voff[r] + (m0 + h) * 128, 0, kCPolicy);
+                        voff[r] + (m0 + h) * 128, 0, 0);
+            }
         }
         return;
     }
-    // edge tiles (and ldc too large for 32-bit column offsets): checked
+    // ldc too large for 32-bit column offsets: checked one by one
     const int64_t ib = i0 + (lane & 31);
     const int64_t jb = j0 + 4 * (lane >> 5);
 #pragma unroll
@@ -237,6 +264,7 @@ __device__ __forceinline__ void epilogue_lds(floatx16 (&acc)[4][4], float alpha,
                                              float *__restrict__ C, int64_t ldc, int64_t i0, int64_t j0,
                                              int lane, int wave, char *ring) {
     char *reg = ring + wave * 32768;
+    const bool lines = whole_lines(C, ldc);
     int voff[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r)
@@ -279,13 +307,19 @@ __device__ __forceinline__ void epilogue_lds(floatx16 (&acc)[4][4], float alpha,
                         l + (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * 512 + (32 * mi + (lane & 31)) * 4);
             if (ni + 2 < 4) refill(ni, h);
             const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc);
+            auto store = [&](auto policy) {
 #pragma unroll
-            for (int mi = 0; mi < 4; ++mi)
+                for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    __builtin_amdgcn_raw_buffer_store_b32(
-                        __builtin_bit_cast(uint32_t, beta * old[mi][r] + alpha * acc[mi][ni][r]), rs,
-                        voff[r] + mi * 128, 0, kCPolicy);
+                    for (int r = 0; r < 16; ++r)
+                        __builtin_amdgcn_raw_buffer_store_b32(
+                            __builtin_bit_cast(uint32_t, beta * old[mi][r] + alpha * acc[mi][ni][r]), rs,
+                            voff[r] + mi * 128, 0, decltype(policy)::value);
+            };
+            if (lines)
+                store(std::integral_constant<int, kCPolicy>{});
+            else
+                store(std::integral_constant<int, 0>{});
         } else {
             const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc);
 #pragma unroll
@@ -298,13 +332,19 @@ __device__ __forceinline__ void epilogue_lds(floatx16 (&acc)[4][4], float alpha,
                         old[q][r] = *reinterpret_cast<const float *>(
                             l + (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * 512 + (32 * (2 * half + q) + (lane & 31)) * 4);
                 if (half == 1 && ni + 2 < 4) refill(ni, h);
+                auto store = [&](auto policy) {
 #pragma unroll
-                for (int q = 0; q < 2; ++q)
+                    for (int q = 0; q < 2; ++q)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        __builtin_amdgcn_raw_buffer_store_b32(
-                            __builtin_bit_cast(uint32_t, beta * old[q][r] + alpha * acc[2 * half + q][ni][r]), rs,
-                            voff[r] + (2 * half + q) * 128, 0, kCPolicy);
+                        for (int r = 0; r < 16; ++r)
+                            __builtin_amdgcn_raw_buffer_store_b32(
+                                __builtin_bit_cast(uint32_t, beta * old[q][r] + alpha * acc[2 * half + q][ni][r]), rs,
+                                voff[r] + (2 * half + q) * 128, 0, decltype(policy)::value);
+                };
+                if (lines)
+                    store(std::integral_constant<int, kCPolicy>{});
+                else
+                    store(std::integral_constant<int, 0>{});
             }
         }
     }
@@ -816,7 +856,7 @@ __device__ __forceinline__ void epilogue_half(floatx16 (&acc)[4][2], int64_t M, 
         }
         return;
     }
-    // edge tiles (and ldc too large for 32-bit column offsets): checked
+    // ldc too large for 32-bit column offsets: checked one by one
     const int64_t ib = i0 + (lane & 31);
     const int64_t jb = j0 + 4 * (lane >> 5);
 #pragma unroll

@@ -300,3 +300,49 @@ def test_otf_gemv_segment_edges(orc, n):
     # both sides: n rounded additions of terms of at most |x| / 2, and d x
     bound = (2 * n + 8) * 2.0 ** -53 * (np.abs(y0) + d * np.abs(x) + 0.5 * np.abs(x).sum())
     assert np.all(np.abs(host(Y) - ref) <= bound)
+
+
+# FP16 and FP8 products whose last tiles are cut at any row and column, with C
+# on whole lines, on 16 bytes and on neither: the entries that exist are those
+# of the product of whole tiles, bit for bit, and no other is written
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("m,n", [(1, 1), (31, 300), (300, 33), (127, 129), (257, 256), (256, 480), (512, 511),
+                                 (481, 512), (385, 4)])
+def test_product_tiles_cut_anywhere(fp8, m, n):
+    torch = torch_cuda()
+    print(f"cut tiles fp8={fp8} m={m} n={n}", flush=True)
+    L = _L()
+    S, k = 512, 256
+    rng = np.random.default_rng(m * 1000 + n)
+    col, row = dev(rng.uniform(-1, 1, S * k).astype(np.float32)), dev(rng.uniform(-1, 1, S * k).astype(np.float32))
+    X, Y = (empty(L.omx_panel_bytes(S, k, int(fp8)), torch.uint8) for _ in range(2))
+    if fp8:
+        ne = L.omx_panel_exps_count(S, k)
+        Xe, Ye, tm = empty(ne, torch.int32), empty(ne, torch.int32), empty(ne, torch.float32)
+        assert L.omx_pack_f8(S, k, ptr(col), 1, S, ptr(X), ptr(Xe), ptr(tm), None) == 0
+        assert L.omx_pack_f8(S, k, ptr(row), k, 1, ptr(Y), ptr(Ye), ptr(tm), None) == 0
+    else:
+        assert L.omx_pack_f16(S, k, ptr(col), 1, S, 0, ptr(X), None, None) == 0
+        assert L.omx_pack_f16(S, k, ptr(row), k, 1, 0, ptr(Y), None, None) == 0
+    c0 = rng.uniform(-1, 1, (S, S)).astype(np.float32)  # c0[column][row]
+
+    def product(mm, nn, beta, ldc, skip):
+        buf = np.full(skip + (nn + 1) * ldc, 7.0, np.float32)
+        view = buf[skip:skip + nn * ldc].reshape(nn, ldc)
+        view[:, :mm] = c0[:nn, :mm] if beta else np.nan
+        B = dev(buf)
+        p = ptr(B) + 4 * skip
+        if fp8:
+            rc = L.omx_gemm_f8_packed(mm, nn, k, -1.0, ptr(X), ptr(Xe), 0, ptr(Y), ptr(Ye), 0, beta, p, ldc, None)
+        else:
+            rc = L.omx_gemm_f16_packed(mm, nn, k, -1.0, ptr(X), 0, ptr(Y), 0, beta, p, ldc, None)
+        assert rc == 0
+        out = host(B)
+        body = out[skip:skip + nn * ldc].reshape(nn, ldc)
+        assert np.all(out[:skip] == 7.0) and np.all(out[skip + nn * ldc:] == 7.0) and np.all(body[:, mm:] == 7.0)
+        return body[:, :mm]
+
+    for beta in (1.0, 0.0):
+        whole = product(S, S, beta, S, 0)
+        for ldc, skip in ((544, 0), (548, 0), (513, 0), (512, 1)):
+            assert np.array_equal(product(m, n, beta, ldc, skip), whole[:n, :m]), (beta, ldc, skip)
