@@ -96,13 +96,14 @@ k_sgemm_nn(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict
 
 // ---------------------------------------------------------------------------
 // The same product on the matrix cores (v_mfma_f32_32x32x2_f32), for the
-// large updates: a 64 x 64 tile per workgroup of four waves (a 32 x 32 MFMA
-// block each), k staged through LDS up to 64 at a time, the next stage's
+// large updates: a kT x kT tile (64, or 128: sgemm_mfma) per workgroup of four
+// waves (a kT/2 square quadrant each, made of 32 x 32 MFMA blocks), k in groups
+// of up to 64, staged through LDS kQ of each half at a time, the next stage's
 // global loads in flight during the current stage's MFMAs.  The MFMA's first
 // operand takes B (lane l: column l % 32), the second A (lane l: row l % 32),
 // so every accumulator register of lane l belongs to row l % 32 of its block
 // and a half-wave's C access is 32 consecutive rows of one column (one
-// 128-byte line).  In a stage of kc columns, lanes 0-31 carry k in [0, kc/2)
+// 128-byte line).  In a group of kc columns, lanes 0-31 carry k in [0, kc/2)
 // and lanes 32-63 k in [kc/2, kc); the MFMA adds the two halves.  Needs A and
 // B 16-byte aligned with lda and ldb multiples of 4, and k % 16 == 0 (so kc
 // is a multiple of 16).
@@ -111,17 +112,16 @@ k_sgemm_nn(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict
 // stood between was the time from a stage's loads to the next's.  A product
 // of whole groups of 64 and whole float4s of rows therefore steps pointers
 // and has no bounds in its loop: with the clamps the compiler put waits
-// between a stage's own loads, and a tile of four waves alone on its CU paid
-// for every address instruction.  Its last stage stands outside the loop, so
-// that C's old values are on their way during that stage's MFMAs.  Edge of 64
-// for every size: four workgroups a CU hide one another's loads and C better
-// than two of 128 x 128 did, whose operands are read half as often.  Measured
-// (128 x 128 or 64 x 64 tiles with bounds in the loop -> now), C -= A B:
-// 30000 x 2304 x 256 420 -> 355 us, 7680 x 7680 x 512 588 -> 523, 2048 x 2048 x
-// 512 47.5 -> 41.7, 30000 x 256 x 256 54.4 -> 46, 512 x 512 x 512 17.6 -> 13.5,
-// 4096 x 4096 x 8192 2190 -> 2150 (128 TFLOP/s; 128-tiles in this form 2045),
-// 60000 x 2304 x 64 289 -> 270.  The tiles in an order that gives each XCD
-// neighbouring ones: within 2 % either way.
+// between a stage's own loads, and four waves alone on their CU paid for
+// every address instruction.  Its last stage stands outside the loop, so that
+// C's old values (kT = 128: those of half its blocks, all spill)
+// are on their way during that stage's MFMAs.  A 128-tile's stages hold half a
+// group, so that three workgroups fit a CU instead of two.  Measured (bounds
+// in the loop, no XCD order -> now), C -= A B: 30000 x 2304 x 256 456 -> 379 us,
+// 2048 x 2048 x 512 47.5 -> 41.7, 30000 x 256 x 256 54.4 -> 46, 512 x 512 x 512
+// 17.6 -> 13.5, 60000 x 2304 x 64 289 -> 270, 4096 x 4096 x 8192 2200 -> 2060,
+// 61440 x 61440 x 2560 161 -> 141 ms (137 TFLOP/s), 20480 x 20480 x 10240 68.8 ->
+// 61.7.
 // ---------------------------------------------------------------------------
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -137,23 +137,24 @@ __host__ __device__ __forceinline__ bool mfma_size(int64_t m, int64_t n, int64_t
     return m * n * batch >= OMX_SGEMM_MFMA_MIN;
 }
 
-constexpr int kT = 64;          // tile edge
 constexpr int kMG = 64;         // k per group
-constexpr int kQ = 32;          // a stage's k in each half of a group
-constexpr int kBLd = 2 * kQ + 4;  // row stride of Bs: conflict-free 16-byte reads
 
+template <int kT>
 __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, float alpha,
                                            const float *__restrict__ A, int64_t lda, const float *__restrict__ B,
                                            int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
-                                           int64_t k0 = 0) {
-    constexpr int kS = kT * kQ / 512;  // float4 loads per thread per operand and stage
-    constexpr int kAK = 1024 / kT;     // stage columns between a thread's A loads
-    constexpr int kBJ = 512 / kQ;      // columns between a thread's B loads
-    __shared__ float As[2 * kQ][kT];   // As[q][i], As[kQ + q][i] = A(i0 + i, p0 + q), A(i0 + i, p1 + q)
-    __shared__ float Bs[kT][kBLd];     // Bs[j][q], Bs[j][kQ + q] = B(p0 + q, j0 + j), B(p1 + q, j0 + j)
+                                           int64_t ti, int64_t tj, int64_t k0 = 0) {
+    constexpr int kB = kT / 64;              // MFMA blocks per quadrant side
+    constexpr int kQ = kT == 64 ? 32 : 16;   // a stage's k in each half of a group
+    constexpr int kS = kT * kQ / 512;        // float4 loads per thread per operand and stage
+    constexpr int kAK = 1024 / kT;           // stage columns between a thread's A loads
+    constexpr int kBJ = 512 / kQ;            // columns between a thread's B loads
+    constexpr int kBLd = 2 * kQ + 4;         // row stride of Bs: conflict-free 16-byte reads
+    __shared__ float As[2 * kQ][kT];         // As[q][i], As[kQ + q][i] = A(i0 + i, p0 + q), A(i0 + i, p1 + q)
+    __shared__ float Bs[kT][kBLd];           // Bs[j][q], Bs[j][kQ + q] = B(p0 + q, j0 + j), B(p1 + q, j0 + j)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, h = lane >> 5;
-    const int64_t i0 = (int64_t)blockIdx.x * kT, j0 = (int64_t)blockIdx.y * kT;
+    const int64_t i0 = ti * kT, j0 = tj * kT;
     const int wi = (wave & 1) * (kT / 2), wj = (wave >> 1) * (kT / 2);
     // global -> LDS: A rows ar .. ar+3 at stage columns ak + kAK s; B column
     // bj + kBJ s, stage rows bk .. bk+3 of half bh.  Rows (columns) past M
@@ -166,33 +167,53 @@ __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, floa
 #pragma unroll
     for (int s = 0; s < kS; ++s) Bcol[s] = B + min(j0 + bj + kBJ * s, N - 1) * ldb;
     f32x4 ra[kS], rb[kS];
-    f32x16 acc;
+    f32x16 acc[kB][kB];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    for (int a = 0; a < kB; ++a)
+#pragma unroll
+        for (int b = 0; b < kB; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
     // the products of a stage's first hc columns of each half
     auto products = [&](int hc) {
         for (int s = 0; s < hc; s += 4) {
-            const f32x4 y = *reinterpret_cast<const f32x4 *>(&Bs[wj + l32][kQ * h + s]);
+            f32x4 y[kB];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[u], As[kQ * h + s + u][wi + l32], acc, 0, 0, 0);
+            for (int b = 0; b < kB; ++b) y[b] = *reinterpret_cast<const f32x4 *>(&Bs[wj + 32 * b + l32][kQ * h + s]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                float x[kB];
+#pragma unroll
+                for (int a = 0; a < kB; ++a) x[a] = As[kQ * h + s + u][wi + 32 * a + l32];
+#pragma unroll
+                for (int a = 0; a < kB; ++a)
+#pragma unroll
+                    for (int b = 0; b < kB; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[b][u], x[a], acc[a][b], 0, 0, 0);
+            }
         }
     };
-    // acc[v] and cv[v]: row i, column j + 8 (v / 4) + v % 4.  C's columns are
-    // walked by one pointer, opaque to the compiler, which otherwise forms all
-    // the addresses beforehand; a column past N repeats the one before it.
-    const int64_t i = i0 + wi + l32, j = j0 + wj + 4 * h;
-    const int ncols = (int)max(min(N - j, (int64_t)kT), (int64_t)0);
-    float cv[16];
-    auto load_c = [&] {
+    // acc[a][b][v] and cv[a][b][v]: row i0 + wi + 32 a + l32, column
+    // jb + 32 b + 8 (v / 4) + v % 4.  C's columns are walked by one pointer,
+    // opaque to the compiler (which otherwise forms all 64 addresses first
+    // and spills), and a column past N repeats the one before it.
+    float cv[kB][kB][16];
+    const int64_t jb = j0 + wj + 4 * h;
+    const int ncols = (int)max(min(N - jb, (int64_t)kT), (int64_t)0);
+    auto load_c = [&](int a0, int a1) {
         if (beta == 0.0f) return;
-        const float *c = C + min(i, M - 1) + min(j, N - 1) * ldc;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            cv[v] = *c;
-            const int step = v % 4 < 3 ? 1 : 5;
-            c += 8 * (v >> 2) + (v & 3) + step < ncols ? step * ldc : 0;
-            asm volatile("" : "+v"(c));
+        for (int a = a0; a < a1; ++a) {
+            const float *c = C + min(i0 + wi + 32 * a + l32, M - 1) + min(jb, N - 1) * ldc;
+#pragma unroll
+            for (int b = 0; b < kB; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    cv[a][b][v] = *c;
+                    const int step = v % 4 < 3 ? 1 : 5;
+                    c += 32 * b + 8 * (v >> 2) + (v & 3) + step < ncols ? step * ldc : 0;
+                    asm volatile("" : "+v"(c));
+                }
         }
     };
     if (K - k0 >= kMG && (K - k0) % kMG == 0 && (M % 4 == 0 || i0 + kT <= M)) {
@@ -200,6 +221,7 @@ __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, floa
         const float *Ap = A + min(arow, M - 4) + (k0 + ak) * lda;
 #pragma unroll
         for (int s = 0; s < kS; ++s) Bcol[s] += k0 + bk + kMG / 2 * bh;
+        int64_t left = (K - k0) / (2 * kQ);
         int t = 0;
         auto load = [&] {
 #pragma unroll
@@ -222,7 +244,7 @@ __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, floa
             for (int s = 0; s < kS; ++s) *reinterpret_cast<f32x4 *>(&Bs[bj + kBJ * s][kQ * bh + bk]) = rb[s];
         };
         load();
-        for (int64_t left = (K - k0) / (2 * kQ); left > 1; --left) {
+        for (; left > 1; --left) {
             put();
             __syncthreads();
             load();
@@ -231,7 +253,7 @@ __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, floa
         }
         put();
         __syncthreads();
-        load_c();   // its latency passes behind the last stage's products
+        load_c(0, 1);   // its latency passes behind the last stage's products
         products(kQ);
     } else {
         int half = (int)min(K - k0, (int64_t)kMG) >> 1, t = 0;
@@ -275,25 +297,40 @@ __device__ __forceinline__ void sgemm_tile(int64_t M, int64_t N, int64_t K, floa
             if (hh <= 0) break;
             __syncthreads();
         }
-        load_c();
+        load_c(0, 1);
     }
-    if (i >= M) return;
-    float *c = C + i + j * ldc;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const float r = beta == 0.0f ? alpha * acc[v] : beta * cv[v] + alpha * acc[v];
-        if (8 * (v >> 2) + (v & 3) < ncols) *c = r;
-        c += (v % 4 < 3 ? 1 : 5) * ldc;
-        asm volatile("" : "+v"(c));
+    for (int a = 0; a < kB; ++a) {
+        if (a > 0) load_c(a, a + 1);
+        const int64_t i = i0 + wi + 32 * a + l32;
+        if (i >= M) continue;
+        float *c = C + i + jb * ldc;
+#pragma unroll
+        for (int b = 0; b < kB; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float r = beta == 0.0f ? alpha * acc[a][b][v] : beta * cv[a][b][v] + alpha * acc[a][b][v];
+                if (32 * b + 8 * (v >> 2) + (v & 3) < ncols) *c = r;
+                c += (v % 4 < 3 ? 1 : 5) * ldc;
+                asm volatile("" : "+v"(c));
+            }
     }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+template <int kT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kT == 64 ? 4 : 3)))
 k_sgemm_mfma(int64_t M, int64_t N, int64_t K, float alpha, const float *__restrict__ A, int64_t lda,
              const float *__restrict__ B, int64_t ldb, float beta, float *__restrict__ C, int64_t ldc,
              int64_t sA, int64_t sB, int64_t sC) {
     const int64_t z = blockIdx.z;
-    sgemm_tile(M, N, K, alpha, A + z * sA, lda, B + z * sB, ldb, beta, C + z * sC, ldc);
+    // Workgroup l runs on XCD l % 8: each XCD takes a contiguous eighth of the
+    // tiles, and these in strips of eight rows of tiles, so that the tiles an
+    // XCD has at a time share their operands in its L2
+    const unsigned gx = gridDim.x, gy = gridDim.y, l = blockIdx.x + gx * blockIdx.y;
+    const unsigned xcd = l & 7, t = xcd * (gx * gy >> 3) + min(xcd, gx * gy & 7) + (l >> 3);
+    const unsigned strip = t / (8 * gy), r = t - strip * 8 * gy, rows = min(8u, gx - 8 * strip);
+    sgemm_tile<kT>(M, N, K, alpha, A + z * sA, lda, B + z * sB, ldb, beta, C + z * sC, ldc,
+                   8 * strip + r % rows, r / rows);
 }
 
 // Two independent batches of products C_p = alpha A_p B_p in one launch
@@ -315,12 +352,13 @@ k_sgemm_twin(SgemmTwin g0, SgemmTwin g1, float alpha, int batch) {
     const bool second = (int)blockIdx.z >= batch;
     const SgemmTwin g = second ? g1 : g0;
     const int64_t z = second ? blockIdx.z - batch : blockIdx.z;
+    constexpr int kT = 64;
     const int64_t i0 = (int64_t)blockIdx.x * kT, j0 = (int64_t)blockIdx.y * kT;
     if (i0 >= g.M || j0 >= g.N) return;
     const int64_t k0 = g.tri == 2 ? j0 : (g.tri == 3 ? i0 : 0);
     const int64_t k1 = g.tri == 1 ? j0 + kT : (g.tri == 4 ? i0 + kT : g.K);
-    sgemm_tile(g.M, g.N, k1 < g.K ? k1 : g.K, alpha, g.A + z * g.sA, g.lda, g.B + z * g.sB, g.ldb, 0.0f,
-                          g.C + z * g.sC, g.ldc, k0);
+    sgemm_tile<kT>(g.M, g.N, k1 < g.K ? k1 : g.K, alpha, g.A + z * g.sA, g.lda, g.B + z * g.sB, g.ldb, 0.0f,
+                          g.C + z * g.sC, g.ldc, blockIdx.x, blockIdx.y, k0);
 }
 
 __device__ __forceinline__ float lane_bcast(float v, int l) {
@@ -1165,8 +1203,20 @@ bool use_mfma(int64_t m, int64_t n, int64_t k, int64_t batch, const float *A, in
 
 int sgemm_mfma(int64_t m, int64_t n, int64_t k, float alpha, const float *A, int64_t lda, int64_t sA, const float *B,
                int64_t ldb, int64_t sB, float beta, float *C, int64_t ldc, int64_t sC, int64_t batch, hipStream_t st) {
-    const dim3 grid((unsigned)omx_cdiv(m, kT), (unsigned)omx_cdiv(n, kT), (unsigned)batch);
-    hipLaunchKernelGGL(k_sgemm_mfma, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, sA, sB, sC);
+    // 128-tiles halve the operands' traffic, which counts where k is deep and
+    // the matrix large (61440 x 61440 x 2560: 141 ms, 64-tiles 155); otherwise
+    // four workgroups a CU of 64-tiles hide one another's loads and C as well
+    // or better (30000 x 2304 x 256: 383 and 393 us; 7680 x 7680 x 512: both
+    // 528), and few tiles leave CUs idle
+    const bool big = k >= 512 && omx_cdiv(m, 128) * omx_cdiv(n, 128) * batch >= 1024;
+    const int t = big ? 128 : 64;
+    const dim3 grid((unsigned)omx_cdiv(m, t), (unsigned)omx_cdiv(n, t), (unsigned)batch);
+    if (big)
+        hipLaunchKernelGGL(k_sgemm_mfma<128>, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, sA,
+                           sB, sC);
+    else
+        hipLaunchKernelGGL(k_sgemm_mfma<64>, grid, dim3(256), 0, st, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, sA,
+                           sB, sC);
     OMX_LAUNCH_CHECK();
     return OMX_OK;
 }
@@ -1207,7 +1257,7 @@ int sgemm_batched(int64_t m, int64_t n, int64_t k, float alpha, const float *A, 
 // two batches of batch products each (k_sgemm_twin)
 int sgemm_twin(const SgemmTwin &g0, const SgemmTwin &g1, float alpha, int64_t batch, hipStream_t st) {
     const int64_t m = std::max(g0.M, g1.M), n = std::max(g0.N, g1.N);
-    const dim3 grid((unsigned)omx_cdiv(m, kT), (unsigned)omx_cdiv(n, kT), (unsigned)(2 * batch));
+    const dim3 grid((unsigned)omx_cdiv(m, 64), (unsigned)omx_cdiv(n, 64), (unsigned)(2 * batch));
     hipLaunchKernelGGL(k_sgemm_twin, grid, dim3(256), 0, st, g0, g1, alpha, (int)batch);
     OMX_LAUNCH_CHECK();
     return OMX_OK;

@@ -260,10 +260,12 @@ def test_merged_launches_leave_the_factors_alone(n, b, alt, flags, prec):
 
 # FP32 product on the matrix cores: with whole groups of 64 in k and whole
 # float4s of rows (or none, in the last row tile) and without either; one,
-# two and many groups; last columns and rows of a tile; nothing else written
+# two and many groups; last columns and rows of a tile (of 128 rows in the last
+# three); nothing else written
 @pytest.mark.parametrize("m,n,k,beta", [(1024, 257, 64, 1.0), (1023, 320, 128, 1.0), (513, 513, 192, 0.5),
                                         (4097, 65, 256, 0.0), (516, 1027, 48, 1.0), (1025, 256, 80, 1.0),
-                                        (524288, 1, 64, 1.0), (2, 131072, 64, 1.0), (2048, 129, 1040, 0.0)])
+                                        (524288, 1, 64, 1.0), (2, 131072, 64, 1.0), (2048, 129, 1040, 0.0),
+                                        (4100, 4033, 576, 1.0), (4099, 4000, 528, 0.5), (4224, 3970, 512, 0.0)])
 def test_sgemm_stage_and_tile_edges(m, n, k, beta):
     torch = torch_cuda()
     print(f"sgemm edges m={m} n={n} k={k} beta={beta}", flush=True)
