@@ -945,10 +945,10 @@ static bool trsv_vec(const float *A, int64_t lda) {
 // and the inversion of the diagonal blocks cost what they save (n = 512:
 // lower 25 us against 19, upper 26 against 28; n = 768: 28 against 30 and 30
 // against 44).  us, one launch against one per block, lower / upper:
-//   n = 1024    33 /   41    35 /    59      n =  61440  1674 /  3640   1697 /  4821
-//   n = 10240  190 /  467   205 /   648      n = 122880  5664 /  8534   5668 / 10740
-//   n = 20480  453 / 1131   464 /  1526      n = 204800 14471 / 18635  14501 / 21080
-// (5.8 TB/s of factor entries at n = 204800: the tiles' traffic).
+//   n = 1024    34 /   41    36 /    59      n =  61440  1687 /  3630   1729 /  4813
+//   n = 10240  198 /  468   209 /   649      n = 122880  5703 /  8509   5707 / 10725
+//   n = 20480  461 / 1128   473 /  1521      n = 204800 14593 / 18587  14619 / 21015
+// (5.7 TB/s of factor entries at n = 204800: the tiles' traffic).
 static int trsv_launch(bool upper, int64_t n, const float *A, int64_t lda, double *x, void *work, size_t work_bytes,
                        hipStream_t st, bool *done) {
     *done = false;
