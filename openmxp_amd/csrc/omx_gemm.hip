@@ -101,9 +101,10 @@ __device__ __forceinline__ void gl_lds16(const char *g, char *l) {
 //   C(i0 + 32 mi + lane%32, j0 + 32 ni + 8 (r/4) + 4 (lane/32) + r%4),
 // so each lane owns 16 columns of one row per 32 x 32 block and every load or
 // store instruction covers 32 consecutive rows of two columns.  They are
-// buffer instructions, one resource per 32-column block (wave-uniform 64-bit base in SGPRs, 16 per-lane 32-bit column offsets, the
-// row block in the immediate), in units of two row blocks of one column block:
-// the next unit's 32 old values are in flight while one is combined and stored.
+// buffer instructions, one resource per 32-column block (wave-uniform 64-bit
+// base in SGPRs, 16 per-lane 32-bit column offsets, the row block in the
+// immediate), in units of two row blocks of one column block: the next unit's
+// 32 old values are in flight while one is combined and stored.
 // Cache policy of the C loads and stores (buffer aux operand): NT (bit 1),
 // non-temporal.  Each C element is read and written once per launch, while
 // the packed panels are re-read by many workgroups through L2; streaming C

@@ -173,12 +173,6 @@ __global__ void k_axpy(int64_t n, double alpha, const double *__restrict__ x,
         y[i] = y[i] + alpha * x[i];
 }
 
-__global__ void k_zero(int64_t n, double *__restrict__ y) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        y[i] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // Triangular solves with the FP32 factors, FP64 vector and arithmetic,
 // without a workspace (or too small, or unaligned): one launch per 256 columns.
