@@ -645,6 +645,16 @@ __device__ __forceinline__ bool pivot_ok(float u) {
     return ex >= 4 && ex <= 250;
 }
 
+// r -= m u in the rows below the pivot.  The others have m = 0 (up to the sign
+// of a zero this leaves r as it is), but where a pivot was not pivot_ok (kDiv)
+// m can be 0 times an infinite reciprocal and u what an earlier such pivot
+// left: finished rows of U are selected there.
+template <bool kDiv>
+__device__ __forceinline__ void lu_update(float &r, float m, float u, bool below) {
+    const float d = __builtin_fmaf(-m, u, r);
+    r = kDiv && !below ? r : d;
+}
+
 // Factorisation of sh.d (see above) by the calling wave's share.  Columns
 // are handed over one by one: the wave that factors writes column g of the
 // factors to sh.d, then sh.prog = g + 1 (LDS operations of a wave complete in
@@ -677,7 +687,7 @@ __device__ __forceinline__ void lu_stages(float (&r)[8], int lane, int wave, Get
             for (int c = 0; c < 8; ++c) u[c] = lane_bcast(r[c], g);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) r[c] = __builtin_fmaf(-m, u[c], r[c]);
+            for (int c = 0; c < 8; ++c) lu_update<kDiv>(r[c], m, u[c], lane > g);
         }
     }
     const int g0 = 8 * wave, ln = lane - g0;
@@ -697,7 +707,7 @@ __device__ __forceinline__ void lu_stages(float (&r)[8], int lane, int wave, Get
         for (int c = k + 1; c < 8; ++c) u[c] = lane_bcast(r[c], g0 + k);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int c = k + 1; c < 8; ++c) r[c] = __builtin_fmaf(-m, u[c], r[c]);
+        for (int c = k + 1; c < 8; ++c) lu_update<kDiv>(r[c], m, u[c], ln > k);
     }
 }
 

@@ -109,6 +109,23 @@ def test_getrf_reports_the_first_zero_pivot(n, k):
     assert _getrf(A, n)[1] == k + 1
 
 
+# a pivot whose reciprocal is infinite or NaN: the rows of U up to and with
+# its own are finished, so they are those of the matrix with a healthy pivot in
+# its place, bit for bit (first, inner and last column of a wave's eight)
+@pytest.mark.parametrize("pivot", [0.0, -0.0, 1e-40, np.nan])
+@pytest.mark.parametrize("n,k", [(64, 0), (64, 5), (64, 62), (64, 63), (192, 70), (576, 515)])
+def test_getrf_keeps_finished_rows(n, k, pivot):
+    A = _dominant(n, n + k)
+    A[k:, :k] = 0.0  # row k reaches its pivot as it is
+    F, _ = _getrf(A, n)
+    A[k, k] = pivot
+    G, info = _getrf(A, n)
+    assert info == (k + 1 if pivot == 0.0 else 0x7fffffff) or np.isnan(pivot)
+    assert np.array_equal(G[k, k], np.float32(pivot), equal_nan=True)
+    F[k, k] = G[k, k] = 1.0
+    assert np.array_equal(G[:k + 1], F[:k + 1])
+
+
 # ranges that pair up evenly, leave an odd one, and pair unequal sizes; merges
 # in LDS (to 256 rows a side) and beyond; aligned and unaligned
 @pytest.mark.parametrize("pad", [0, 1])
