@@ -662,8 +662,10 @@ k_trsv_fused(int64_t n, const float *__restrict__ A, int64_t lda, double *__rest
             s = d;
         };
         // (rows past the matrix, in the lower solve's last block, read within
-        // the column's padding; their sums are not used)
-        const float *rows = A + min(d0 + 4 * lane, (n - 1) & ~(int64_t)3);
+        // the column's padding, and not the last column's; their sums are not
+        // used.  The upper solve's first block, whose tile holds the last
+        // column, is read within the matrix and not used)
+        const float *rows = A + min(d0 + 4 * lane, (kUpper ? n - 4 : n - 1) & ~(int64_t)3);
         f32x4 v[kTC];
         auto load_tile = [&](int64_t J) {
             const int64_t c0 = J * kTB + kTC * wave;

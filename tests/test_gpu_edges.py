@@ -194,6 +194,30 @@ def test_trsv_with_workspace(n, lda):
         assert np.all(np.isfinite(g[before])) and np.all(np.isnan(g[after]))
 
 
+# the smallest buffer a factor may lie in: it ends with the last column's row n,
+# and nothing beyond is read (the bytes after it are another tensor's)
+@pytest.mark.parametrize("n", [513, 770, 1023])
+def test_trsv_smallest_buffer(n):
+    torch = torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    lda = (n + 3) // 4 * 4
+    F = (rng.uniform(-1, 1, (n, n)) / n + np.diag(rng.uniform(1, 2, n))).astype(np.float32)
+    store = np.full((n, lda), np.nan, np.float32)
+    store[:, :n] = F.T
+    Ad = dev(store.reshape(-1)[:(n - 1) * lda + n])
+    wb = L.omx_trsv_workspace_bytes(n)
+    W = empty(wb, torch.uint8)
+    r = rng.uniform(-1, 1, n)
+    F64 = F.astype(np.float64)
+    for solve, T in ((L.omx_trsv_lower_unit_f32f64, np.tril(F64, -1) + np.eye(n)),
+                     (L.omx_trsv_upper_f32f64, np.triu(F64))):
+        xd = dev(r)
+        assert solve(n, n, ptr(Ad), lda, ptr(xd), ptr(W), wb, None) == 0
+        want = np.linalg.solve(T, r)
+        assert np.max(np.abs(host(xd) - want)) <= 1e-13 * np.max(np.abs(want))
+
+
 # one workgroup's rows, one more, ragged ends; the largest entries at either
 # end of the sums
 @pytest.mark.parametrize("n", [2, 63, 64, 1023, 1024, 1025, 2048, 5000])
