@@ -214,8 +214,7 @@ size_t omx_trsv_workspace_bytes(int64_t n);
  * arithmetic.  `b` is the factorisation's block size and only checked
  * (n % b == 0); the solve walks blocks of 256: each block row adds up
  * L_ij x_j over the blocks before it and is then solved with its diagonal
- * block (with the workspace, by the FP64 inverses of that block's 64 x 64
- * diagonal sub-blocks).  Replaces trsvL_h
+ * block by substitution, with or without the workspace.  Replaces trsvL_h
  * (panel_trsv.hpp:308-449: cast_copy_general + rocblas_dtrsv +
  * HPLMXP_gemv + daxpy) for one GPU, without the reference's per-block-column
  * swap of accumulation buffers. */

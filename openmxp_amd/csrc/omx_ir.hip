@@ -456,41 +456,37 @@ k_trsv_upper_step(int64_t n, int64_t j0, const float *__restrict__ A, int64_t ld
 // waits for blocks whose tickets were taken before its own, so whatever is
 // resident, the first unfinished block never waits).  For its block row I a
 // workgroup
-//   1. inverts the four 64 x 64 diagonal sub-blocks in FP64 (MFMA, below) and
-//      keeps the six sub-blocks between them in LDS: none of this needs x;
+//   1. keeps its diagonal block in LDS and registers, none of which needs x;
 //   2. adds up M(I, J) x_J in registers for J in solution order as the x_J
 //      appear; the next 256 x 256 tile of M is loaded while it waits;
-//   3. finishes x_I in four stages (a product with an inverse, then with the
-//      sub-blocks beyond it) and publishes it.
+//   3. solves x_I by substitution, 16 rows a phase, a wave each: the rows'
+//      triangle in the lanes (tri16_solve), then their products with the later
+//      waves' rows; and publishes it.
 // Published values are their own flags: xs starts as kUnset, a NaN that no
 // result is published as; readers poll it with device-scope loads.
 // The launch per 256 columns it replaces took 14 (lower) and 18 us (upper)
 // however few rows were left: launch, 256 KB through one CU, and 256
-// dependent steps.  A block now takes 4.5 us from x_J to x_I (hand-over
-// between XCDs 0.5, the last tile 0.5, sums 1.0, four stages 2.5), 5-7 while
-// hundreds of workgroups stream their tiles; where the matrix is large the
-// tiles' traffic bounds it (figures at trsv_launch).
+// dependent steps.  A block now takes 7 us from x_J to x_I: hand-over between
+// XCDs 0.5, the last tile 0.5, sums 1.0, 16 phases of 0.3 (16 FMAs 0.1, the
+// way to the next wave through LDS and the sums of its lanes 0.2).  Products
+// with FP64 inverses of the 64 x 64 diagonal sub-blocks in place of the
+// substitution took 5 to 6 us, but are not backward stable: with factors of a
+// randsvd system of condition 1e6 a row was off by 3e-12 of its terms' sum,
+// which substitution keeps at 3e-16 (per-block launches 4e-16), and with one
+// pivot of 1e-12 by 1e-5.  Where the matrix is large the tiles' traffic bounds
+// it (figures at trsv_launch).
 // ---------------------------------------------------------------------------
 constexpr uint64_t kUnset = 0x7FF4A5A5D00D5EEDull;  // a signalling NaN: arithmetic quiets it
 constexpr int kOffSub = kSB * kSB;                  // entries of a sub-block between the diagonal ones
-constexpr int kDiagLd = kSB + 4;                    // column stride of a staged diagonal sub-block
-
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-struct __align__(16) TrsvPrep {
-    float diag[4][kSB * kDiagLd];  // diag[k][c kDiagLd + r]: sub-block k, masked to its triangle
-    double inv[16][16][17];        // inverses of the 16 x 16 blocks on the diagonal: [block][row][column]
-};
+constexpr int kT16 = 20;                            // row stride of a staged 16 x 16 triangle
 
 struct __align__(16) TrsvFused {
-    union {
-        TrsvPrep prep;
-        float off[6][kOffSub];     // sub-blocks (t, s) at slot off_slot: [c 64 + (r ^ 16 (c % 4))]
-    };
-    double part[kTW][kTB];         // per-wave sums of step 2
-    double xv[2][kTB];             // x_J, alternating
+    double xd[kTB];                // x_I (first: its reads have no address to form)
     double rd[kTB];                // r_I less what is known
-    double xd[kTB];                // x_I
+    double xv[2][kTB];             // x_J, alternating
+    double part[kTW][kTB];         // per-wave sums of step 2
+    float t16[kTW][16][kT16];      // the 16 x 16 triangles on the diagonal, negated: [block][row][column]
+    float off[6][kOffSub];         // sub-blocks (t, s) at slot off_slot: [c 64 + (r ^ 16 (c % 4))]
     int ticket;
 };
 
@@ -520,41 +516,49 @@ __device__ __forceinline__ double sum_groups(double v) {
            __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
 }
 
-// Rows [16 rb, 16 rb + 16) of the inverse of diagonal sub-block k, transposed,
-// as MFMA accumulators: z[b][i] in lane l is the entry (row 16 rb + l % 16,
-// column 16 b + 4 i + l / 16).  v_mfma_f64_16x16x4_f64 leaves row 4 i + l / 16
-// of its result in register i of lane l, which is the lane's share of the
-// second operand's k = 4 i + l / 16: each block of the solution feeds the
-// next products as it is.  Solves T^T Z = I(:, rb) block by block.
+// v += x m with x of lane q of the lane's row of 16: one FMA, whose DPP form
+// reads x across the row (after two wait states if x was just written)
+#define OMX_ROW_FMA(v, x, m, q) "s_nop 1\n\tv_fmac_f64_dpp " v ", " x ", " m " row_newbcast:" q " row_mask:0xf bank_mask:0xf\n\t"
+
+// Substitution with a 16 x 16 unit triangle: lane i of each row of 16 lanes
+// holds entry i of the right-hand side v and the negated row i of the triangle,
+// zero on and outside its diagonal: entries solved before stay as they are.
+// (One asm block: between two the compiler puts a wait state more.)
 template <bool kUpper>
-__device__ __forceinline__ void inverse_rows(const TrsvPrep &p, int k, int rb, int lane, f64x4 (&z)[4]) {
-    const int i16 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) z[b][i] = (b == rb && 4 * i + g == i16) ? 1.0 : 0.0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int b = kUpper ? q : 3 - q;
-        if (kUpper ? b >= rb : b <= rb) {  // (zero elsewhere; rb is the wave's)
-            // z_b <- inv16(T_bb)^T z_b
-            f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p.inv[4 * k + b][4 * i + g][i16], z[b][i], acc, 0, 0, 0);
-            z[b] = acc;
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-                if (kUpper ? m <= b : m >= b) continue;
-                // z_m -= T(b, m)^T z_b
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    z[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        -(double)p.diag[k][(16 * m + i16) * kDiagLd + 16 * b + 4 * i + g], z[b][i], z[m], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+__device__ __forceinline__ double tri16_solve(double v, const double (&nt)[16]) {
+    if (kUpper)
+        asm(OMX_ROW_FMA("%0", "%0", "%1", "15") OMX_ROW_FMA("%0", "%0", "%2", "14") OMX_ROW_FMA("%0", "%0", "%3", "13")
+            OMX_ROW_FMA("%0", "%0", "%4", "12") OMX_ROW_FMA("%0", "%0", "%5", "11") OMX_ROW_FMA("%0", "%0", "%6", "10")
+            OMX_ROW_FMA("%0", "%0", "%7", "9") OMX_ROW_FMA("%0", "%0", "%8", "8") OMX_ROW_FMA("%0", "%0", "%9", "7")
+            OMX_ROW_FMA("%0", "%0", "%10", "6") OMX_ROW_FMA("%0", "%0", "%11", "5") OMX_ROW_FMA("%0", "%0", "%12", "4")
+            OMX_ROW_FMA("%0", "%0", "%13", "3") OMX_ROW_FMA("%0", "%0", "%14", "2") OMX_ROW_FMA("%0", "%0", "%15", "1")
+            : "+&v"(v)
+            : "v"(nt[15]), "v"(nt[14]), "v"(nt[13]), "v"(nt[12]), "v"(nt[11]), "v"(nt[10]), "v"(nt[9]), "v"(nt[8]),
+              "v"(nt[7]), "v"(nt[6]), "v"(nt[5]), "v"(nt[4]), "v"(nt[3]), "v"(nt[2]), "v"(nt[1]));
+    else
+        asm(OMX_ROW_FMA("%0", "%0", "%1", "0") OMX_ROW_FMA("%0", "%0", "%2", "1") OMX_ROW_FMA("%0", "%0", "%3", "2")
+            OMX_ROW_FMA("%0", "%0", "%4", "3") OMX_ROW_FMA("%0", "%0", "%5", "4") OMX_ROW_FMA("%0", "%0", "%6", "5")
+            OMX_ROW_FMA("%0", "%0", "%7", "6") OMX_ROW_FMA("%0", "%0", "%8", "7") OMX_ROW_FMA("%0", "%0", "%9", "8")
+            OMX_ROW_FMA("%0", "%0", "%10", "9") OMX_ROW_FMA("%0", "%0", "%11", "10") OMX_ROW_FMA("%0", "%0", "%12", "11")
+            OMX_ROW_FMA("%0", "%0", "%13", "12") OMX_ROW_FMA("%0", "%0", "%14", "13") OMX_ROW_FMA("%0", "%0", "%15", "14")
+            : "+&v"(v)
+            : "v"(nt[0]), "v"(nt[1]), "v"(nt[2]), "v"(nt[3]), "v"(nt[4]), "v"(nt[5]), "v"(nt[6]), "v"(nt[7]),
+              "v"(nt[8]), "v"(nt[9]), "v"(nt[10]), "v"(nt[11]), "v"(nt[12]), "v"(nt[13]), "v"(nt[14]));
+    return v;
+}
+
+// The same where an entry is infinite or NaN, which times a zero multiplier is
+// no 0: solved entries are left by selection.  nt: the lane's negated row of
+// the triangle in LDS, not scaled; u: its diagonal (lower: 1).
+template <bool kUpper>
+__device__ __forceinline__ double tri16_select(double v, int i16, const float *nt, double u) {
+#pragma unroll 1
+    for (int q = 0; q < 16; ++q) {
+        const int c = kUpper ? 15 - q : q;
+        const double d = __builtin_fma(__shfl(kUpper ? v / u : v, c, 16), (double)nt[c], v);
+        v = (kUpper ? i16 < c : i16 > c) ? d : v;
     }
+    return kUpper ? v / u : v;
 }
 
 // Barrier that orders LDS accesses only: __syncthreads() would also wait for
@@ -587,53 +591,30 @@ k_trsv_fused(int64_t n, const float *__restrict__ A, int64_t lda, double *__rest
         const int64_t d0 = I * kTB;
         const int dim = (int)min((int64_t)kTB, n - d0);
         const float *D = A + d0 + d0 * lda;
-        // ---- 1. the diagonal block ----
+        // ---- 1. the diagonal block: this wave's rows 16 wave .. + 15, lane
+        // (i16, g) row i16.  Their triangle goes to LDS; sub[c][b]: columns
+        // 4 b + g of the 16 x 16 block left (right) of it that is solved c-th
+        // in the 64 x 64 sub-block.  Rows and columns past the matrix: the
+        // identity ----
+        const int k4 = wave >> 2, rb = wave & 3, row = 16 * wave + i16;
+        float sub[3][4], ud = 1.0f;
         {
-            float v[16];
+            const float *Drow = D + min(row, dim - 1);
+            auto entry = [&](int c, bool in) {
+                const float e = Drow[(int64_t)min(c, dim - 1) * lda];
+                return in && row < dim && c < dim ? e : 0.0f;
+            };
+            f32x4 t;
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int r = kSB * (q >> 2) + lane, c = kSB * (q >> 2) + wave + 16 * (q & 3);
-                v[q] = D[min(r, dim - 1) + (int64_t)min(c, dim - 1) * lda];
-            }
+            for (int j = 0; j < 4; ++j)
+                t[j] = -entry(16 * wave + 4 * g + j, kUpper ? 4 * g + j > i16 : 4 * g + j < i16);
+            *reinterpret_cast<f32x4 *>(&sh.t16[wave][i16][4 * g]) = t;
+            if (kUpper && row < dim) ud = Drow[(int64_t)row * lda];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                // rows and columns past the matrix: the identity
-                const int r = lane, c = wave + 16 * (q & 3), o = kSB * (q >> 2);
-                const bool in = o + r < dim && o + c < dim && (kUpper ? r <= c : r > c);
-                const bool one = r == c && (!kUpper || o + r >= dim);
-                sh.prep.diag[q >> 2][c * kDiagLd + r] = in ? v[q] : (one ? 1.0f : 0.0f);
-            }
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) sub[c][b] = entry(kSB * k4 + 16 * (kUpper ? 3 - c : c) + 4 * b + g, true);
         }
-        lds_sync();
-        {
-            // wave w: 16 x 16 block w % 4 of sub-block w / 4, lane c its column c
-            const float *T = &sh.prep.diag[wave >> 2][(wave & 3) * 16 * (kDiagLd + 1)];
-            double y[16], rec = 1.0;
-            if (kUpper) rec = 1.0 / (double)T[i16 * kDiagLd + i16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int r = kUpper ? 15 - q : q;
-                double s = r == i16 ? 1.0 : 0.0;
-#pragma unroll
-                for (int u = 0; u < q; ++u) {
-                    const int c = kUpper ? 15 - u : u;
-                    s = __builtin_fma(-(double)T[c * kDiagLd + r], y[c], s);
-                }
-                y[r] = kUpper ? s * bcast_lane(rec, r) : s;
-                // (entry by entry: all of T's entries fetched ahead would spill)
-                asm volatile("" : "+v"(y[r]));
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            if (lane < 16) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sh.prep.inv[wave][r][lane] = y[r];
-            }
-        }
-        lds_sync();
-        const int k4 = wave >> 2, rb = wave & 3;  // this wave: rows [16 rb, 16 rb + 16) of sub-block k4
-        f64x4 z[4];
-        inverse_rows<kUpper>(sh.prep, k4, rb, lane, z);
-        lds_sync();
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
             const int hi = q < 1 ? 1 : (q < 3 ? 2 : 3), lo = q - hi * (hi - 1) / 2;
@@ -737,78 +718,65 @@ k_trsv_fused(int64_t n, const float *__restrict__ A, int64_t lda, double *__rest
             sh.rd[tid] = tid < dim ? r_in - q[0] : 0.0;
         }
         lds_sync();
-        // ---- 3. x_I: stage st solves sub-block st with its inverse, then
-        // takes its products off the next one (the others' sums wait) ----
-        const double r_own = sh.rd[kSB * k4 + 16 * rb + i16];
-        double acc = 0.0;  // this lane's share of what its row loses to solved sub-blocks
-#pragma unroll 1
-        for (int q = 0; q < 4; ++q) {
-            const int st = kUpper ? 3 - q : q;
-            const bool later = kUpper ? k4 < st : k4 > st;
-            // (opaque, as above: what is derived from them stays in the loop)
-            int own = 16 * rb + i16, gq = g;
-            asm volatile("" : "+v"(own), "+v"(gq));
-            if (k4 == st) {
-                const double *r = sh.rd + kSB * st + gq;
-                double rc[16], y = 0.0, y2 = 0.0;
+        // ---- 3. x_I: phase p solves 16 rows by substitution in their wave
+        // and takes them off the rows of the later waves (whose sums wait) ----
+        // The upper solve's rows are scaled by their diagonals beforehand (the
+        // right-hand side divided, as diag_solve's quotient), so that its
+        // chain is one FMA an entry too.
+        const double r_own = sh.rd[row], u = (double)ud, y = kUpper ? 1.0 / u : 1.0;
+        double nt[16], acc = 0.0;  // acc: this lane's share of what its row loses to solved rows
 #pragma unroll
-                for (int b = 0; b < 16; ++b) rc[b] = r[4 * b];
-                __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < 16; j += 4) {
+            const f32x4 t = *reinterpret_cast<const f32x4 *>(&sh.t16[wave][i16][j]);
 #pragma unroll
-                for (int b = 0; b < 16; b += 2) {
-                    y = __builtin_fma(z[b >> 2][b & 3], rc[b], y);
-                    y2 = __builtin_fma(z[(b + 1) >> 2][(b + 1) & 3], rc[b + 1], y2);
-                }
-                y = sum_groups(y + y2);
-                if (__builtin_expect(!__all(fabs(y) < __builtin_inf()), 0)) {
-                    // an infinity or NaN may have met the inverse's zeros:
-                    // once more with the row's own triangle only
-                    y = 0.0;
-#pragma unroll
-                    for (int b = 0; b < 16; ++b) {
-                        const int c = 4 * b + gq;
-                        y = __builtin_fma(z[b >> 2][b & 3], (kUpper ? c >= own : c <= own) ? rc[b] : 0.0, y);
-                    }
-                    y = sum_groups(y);
-                }
-                if (gq == 0) {
-                    const int row = kSB * st + own;
-                    sh.xd[row] = y;
-                    if (row < dim) {
-                        uint64_t w = __builtin_bit_cast(uint64_t, y);
-                        if (w == kUnset) w |= 1ull << 51;  // (quiet)
-                        __hip_atomic_store(xs + d0 + row, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        x[d0 + row] = y;
-                    }
-                }
-                lds_sync();
-            } else if (later) {
-                // (barriers in each branch: the waves' roles share no registers)
-                const float *src = sh.off[off_slot(k4, st)] + (own ^ (gq << 4)) + gq * kSB;
-                const double *xd = sh.xd + kSB * st + gq;
-                float o[16];
-                double xc[16], a2 = 0.0;
-#pragma unroll
-                for (int b = 0; b < 16; ++b) o[b] = src[4 * b * kSB];
-                lds_sync();
-#pragma unroll
-                for (int b = 0; b < 16; ++b) xc[b] = xd[4 * b];
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int b = 0; b < 16; b += 2) {
-                    acc = __builtin_fma((double)o[b], xc[b], acc);
-                    a2 = __builtin_fma((double)o[b + 1], xc[b + 1], a2);
-                }
-                acc += a2;
-                if (kUpper ? k4 == st - 1 : k4 == st + 1) {
-                    const double d = sum_groups(acc);
-                    if (gq == 0) sh.rd[kSB * k4 + own] = r_own - d;
-                }
-            } else {
-                lds_sync();
+            for (int e = 0; e < 4; ++e) {
+                nt[j + e] = kUpper ? (double)t[e] * y : (double)t[e];
+                asm volatile("" : "+v"(nt[j + e]));  // (converted now, not in the chain)
             }
-            lds_sync();
         }
+        const int own = kUpper ? 15 - wave : wave;  // this wave's phase
+        // phase p: the products with the rows it solves, of which o are this
+        // lane's four entries
+        auto wait = [&](int p, const float (&o)[4]) {
+            double m[4], xc[4];
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                m[b] = (double)o[b];
+                asm volatile("" : "+v"(m[b]));
+            }
+            const double *xd = sh.xd + 16 * (kUpper ? 15 - p : p) + g;
+            lds_sync();
+            if (p == own - 1) __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) xc[b] = xd[4 * b];
+            acc += __builtin_fma(m[1], xc[1], m[0] * xc[0]) + __builtin_fma(m[3], xc[3], m[2] * xc[2]);
+        };
+#pragma unroll 1
+        for (int p = 0; p < (own & ~3); ++p) {  // other sub-blocks
+            const int wp = kUpper ? 15 - p : p;
+            const float *src = sh.off[off_slot(k4, wp >> 2)] + (16 * (wp & 3) + g) * kSB + ((16 * rb + i16) ^ (g << 4));
+            const float o[4] = {src[0], src[4 * kSB], src[8 * kSB], src[12 * kSB]};
+            wait(p, o);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)  // its own
+            if (c < (own & 3)) wait((own & ~3) + c, sub[c]);
+        {
+            const double r = r_own - sum_groups(acc), q0 = r * y;
+            double v = tri16_solve<kUpper>(kUpper ? __builtin_fma(__builtin_fma(-u, q0, r), y, q0) : r, nt);
+            if (__builtin_expect(!__all(fabs(v) < __builtin_inf()), 0))
+                v = tri16_select<kUpper>(r, i16, sh.t16[wave][i16], u);
+            if (g == 0) sh.xd[row] = v;
+            lds_sync();
+            __builtin_amdgcn_s_setprio(0);
+            if (g == 0 && row < dim) {
+                uint64_t w = __builtin_bit_cast(uint64_t, v);
+                if (w == kUnset) w |= 1ull << 51;  // (quiet)
+                __hip_atomic_store(xs + d0 + row, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                x[d0 + row] = v;
+            }
+        }
+        for (int p = own + 1; p < 16; ++p) lds_sync();
     }
 }
 
@@ -938,13 +906,12 @@ static bool trsv_vec(const float *A, int64_t lda) {
 
 // The solve in one launch when the caller gives the workspace; OMX_OK and
 // *done = true if it was queued.  From three blocks on: with two the launch
-// and the inversion of the diagonal blocks cost what they save (n = 512:
-// lower 25 us against 19, upper 26 against 28; n = 768: 28 against 30 and 30
-// against 44).  us, one launch against one per block, lower / upper:
-//   n = 1024    34 /   41    36 /    59      n =  61440  1687 /  3630   1729 /  4813
-//   n = 10240  198 /  468   209 /   649      n = 122880  5703 /  8509   5707 / 10725
-//   n = 20480  461 / 1128   473 /  1521      n = 204800 14593 / 18587  14619 / 21015
-// (5.7 TB/s of factor entries at n = 204800: the tiles' traffic).
+// and the diagonal block's staging cost what they save.  us, a launch per block
+// -> one launch, lower | upper:
+//   n =   768    30 ->   29 |   43 ->   29    n =  61440   3674 ->  1908 |  4807 ->  1940
+//   n =  1024    40 ->   35 |   59 ->   36    n = 122880   8501 ->  5661 | 10737 ->  5697
+//   n = 10240   461 ->  282 |  652 ->  295    n = 204800  18568 -> 14521 | 21010 -> 14584
+// (5.8 TB/s of factor entries at n = 204800: the tiles' traffic).
 static int trsv_launch(bool upper, int64_t n, const float *A, int64_t lda, double *x, void *work, size_t work_bytes,
                        hipStream_t st, bool *done) {
     *done = false;

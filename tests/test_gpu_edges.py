@@ -194,6 +194,108 @@ def test_trsv_with_workspace(n, lda):
         assert np.all(np.isfinite(g[before])) and np.all(np.isnan(g[after]))
 
 
+def _lu_nopiv_f32(A):
+    F = A.astype(np.float32)
+    for k in range(F.shape[0] - 1):
+        F[k + 1:, k] /= F[k, k]
+        F[k + 1:, k + 1:] -= np.outer(F[k + 1:, k], F[k, k + 1:])
+    return F
+
+
+def _trsv_factor(kind, n, rng):
+    """LU factors whose 64 x 64 diagonal sub-blocks are ill-conditioned."""
+    if kind == "randsvd":  # condition 1e6, no pivoting
+        Q = [np.linalg.qr(rng.standard_normal((n, n)))[0] for _ in range(2)]
+        return _lu_nopiv_f32((Q[0] * np.logspace(0, -6, n)) @ Q[1])
+    F = rng.uniform(-1, 1, (n, n)) / n
+    for o in range(0, n, 64):
+        F[o:o + 64, o:o + 64] *= n / 4
+    F[np.arange(n), np.arange(n)] = rng.uniform(1, 2, n)
+    for k in (20, n // 2 + 5, n - 30):  # a small pivot and the multipliers that it leaves
+        F[k, k] = kind
+        F[k + 1:k // 64 * 64 + 64, k] /= kind
+    return F.astype(np.float32)
+
+
+# the one-launch solves and the launch per block on ill-conditioned diagonal
+# sub-blocks: the backward error of each row is that of a substitution.  A
+# term of a row meets at most 118 roundings (its sub-block's substitution 63 or
+# 64, the sums of the columns before it 48 + 4, or 16 a tile and the tiles' sums)
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("n", [768, 1036])
+@pytest.mark.parametrize("kind", [1e-3, 1e-6, 1e-12, "randsvd"])
+def test_trsv_backward_error(kind, n, workspace):
+    torch = torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    F = _trsv_factor(kind, n, rng)
+    Ad = dev(F.T.copy())
+    wb = L.omx_trsv_workspace_bytes(n) if workspace else 0
+    W = empty(max(wb, 8), torch.uint8).fill_(255)
+    F64 = F.astype(np.float64)
+    for solve, T in ((L.omx_trsv_lower_unit_f32f64, np.tril(F64, -1) + np.eye(n)),
+                     (L.omx_trsv_upper_f32f64, np.triu(F64))):
+        r = T @ rng.uniform(-1, 1, n)
+        xd = dev(r)
+        assert solve(n, n, ptr(Ad), n, ptr(xd), ptr(W) if workspace else None, wb, None) == 0
+        x, T = host(xd).astype(np.longdouble), T.astype(np.longdouble)
+        err = np.abs(r - T @ x) / (np.abs(r) + np.abs(T) @ np.abs(x))
+        print(f"trsv {kind} n={n} workspace={workspace}: backward error {float(err.max()):.2e}", flush=True)
+        assert err.max() <= 128 * 2.0 ** -53
+
+
+# a zero u_kk makes x_k infinite; what was solved before it stays a solution
+@pytest.mark.parametrize("k", [0, 13, 16, 63, 300, 575])
+def test_trsv_zero_pivot_leaves_the_solved_entries(k):
+    torch = torch_cuda()
+    L, n = _L(), 576
+    rng = np.random.default_rng(k)
+    F = (np.triu(rng.uniform(-1, 1, (n, n)) / n, 1) + np.diag(rng.uniform(1, 2, n))).astype(np.float32)
+    F[k, k] = 0.0
+    r = rng.uniform(-1, 1, n)
+    wb = L.omx_trsv_workspace_bytes(n)
+    Ad, xd, W = dev(F.T.copy()), dev(r), empty(wb, torch.uint8).fill_(255)
+    assert L.omx_trsv_upper_f32f64(n, n, ptr(Ad), n, ptr(xd), ptr(W), wb, None) == 0
+    x = host(xd)
+    assert not np.any(np.isfinite(x[:k + 1])) and np.isinf(x[k])
+    T, x, r = F[k + 1:, k + 1:].astype(np.longdouble), x[k + 1:].astype(np.longdouble), r[k + 1:]
+    assert np.all(np.abs(r - T @ x) <= 128 * 2.0 ** -53 * (np.abs(r) + np.abs(T) @ np.abs(x)))
+
+
+# more blocks than workgroups (a workgroup solves several): a factor with a
+# few bands, within and across blocks, solved on the host band by band
+@pytest.mark.parametrize("n", [65792, 66052])
+def test_trsv_more_blocks_than_workgroups(n):
+    torch = torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    bands = [1, 17, 64, 255, 256, 300, 5000, 65536]
+    A = torch.zeros(n * n, dtype=torch.float32, device="cuda")  # column-major
+    d = rng.uniform(1, 2, n).astype(np.float32)
+    A[::n + 1] = dev(d)
+    lo, up = {}, {}
+    for o in bands:
+        lo[o], up[o] = (rng.uniform(-0.2, 0.2, n - o).astype(np.float32) for _ in range(2))
+        A[o::n + 1][:n - o] = dev(lo[o])            # (i + o, i)
+        A[o * n::n + 1][:n - o] = dev(up[o])        # (i, i + o)
+    wb = L.omx_trsv_workspace_bytes(n)
+    W = empty(wb, torch.uint8).fill_(255)
+    for solve, coef, upper in ((L.omx_trsv_lower_unit_f32f64, lo, False), (L.omx_trsv_upper_f32f64, up, True)):
+        r = rng.uniform(-1, 1, n)
+        xd = dev(r)
+        print(f"trsv n={n} upper={upper}", flush=True)
+        assert solve(n, n, ptr(A), n, ptr(xd), ptr(W), wb, None) == 0
+        x = host(xd)
+        res, mag = r - x * (d.astype(np.float64) if upper else 1.0), np.abs(r) + np.abs(x) * 2
+        for o in bands:
+            t = coef[o].astype(np.float64) * (x[o:] if upper else x[:-o])
+            (res[:-o] if upper else res[o:])[:] -= t
+            (mag[:-o] if upper else mag[o:])[:] += np.abs(t)
+        # 118 roundings a term (above), and those of this check
+        assert np.all(np.abs(res) <= 160 * 2.0 ** -53 * mag)
+    del A
+
+
 # the smallest buffer a factor may lie in: it ends with the last column's row n,
 # and nothing beyond is read (the bytes after it are another tensor's)
 @pytest.mark.parametrize("n", [513, 770, 1023])
