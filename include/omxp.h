@@ -84,7 +84,9 @@ int omx_rhs_f64(int64_t n, uint64_t seed, double *b, void *stream);
  * Refinement kernels (FP64).
  * ------------------------------------------------------------------------- */
 
-/* Bytes of scratch omx_otf_gemv_f64 needs for order n. */
+/* Bytes of scratch with which omx_otf_gemv_f64 runs fastest at order n.  It
+ * takes fewer, and then forms fewer column segments: for n <= 16384 down to
+ * 8 n ceil(n / 256) (none, and `work` may be NULL, for n <= 256). */
 size_t omx_otf_gemv_workspace_bytes(int64_t n);
 
 /* y <- y + alpha * A x with A the generated order-n matrix, regenerated from

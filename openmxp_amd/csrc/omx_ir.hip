@@ -29,11 +29,12 @@ constexpr int kGemvMaxSeg = 64;
 // steps).  At n = 1024 segments of 256 columns left 15 of 16 SIMDs without a
 // wave, and the columns of the diagonal, a load and a step at a time,
 // took longer than all others: 22.4 us, 10.6 now; 5120 29.0 -> 20, 10240 48 -> 39.
-int gemv_segments(int64_t n) {
+// mincols = 256: the fewer segments of a call with a smaller workspace.
+int gemv_segments(int64_t n, int64_t mincols = 64) {
     const int64_t nrb = omx_cdiv(n, kGemvRows);
     int64_t s = omx_cdiv(kGemvTargetWG, nrb);
     if (s > kGemvMaxSeg) s = kGemvMaxSeg;
-    const int64_t smax = omx_cdiv(n, 64);
+    const int64_t smax = omx_cdiv(n, mincols);
     if (s > smax) s = smax;
     if (s < 1) s = 1;
     return (int)s;
@@ -787,24 +788,14 @@ int grid_for(int64_t n, int threads) {
     return (int)g;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t omx_otf_gemv_workspace_bytes(int64_t n) {
-    if (n <= 0) return 0;
-    const int s = gemv_segments(n);
-    return s > 1 ? (size_t)s * (size_t)n * sizeof(double) : 0;
+// bytes of nseg column segments' partial sums
+size_t segment_bytes(int64_t n, int nseg) {
+    return nseg > 1 ? (size_t)nseg * (size_t)n * sizeof(double) : 0;
 }
 
-}  // extern "C"
-
-namespace {
-
-// The residual GEMV's launches; part holds omx_otf_gemv_workspace_bytes(n).
-int otf_gemv_launch(int64_t n, uint64_t seed, const double *diag, double alpha, const double *x, double *y,
+// The residual GEMV's launches; work holds segment_bytes(n, nseg).
+int otf_gemv_launch(int64_t n, int nseg, uint64_t seed, const double *diag, double alpha, const double *x, double *y,
                     void *work, hipStream_t st) {
-    const int nseg = gemv_segments(n);
     const int64_t seglen = omx_cdiv(n, nseg);
     const int64_t nrb = omx_cdiv(n, kGemvRows);
     double *part = nseg > 1 ? static_cast<double *>(work) : nullptr;
@@ -842,13 +833,19 @@ int noalloc_scratch(double **out) {
 
 extern "C" {
 
+size_t omx_otf_gemv_workspace_bytes(int64_t n) {
+    return n > 0 ? segment_bytes(n, gemv_segments(n)) : 0;
+}
+
 int omx_otf_gemv_f64(int64_t n, uint64_t seed, const double *diag, double alpha,
                      const double *x, double *y, void *work, size_t work_bytes,
                      void *stream) {
     if (n <= 0 || !diag || !x || !y) return OMX_ERR_ARG;
-    const size_t need = omx_otf_gemv_workspace_bytes(n);
-    if (need > 0 && (!work || work_bytes < need)) return OMX_ERR_WORKSPACE;
-    return otf_gemv_launch(n, seed, diag, alpha, x, y, work, omx_stream(stream));
+    const size_t have = work ? work_bytes : 0;
+    int nseg = gemv_segments(n);
+    if (have < segment_bytes(n, nseg)) nseg = gemv_segments(n, 256);
+    if (have < segment_bytes(n, nseg)) return OMX_ERR_WORKSPACE;
+    return otf_gemv_launch(n, nseg, seed, diag, alpha, x, y, work, omx_stream(stream));
 }
 
 int omx_otf_gemv_f64_noalloc(int64_t n, uint64_t seed, const double *diag, double alpha, const double *x,
@@ -858,7 +855,7 @@ int omx_otf_gemv_f64_noalloc(int64_t n, uint64_t seed, const double *diag, doubl
     double *part = nullptr;
     const int rc = noalloc_scratch(&part);
     if (rc) return rc;
-    return otf_gemv_launch(n, seed, diag, alpha, x, y, part, omx_stream(stream));
+    return otf_gemv_launch(n, gemv_segments(n), seed, diag, alpha, x, y, part, omx_stream(stream));
 }
 
 int omx_norm_inf_f64(int64_t n, const double *x, double *result, void *stream) {

@@ -447,6 +447,27 @@ def test_otf_gemv_segment_edges(orc, n):
     assert np.all(np.abs(host(Y) - ref) <= bound)
 
 
+# a workspace for segments of 256 columns (none up to n = 256) is taken, with
+# fewer segments; one byte less is refused
+@pytest.mark.parametrize("n", [1, 100, 256, 257, 1024, 5000, 16000])
+def test_otf_gemv_smaller_workspace(orc, n):
+    torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(n)
+    d, x, y0 = rng.uniform(n, 2 * n, n), rng.standard_normal(n), rng.standard_normal(n)
+    segs = min(64, -(-n // 256))
+    wb = segs * n * 8 if segs > 1 else 0
+    D, X, Y, W = dev(d), dev(x), dev(y0), dev(np.full(wb // 8 + 8, np.nan))
+    if wb:
+        assert L.omx_otf_gemv_f64(n, 42, ptr(D), -1.0, ptr(X), ptr(Y), ptr(W), wb - 1, None) == -3
+        assert L.omx_otf_gemv_f64(n, 42, ptr(D), -1.0, ptr(X), ptr(Y), None, wb, None) == -3
+    assert L.omx_otf_gemv_f64(n, 42, ptr(D), -1.0, ptr(X), ptr(Y), ptr(W) if wb else None, wb, None) == 0
+    assert np.all(np.isnan(host(W)[wb // 8:]))
+    ref = orc.otf_gemv(n, 42, d, -1.0, x, y0)
+    bound = (2 * n + 8) * 2.0 ** -53 * (np.abs(y0) + d * np.abs(x) + 0.5 * np.abs(x).sum())
+    assert np.all(np.abs(host(Y) - ref) <= bound)
+
+
 # FP16 and FP8 products whose last tiles are cut at any row and column, with C
 # on whole lines, on 16 bytes and on neither: the entries that exist are those
 # of the product of whole tiles, bit for bit, and no other is written
