@@ -41,17 +41,18 @@ int gemv_segments(int64_t n, int64_t mincols = 64) {
 }
 
 // The generator's state with its top bit flipped, t = s + 2^63 mod 2^64, steps
-// by the same map as s (its multiplier is odd).  double(int64(s)) from it:
-// 2^52 + lo and 2^84 + 2^32 hi are t's halves under constant high words, and
-// (2^84 + 2^32 hi) - (2^84 + 2^63 + 2^52) is exact, so the last addition rounds
-// the exact integer once, as the conversion does.
+// by the same map as s (its multiplier is odd).  2^-64 double(int64(s)) from it
+// (the factor keeps the sums within the range that the entries' have):
+// 2^-64 times 2^52 + lo and 2^84 + 2^32 hi are t's halves under constant high
+// words, and 2^-64 ((2^84 + 2^32 hi) - (2^84 + 2^63 + 2^52)) is exact, so the
+// last addition rounds the exact integer once, as the conversion does.
 __device__ __forceinline__ double otf_int(uint64_t t) {
-    const double lo = __builtin_bit_cast(double, 0x4330000000000000ull | (uint32_t)t);
-    const double hi = __builtin_bit_cast(double, 0x4530000000000000ull | (t >> 32));
-    return (hi - 0x1.00000801p84) + lo;  // 2^84 + 2^63 + 2^52
+    const double lo = __builtin_bit_cast(double, 0x3F30000000000000ull | (uint32_t)t);
+    const double hi = __builtin_bit_cast(double, 0x4130000000000000ull | (t >> 32));
+    return (hi - 0x1.00000801p20) + lo;  // 2^20 + 2^-1 + 2^-12
 }
 
-// acc += int64(s_ij) x_j for the columns j of [j0, j1), in column order, the
+// acc += 2^-64 int64(s_ij) x_j for the columns j of [j0, j1), in column order, the
 // row's state t stepping by the map jn per column (t leaves as the state of
 // column j1).  The entries' common factor is applied to the sum, and the
 // conversion above takes two additions in place of two conversions, which run
@@ -114,7 +115,7 @@ k_otf_gemv(int64_t n, uint64_t x00, omx_map jn, const double *__restrict__ diag,
     otf_columns<false>(t, acc, jn, x, c0, lo);
     otf_columns<true>(t, acc, jn, x, lo, hi, (int)(i - lo));
     otf_columns<false>(t, acc, jn, x, hi, c1);
-    acc *= 0x1.fffffffffffffp-65;  // RandStat's scale (omx_lcg_value)
+    acc *= 0x1.fffffffffffffp-1;  // the rest of RandStat's scale (omx_lcg_value)
     if (i >= lo && i < hi) acc = __builtin_fma(diag[i], x[i], acc);
     if (part)
         part[seg * n + i] = acc;

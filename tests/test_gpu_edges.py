@@ -468,6 +468,22 @@ def test_otf_gemv_smaller_workspace(orc, n):
     assert np.all(np.abs(host(Y) - ref) <= bound)
 
 
+# x at either end of the FP64 range: a power of two times x gives that times y,
+# bit for bit (no product or sum leaves the range)
+@pytest.mark.parametrize("e", [1005, -900])
+def test_otf_gemv_range(e):
+    torch = torch_cuda()
+    L, n = _L(), 1000
+    rng = np.random.default_rng(5)
+    D, wb = dev(rng.uniform(n, 2 * n, n)), L.omx_otf_gemv_workspace_bytes(n)
+    W, x, y = empty(wb, torch.uint8), rng.uniform(-1, 1, n), []
+    for s in (0, e):
+        X, Y = dev(np.ldexp(x, s)), dev(np.zeros(n))
+        assert L.omx_otf_gemv_f64(n, 42, ptr(D), -1.0, ptr(X), ptr(Y), ptr(W), wb, None) == 0
+        y.append(host(Y))
+    assert np.array_equal(np.ldexp(y[0], e), y[1])
+
+
 # FP16 and FP8 products whose last tiles are cut at any row and column, with C
 # on whole lines, on 16 bytes and on neither: the entries that exist are those
 # of the product of whole tiles, bit for bit, and no other is written
