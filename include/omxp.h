@@ -209,7 +209,14 @@ int omx_lowrank_gemv_f64(int64_t n, int64_t rank, const double *sigma,
 /* Bytes of scratch with which the triangular solves of order n run as one
  * launch instead of one per 256 columns (n > 512, A 16-byte aligned, lda % 4
  * == 0, work 8-byte aligned).  They work in place on x without it: `work` may
- * be NULL or smaller.  Calls that overlap need a workspace each. */
+ * be NULL or smaller, and is then not touched.
+ *
+ * Otherwise the solve writes to work, and its workgroups wait for values that
+ * other workgroups put there: nothing else may write to it from the call until
+ * the solve has finished on the GPU.  Solves that overlap (other streams,
+ * threads, captured graphs) need a workspace each: with one between them a
+ * solve's values are cleared by the other's start, and it waits for them for
+ * ever.  A caller that has one buffer for all its streams passes NULL. */
 size_t omx_trsv_workspace_bytes(int64_t n);
 
 /* x <- L^-1 x with L the unit-lower FP32 factor stored in A (order n), FP64
