@@ -160,7 +160,7 @@ struct omx_solver {
     hipStream_t crit = nullptr, bulk = nullptr;
     std::vector<hipEvent_t> ev_panel, ev_t0, ev_t1;
     int64_t G = 2;                      // panels per trailing update (group)
-    DevBuf Lp[2], Rp[2], Tp;            // FP16 group buffers (K = G b) and the -alt temporaries (column, row panel)
+    DevBuf Lp[2], Rp[2], Tp;            // FP16 group buffers (K = G b) and the -alt temporary
     DevBuf L8[2], R8[2], Le[2], Re[2];  // FP8 group buffers and their exponents
     DevBuf L8max, R8max;                // tile max-abs scratch
     int scale16 = 0;                    // FP16 Schur panels with per-strip scales
@@ -371,7 +371,7 @@ int omx_solver_create(int64_t n, int64_t b, int alt, int flags, omx_solver **out
     s->last_sched.assign(nb, 0);
     s->prec.assign(nb, 0);
     s->last_feat.assign((size_t)nb * OMX_MLP_NFEATURES, 0.0f);
-    if ((rc = dalloc(s->Tp, 2 * omx_panel_bytes(rows, b, 0)))) return fail(rc);
+    if ((rc = dalloc(s->Tp, omx_panel_bytes(rows, b, 0)))) return fail(rc);
     if ((rc = dalloc(s->Wup, (size_t)b * b * 4)) || (rc = dalloc(s->Wlo, (size_t)b * b * 4)) ||
         (rc = dalloc(s->Wtmp, (size_t)b * b * 4)) ||
         (rc = dalloc(s->Wup_h, omx_panel_bytes(b, b, 0))) || (rc = dalloc(s->Wlo_h, omx_panel_bytes(b, b, 0))))
@@ -675,7 +675,7 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
     const bool learned = !sched && s->has_policy;
     const bool stats = s->fp8 != 0;
     int *info = static_cast<int *>(s->info.p);  // one slot per diagonal block
-    uint16_t *Tp = static_cast<uint16_t *>(s->Tp.p), *Tr = Tp + s->Tp.bytes / 4;
+    uint16_t *Tp = static_cast<uint16_t *>(s->Tp.p);
     float *Wup = static_cast<float *>(s->Wup.p), *Wlo = static_cast<float *>(s->Wlo.p);
     uint16_t *Wup_h = static_cast<uint16_t *>(s->Wup_h.p), *Wlo_h = static_cast<uint16_t *>(s->Wlo_h.p);
     s->bulk_count = 0;
@@ -742,14 +742,19 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
                 const int ml = s->alt == 2 ? OMX_MASK_R_GT_K_UNIT : OMX_MASK_NONE;
                 float *lmax = stats ? static_cast<float *>(s->L8max.p) : nullptr;
                 float *rmax = stats ? static_cast<float *>(s->R8max.p) : nullptr;
+                // the row panel's operand lies in the panel's own window of
+                // the group buffer, which is free until pack_panel
+                const int64_t ldk = s->G * b, k0 = pwin(i, b, s->G);
+                uint16_t *Rp = static_cast<uint16_t *>(s->Rp[pbuf(i, s->G)].p);
+                uint16_t *Rw = Rp + (k0 / OMX_STRIP) * (ldk / OMX_KSTAGE16) * 16384;
                 const omx_pack_job pk[4] = {
                     {b, b, Wup, b, 1, mu, Wup_h, b, 0, 0, nullptr, nullptr},
                     {rest, b, Acol, 1, lda, OMX_MASK_NONE, Tp, b, 0, 0, nullptr, nullptr},
                     {b, b, Wlo, 1, b, ml, Wlo_h, b, 0, 0, nullptr, nullptr},
-                    {rest, b, Arow, lda, 1, OMX_MASK_NONE, Tr, b, 0, 0, nullptr, nullptr}};
+                    {rest, b, Arow, lda, 1, OMX_MASK_NONE, Rw, ldk, k0, 0, nullptr, nullptr}};
                 const omx_gemm_job pr[2] = {
                     {rest, b, b, Tp, nullptr, 0, b, 0, Wup_h, nullptr, 0, b, 0, Acol, lda, 1, lmax},
-                    {b, rest, b, Wlo_h, nullptr, 0, b, 0, Tr, nullptr, 0, b, 0, Arow, lda, 2, rmax}};
+                    {b, rest, b, Wlo_h, nullptr, 0, b, 0, Rp, nullptr, k0, ldk, k0, Arow, lda, 2, rmax}};
                 if (!T.on) {
                     // one launch for the four packs, one for the two products
                     // (LU at n = 10240, b = 256: 10 launches of a step's
@@ -761,9 +766,10 @@ int omx_lu_factor(omx_solver *s, float *A, int64_t lda, const int *sched, double
                     TIMED(T, kT_CONV_L, cs, (double)(rest + b) * b, omx_pack_f16_jobs(2, pk, cs));
                     TIMED(T, kT_TRSM_L, cs, 2.0 * rb2,
                           omx_gemm_f16_packed_tri(rest, b, b, 1.0f, Tp, Wup_h, 1, 0.0f, Acol, lda, lmax, cs));
-                    TIMED(T, kT_CONV_R, cs, (double)(rest + b) * b, omx_pack_f16_jobs(2, pk + 2, cs));
+                    const omx_pack_job pt[2] = {pk[2], {rest, b, Arow, lda, 1, OMX_MASK_NONE, Tp, b, 0, 0, nullptr, nullptr}};
+                    TIMED(T, kT_CONV_R, cs, (double)(rest + b) * b, omx_pack_f16_jobs(2, pt, cs));
                     TIMED(T, kT_TRSM_R, cs, 2.0 * rb2,
-                          omx_gemm_f16_packed_tri(b, rest, b, 1.0f, Wlo_h, Tr, 2, 0.0f, Arow, lda, rmax, cs));
+                          omx_gemm_f16_packed_tri(b, rest, b, 1.0f, Wlo_h, Tp, 2, 0.0f, Arow, lda, rmax, cs));
                 }
                 have_max = stats;
             }

@@ -401,6 +401,25 @@ def test_merged_launches_leave_the_factors_alone(n, b, alt, flags, prec):
     assert np.array_equal(_lu(n, b, alt, flags, sched[:nb]), _lu(n, b, alt, flags | 8, sched[:nb]))
 
 
+# device memory of a solver: the group buffers, one packed panel for the
+# inverse products, and what is small beside them (GMRES's basis, the inverses
+# and a page an allocation within 128 MiB; a second panel would be 288 MiB)
+def test_solver_memory():
+    import ctypes as C
+    torch = torch_cuda()
+    L = _L()
+    n, b = 40960, 4096
+    h = C.c_void_p()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    assert L.omx_solver_create(n, b, 1, 0, C.byref(h)) == 0
+    used = free - torch.cuda.mem_get_info()[0]
+    L.omx_solver_destroy(h)
+    panels = 4 * L.omx_panel_bytes(n - b, 2 * b, 0) + L.omx_panel_bytes(n - b, b, 0)
+    inverses = 3 * 4 * b * b + 2 * L.omx_panel_bytes(b, b, 0)
+    assert used <= panels + inverses + (128 << 20), (used, panels, inverses)
+
+
 # FP32 product on the matrix cores: with whole groups of 64 in k and whole
 # float4s of rows (or none, in the last row tile) and without either; one,
 # two and many groups; last columns and rows of a tile (of 128 rows in the last
