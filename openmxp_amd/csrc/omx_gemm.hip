@@ -117,7 +117,9 @@ constexpr int kCPolicy = 2;
 // without a cache between the parts go to memory by themselves: there C goes
 // through L2.  C -= X Y at 7936 x 12544 x 2560: FP16 605 -> 526 us (ldc 7937),
 // 531 -> 505 (ldc 7940); FP8 437 -> 325, 317 -> 304; on whole lines (ldc 7936)
-// without this 3 to 5 % slower in FP8.
+// without this 3 to 5 % slower in FP8.  C = X Y (beta = 0): 7936 x 2560 x 2560
+// at ldc 7940 FP16 151 -> 123 us, FP8 95 -> 65; 20479 x 20479 x 512 at ldc 20479
+// 1244 -> 824, 1277 -> 672.  (epilogue_half keeps the policy for every ldc.)
 __device__ __forceinline__ bool whole_lines(const float *C, int64_t ldc) {
     return ldc % 32 == 0 && (reinterpret_cast<uintptr_t>(C) & 127) == 0;
 }
@@ -153,21 +155,28 @@ __device__ __forceinline__ void epilogue(floatx16 (&acc)[4][4], int64_t M, int64
             voff[r] = (int)(((8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * ldc + (lane & 31)) * 4);
         if (kBetaZero) {
             const int64_t cols = N - j0 - 4 * (lane >> 5);
+            auto store = [&](auto policy) {
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
-                const __amdgpu_buffer_rsrc_t rs = colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc, N - j0 - 32 * ni);
+                for (int ni = 0; ni < 4; ++ni) {
+                    const __amdgpu_buffer_rsrc_t rs =
+                        colblock_rsrc(C + (j0 + 32 * ni) * ldc + i0, ldc, N - j0 - 32 * ni);
 #pragma unroll
-                for (int mi = 0; mi < 4; ++mi) {
-                    if (mi >= rows) continue;
+                    for (int mi = 0; mi < 4; ++mi) {
+                        if (mi >= rows) continue;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const float v = alpha * acc[mi][ni][r];
-                        if (8 * (r >> 2) + (r & 3) < cols - 32 * ni) mx = fmaxf(mx, fabsf(v));
-                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs, voff[r] + mi * 128,
-                                                              0, kCPolicy);
+                        for (int r = 0; r < 16; ++r) {
+                            const float v = alpha * acc[mi][ni][r];
+                            if (8 * (r >> 2) + (r & 3) < cols - 32 * ni) mx = fmaxf(mx, fabsf(v));
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), rs,
+                                                                  voff[r] + mi * 128, 0, decltype(policy)::value);
+                        }
                     }
                 }
-            }
+            };
+            if (whole_lines(C, ldc))
+                store(std::integral_constant<int, kCPolicy>{});
+            else
+                store(std::integral_constant<int, 0>{});
             return;
         }
         // old values in units of two row blocks of one column block (32
@@ -857,7 +866,7 @@ __device__ __forceinline__ void epilogue_half(floatx16 (&acc)[4][2], int64_t M, 
         }
         return;
     }
-    // ldc too large for 32-bit column offsets: checked one by one
+    // edge tiles (and ldc too large for 32-bit column offsets): checked one by one
     const int64_t ib = i0 + (lane & 31);
     const int64_t jb = j0 + 4 * (lane >> 5);
 #pragma unroll
