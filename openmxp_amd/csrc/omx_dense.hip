@@ -712,8 +712,8 @@ __device__ __forceinline__ void lu_stages(float (&r)[8], int lane, int wave, Get
 }
 
 // A: the order-n block; j: first column of the step; np: 128-row workgroups
-// of the column block (= those of the row block); nti: of them a column of
-// trailing tiles has; first: info is set, not lowered
+// of the column block (= those of the row block).  The first step (no update:
+// kUpd false) sets info, the later ones lower it.
 template <bool kUpd, bool kVec>
 __global__ void __launch_bounds__(kGT) __attribute__((amdgpu_waves_per_eu(4)))
 k_getrf_step64(int64_t n, int64_t j, int np, float *__restrict__ A, int64_t lda, int *__restrict__ info) {

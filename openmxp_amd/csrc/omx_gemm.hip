@@ -1282,15 +1282,10 @@ int resolve_job(const omx_gemm_job &q, int64_t es, bool fp8, GemmJob &j) {
     return OMX_OK;
 }
 
-bool pair_splits(const omx_gemm_job *q) {
-    // a product without rows or columns, or the other kernel family
-    return use_half_tiles() || q[0].m == 0 || q[0].n == 0 || q[1].m == 0 || q[1].n == 0;
-}
-
 }  // namespace
 
 int omx_gemm_f16_pair(const omx_gemm_job *q, float alpha, float beta, void *stream) {
-    if (pair_splits(q)) {
+    if (use_half_tiles()) {  // the other kernel family
         for (int i = 0; i < 2; ++i) {
             const int rc = gemm_f16_launch(q[i].m, q[i].n, q[i].k, alpha, static_cast<const uint16_t *>(q[i].X), nullptr,
                                            q[i].x_row0, q[i].x_ldk, q[i].x_k0, static_cast<const uint16_t *>(q[i].Y),
@@ -1322,13 +1317,13 @@ int omx_gemm_f16_pair(const omx_gemm_job *q, float alpha, float beta, void *stre
     return OMX_OK;
 }
 
-int omx_gemm_f8_pair(const omx_gemm_job *q, float alpha, float beta, void *stream) {
-    if (pair_splits(q) || beta == 0.0f) {
+int omx_gemm_f8_pair(const omx_gemm_job *q, float alpha, void *stream) {
+    if (use_half_tiles()) {
         for (int i = 0; i < 2; ++i) {
             const int rc = omx_gemm_f8_packed_window(q[i].m, q[i].n, q[i].k, alpha, static_cast<const uint8_t *>(q[i].X),
                                                      q[i].xexp, q[i].x_row0, q[i].x_ldk, q[i].x_k0,
                                                      static_cast<const uint8_t *>(q[i].Y), q[i].yexp, q[i].y_row0,
-                                                     q[i].y_ldk, q[i].y_k0, beta, q[i].C, q[i].ldc, stream);
+                                                     q[i].y_ldk, q[i].y_k0, 1.0f, q[i].C, q[i].ldc, stream);
             if (rc) return rc;
         }
         return OMX_OK;
@@ -1341,7 +1336,7 @@ int omx_gemm_f8_pair(const omx_gemm_job *q, float alpha, float beta, void *strea
     const int64_t split = (int64_t)j[0].tiles_m * j[0].tiles_n, total = split + (int64_t)j[1].tiles_m * j[1].tiles_n;
     if (total >= ((int64_t)1 << 31)) return OMX_ERR_ARG;
     hipLaunchKernelGGL((k_gemm_f8<false, kNbuf, true>), dim3((unsigned)total), dim3(kThreads), 0, omx_stream(stream),
-                       j[0].M, j[0].N, j[0].K, alpha, beta, j[0].X, j[0].xexp, j[0].Y, j[0].yexp, j[0].C, j[0].ldc,
+                       j[0].M, j[0].N, j[0].K, alpha, 1.0f, j[0].X, j[0].xexp, j[0].Y, j[0].yexp, j[0].C, j[0].ldc,
                        j[0].tiles_m, j[0].tiles_n, j[0].xstrip, j[0].ystrip, j[0].xet, j[0].yet, j[1], (int)split);
     OMX_LAUNCH_CHECK();
     return OMX_OK;

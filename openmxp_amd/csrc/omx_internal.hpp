@@ -41,6 +41,7 @@ struct omx_gemm_job {
 // up to four FP16 / two FP8 panels of equal k
 OMX_HIDDEN int omx_pack_f16_jobs(int count, const omx_pack_job *jobs, void *stream);
 OMX_HIDDEN int omx_pack_f8_jobs(int count, const omx_pack_job *jobs, void *stream);
-// C_i = beta C_i + alpha X_i Y_i^T, i = 0, 1
+// C_i = beta C_i + alpha X_i Y_i^T, i = 0, 1 (FP8: beta = 1); both with rows
+// and columns
 OMX_HIDDEN int omx_gemm_f16_pair(const omx_gemm_job *jobs, float alpha, float beta, void *stream);
-OMX_HIDDEN int omx_gemm_f8_pair(const omx_gemm_job *jobs, float alpha, float beta, void *stream);
+OMX_HIDDEN int omx_gemm_f8_pair(const omx_gemm_job *jobs, float alpha, void *stream);

@@ -508,7 +508,7 @@ static int apply_panels(omx_solver *s, int64_t i0, int64_t i1, const Target *t, 
         // (n = 61440, b = 2560: 116.6 ms by themselves, 120 in one launch)
         const bool pair = nq == 2 && q[0].m * q[0].n <= (int64_t)256 * OMX_STRIP * OMX_STRIP;
         if (pair && cls > 0)
-            RC(omx_gemm_f8_pair(q, -1.0f, 1.0f, st));
+            RC(omx_gemm_f8_pair(q, -1.0f, st));
         else if (pair && !s->scale16)
             RC(omx_gemm_f16_pair(q, -1.0f, 1.0f, st));
         else
