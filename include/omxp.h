@@ -514,7 +514,7 @@ typedef struct omx_solver omx_solver;
 #define OMX_SOLVER_FP8 1     /* flag of omx_solver_create: also allocate FP8 panels */
 #define OMX_SOLVER_SCALE16 2 /* flag: FP16 Schur panels with per-strip pow2 scales */
 #define OMX_SOLVER_GROUP4 4  /* flag: one trailing update per 4 panels (depth 4b) instead of per 2 */
-#define OMX_SOLVER_TIMERS 8  /* flag: phase timers (HIP events around every timed phase) */
+#define OMX_SOLVER_TIMERS 8  /* flag: phase timers (HIP events around every timed phase; more launches, see omx_solver_timers) */
 
 /* Create a solver for order n, block b (n % b == 0, b % 256 == 0), panel
  * method alt (0: FP32 TRSM, 1: FP16 GEMM with the TRSM-on-identity inverse,
@@ -596,7 +596,11 @@ int omx_solver_last_schedule(omx_solver *s, int *sched, float *features);
  * FP16/FP8 packs), GEMM_UPDATE (every Schur product: trailing, look-ahead
  * and within a group), IR_GEMV, IR_TRSV; TOTAL is the wall time of those
  * calls.  Phases on the two streams overlap, so the items can sum to more
- * than TOTAL.  seconds, ops: host arrays of OMX_TIMER_ITEMS doubles.
+ * than TOTAL.  To be timed by themselves, a step's packs and its two panel
+ * products run as launches of their own, which without the flag share one
+ * launch each: the factors are the same, TOTAL is longer (where b is small by
+ * several launches' time a step).  seconds, ops: host arrays of
+ * OMX_TIMER_ITEMS doubles.
  * Returns OMX_ERR_ARG when the solver has no timers. */
 #define OMX_TIMER_ITEMS 23
 int omx_solver_timers(const omx_solver *s, double *seconds, double *ops);

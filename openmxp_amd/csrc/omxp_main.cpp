@@ -385,6 +385,8 @@ int main(int argc, char **argv) {
             const int gu = 10, gp = 11;  // GEMM_UPDATE, GEMM_PROGRESS
             const double gt = sec[gu] + sec[gp];
             std::printf("GEMM_TOTAL: %f Tflops\n", gt > 0 ? 1e-12 * (ops[gu] + ops[gp]) / gt : 0.0);
+            std::printf("(timed phases run as launches of their own; without -timer a step's packs, and its panel "
+                        "products, share launches)\n");
             if (sec[OMX_TIMER_ITEMS - 1] < 0)
                 std::printf("(MISC = TOTAL - the items is negative: the trailing updates on the bulk stream run "
                             "beside the factorisation's items, %.3f s of overlap)\n",

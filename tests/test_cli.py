@@ -84,6 +84,14 @@ def test_timer_report():
     assert any(l.startswith("GEMM_TOTAL:") and float(l.split()[1]) > 0 for l in r.stdout.splitlines())
 
 
+@pytest.mark.gpu
+def test_timer_report_names_its_launches():
+    """The table is of a run whose timed phases share no launch."""
+    from tests.gpu_util import torch_cuda
+    torch_cuda()
+    note = "timed phases run as launches of their own"
+    assert note in run(1024, 256, "-timer").stdout and note not in run(1024, 256).stdout
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("extra", [("--highammat",), ("--highammat-paper", "-cond", "1e4", "-ir", "gmres"),
