@@ -126,6 +126,31 @@ def test_getrf_keeps_finished_rows(n, k, pivot):
     assert np.array_equal(G[:k + 1], F[:k + 1])
 
 
+# The pivots' reciprocals (hardware reciprocal and one Newton step) are the
+# rounded quotients 1 / u: every mantissa, and a sample of exponents and signs.
+# A diagonal matrix with ones in its last row leaves 63 of them there.
+def test_getrf_reciprocals_are_rounded_quotients():
+    torch = torch_cuda()
+    L = _L()
+    rng = np.random.default_rng(0)
+    u = np.arange(0x3f800000, 0x40000000, dtype=np.uint32)
+    v = rng.integers(0, 1 << 32, 1 << 18, dtype=np.uint32) & 0x807fffff | \
+        (rng.integers(4, 251, 1 << 18, dtype=np.uint32) << 23)
+    u = np.concatenate([u, v])
+    nm = -(-len(u) // 63)
+    u = np.concatenate([u, np.full(nm * 63 - len(u), u[0])]).view(np.float32).reshape(nm, 63)
+    A = torch.zeros((nm, 64, 64), dtype=torch.float32, device="cuda")  # [matrix][column][row]
+    i = torch.arange(63, device="cuda")
+    A[:, i, i] = dev(u)
+    A[:, :, 63] = 1.0
+    base = ptr(A)
+    torch.cuda.synchronize()
+    for q in range(nm):
+        assert L.omx_getrf_nopiv_f32(64, base + q * 64 * 64 * 4, 64, None, None) == 0
+    got = host(A[:, :63, 63].contiguous())
+    assert np.array_equal(got, np.float32(1.0) / u)
+
+
 # ranges that pair up evenly, leave an odd one, and pair unequal sizes; merges
 # in LDS (to 256 rows a side) and beyond; aligned and unaligned
 @pytest.mark.parametrize("pad", [0, 1])
