@@ -324,7 +324,8 @@ PEAK_FP64_VALU_TFLOPS = 78.6  # MI355X FP64 vector
 
 def ir_kernels(gs, seed, reps=3):
     """The refinement's two HBM-bound triangular solves with the FP32 factors
-    (2 n^2 bytes of factor read each: half the n x n FP32 matrix) and its
+    (2 n^2 bytes of factor read each: half the n x n FP32 matrix), with the
+    workspace as the solver calls them (n > 512: one launch each), and its
     VALU-bound residual GEMV (n^2 LCG values regenerated, n^2 FP64 FMAs),
     each timed with HIP events on the null stream the C ABI launches on,
     on the factored matrix in gs.A."""
@@ -335,6 +336,8 @@ def ir_kernels(gs, seed, reps=3):
     y = torch.empty_like(x)
     wb = L.omx_otf_gemv_workspace_bytes(n)
     w = torch.empty(max(wb, 8) // 8, dtype=torch.float64, device="cuda")
+    tb = L.omx_trsv_workspace_bytes(n)
+    tw = torch.empty(max(tb, 8) // 8, dtype=torch.float64, device="cuda")
 
     def timed(fn):
         ts = []
@@ -347,8 +350,9 @@ def ir_kernels(gs, seed, reps=3):
             ts.append(e0.elapsed_time(e1) * 1e-3)
         return min(ts)
 
-    tl = timed(lambda: L.omx_trsv_lower_unit_f32f64(n, b, gs.A.data_ptr(), gs.lda, x.data_ptr(), None, 0, None))
-    tu = timed(lambda: L.omx_trsv_upper_f32f64(n, b, gs.A.data_ptr(), gs.lda, x.data_ptr(), None, 0, None))
+    tl = timed(lambda: L.omx_trsv_lower_unit_f32f64(n, b, gs.A.data_ptr(), gs.lda, x.data_ptr(), tw.data_ptr(), tb,
+                                                         None))
+    tu = timed(lambda: L.omx_trsv_upper_f32f64(n, b, gs.A.data_ptr(), gs.lda, x.data_ptr(), tw.data_ptr(), tb, None))
     tg = timed(lambda: L.omx_otf_gemv_f64(n, seed, gs.d.data_ptr(), -1.0, x.data_ptr(), y.data_ptr(), w.data_ptr(),
                                           wb, None))
     tri = 2.0 * n * n
@@ -357,15 +361,14 @@ def ir_kernels(gs, seed, reps=3):
         gbs = tri / t * 1e-9
         out[name] = {"ms": round(t * 1e3, 3), "bound": "hbm", "achieved": round(gbs, 1), "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": round(gbs / PEAK_HBM_GBS, 4),
-                     "bytes": tri, "launches": n // 256}
+                     "bytes": tri, "launches": 2 if n > 512 else -(-n // 256)}
     tf = 2.0 * n * n / tg * 1e-12
     out["otf_gemv"] = {"ms": round(tg * 1e3, 3), "bound": "valu", "elements_per_s": round(n * n / tg, 1),
                        "fp64_tflops": round(tf, 2), "peak_fp64_valu_tflops": PEAK_FP64_VALU_TFLOPS,
                        "fp64_frac": round(tf / PEAK_FP64_VALU_TFLOPS, 4),
-                       "note": "each element is one LCG step (64-bit integer multiply-add), an int64->FP64 "
-                               "conversion and scaling, and one FP64 FMA: the FP64 fraction understates the "
-                               "VALU issue rate (9 VALU instructions per element, SIMDs issuing VALU ~96 % of "
-                               "their cycles: profiles/ir_kernels_n204800.txt)"}
+                       "note": "each element is one LCG step (64-bit integer multiply-add), two FP64 additions "
+                               "that convert it, and one FP64 FMA: the FP64 fraction understates the VALU "
+                               "issue rate (9 VALU instructions per element: profiles/ir_kernels_n204800.txt)"}
     return out
 
 
@@ -450,7 +453,7 @@ def summarize_ir(fetch_csv, sq_csv, n):
         durs = collections.defaultdict(dict)
         for r in csv.DictReader(open(path)):
             name = r["Kernel_Name"]
-            key = ("trsv_lower" if "k_trsv_lower" in name else "trsv_upper" if "k_trsv_upper" in name
+            key = ("trsv_lower" if "k_trsv_fused<false>" in name else "trsv_upper" if "k_trsv_fused<true>" in name
                    else "otf_gemv" if "k_otf_gemv" in name else None)
             if key is None:
                 continue
@@ -462,11 +465,10 @@ def summarize_ir(fetch_csv, sq_csv, n):
     for key in ("trsv_lower", "trsv_upper"):
         if key not in fc:
             continue
-        nd = len(fd[key])
-        solves = nd / (n // 256) if n >= 256 else nd
+        solves = len(fd[key])
         fetched = fc[key]["FETCH_SIZE"] * 1024 * 2.0
         sec = sum(fd[key].values()) * 1e-9
-        print(f"{key}: {nd} launches ({solves:.0f} solves), {sec * 1e3:.2f} ms in all, "
+        print(f"{key}: {solves} solves, {sec * 1e3:.2f} ms in all, "
               f"{tri * solves / sec * 1e-9:.1f} GB/s of factor reads (8000 peak); "
               f"fetched past L2 {fetched / solves:.4e} bytes per solve = {fetched / (tri * solves):.3f} x the 2 n^2 "
               "factor bytes")
@@ -729,6 +731,7 @@ def main():
     if args.ir_sweep:
         gs = GpuSolve(args.n, args.b, args.alt, fp8=False, group=2)
         gs.generate(args.seed)
+        gs.A.mul_(1.0 / args.n)  # stands in for the factors: solutions of that size, not ones that overflow
         print(json.dumps({"ir_sweep": ir_kernels(gs, args.seed), "n": args.n, "b": args.b}))
         return
     if args.gpus != 1:
